@@ -25,8 +25,8 @@ bc_error bc_amd_generator_multiples(const void *scalars, void *bases, unsigned c
  * (sum = 2*sum + results[j][i] for i = 253..0) as a canonical affine
  * Montgomery point, (0, 0) for infinity.  `results` is a host array of
  * `count` device pointers (254 Jacobian points each); `points` is device
- * memory.  One thread per MSM: the 253 dependent doublings take about a
- * millisecond whatever the count. */
+ * memory.  The 253 dependent doublings of one MSM take under a millisecond;
+ * MSMs of one call run side by side. */
 bc_error bc_amd_msm_fold(const void *const *results, void *points, unsigned count, bc_stream stream);
 
 /* msm_execute_async without any allocation.  No counterpart in the
