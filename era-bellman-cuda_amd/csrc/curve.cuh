@@ -8,6 +8,7 @@
 #pragma once
 
 #include "device.cuh"
+#include "inverse.cuh"
 
 namespace bc {
 

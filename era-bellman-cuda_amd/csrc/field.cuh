@@ -277,19 +277,6 @@ template <class F> BC_HD fe pow_u64(const fe &a, uint64_t e) {
   return acc;
 }
 
-// a^(m-2) = a^-1 (Fermat); a^-1 = 0 for a = 0.  Montgomery in and out.
-template <class F> BC_HD fe inverse(const fe &a) {
-  fe e;
-  sub_const(e, fe_const<F>(F::m), {2, 0, 0, 0, 0, 0, 0, 0});
-  fe acc = fe_one<F>(), b = a;
-  for (int i = 0; i < 256; i++) {
-    if ((e.v[i >> 5] >> (i & 31)) & 1)
-      acc = mul<F>(acc, b);
-    b = mul<F>(b, b);
-  }
-  return acc;
-}
-
 // c-bit field of a 256-bit value starting at bit offset (bits beyond 255 read as 0)
 BC_HD uint32_t extract_bits(const fe &a, unsigned offset, unsigned count) {
   const unsigned li = offset >> 5, sh = offset & 31;

@@ -29,6 +29,7 @@
 
 #include "batch.h"
 #include "common.h"
+#include "inverse.cuh"
 #include "ntt.h"
 #include "tables.h"
 #include "tuning.h"
