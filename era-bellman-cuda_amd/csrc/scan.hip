@@ -150,49 +150,131 @@ hipError_t scan_u32_exclusive(const uint32_t *in, uint32_t *out, size_t n, arena
 }
 
 // ---------------- Fr inclusive prefix product ----------------
-__global__ __launch_bounds__(SCAN_BLOCK) void prefix_product_block_kernel(const fe *in, fe *out, fe *block_totals, size_t n) {
-  using F = FrParams;
-  __shared__ fe sh[SCAN_BLOCK];
-  const size_t base = (size_t)blockIdx.x * SCAN_TILE + threadIdx.x * SCAN_ITEMS;
-  fe v[SCAN_ITEMS];
-  fe acc = fe_one<F>();
+// A product is about 0.5 us of a SIMD's time whatever the wave's lanes hold, so
+// a block that scans a tile has four waves, one per SIMD, and a scan of few
+// elements is spread over the CUs: tiles of PP_TILE elements are scanned, the
+// tile products are scanned, and a second launch multiplies every tile by the
+// product before it (65539 elements 37 -> 31 us, of which the 16 products
+// in sequence of a tile are 8).  That is 4.5 products and 128 bytes an element.
+// Above PP_TILES_MAX elements a thread instead takes PP_CHUNK consecutive ones:
+// one launch multiplies up every chunk, the chunk products are scanned as above,
+// and one launch walks every chunk again from the product before it: 2.6
+// products and 100 bytes an element (4194299 elements 212 -> 163 us; at 2^20
+// the two are equal).
+constexpr unsigned PP_WAVES = SCAN_BLOCK / 64;
+constexpr unsigned PP_TILE = SCAN_BLOCK * 4;
+constexpr unsigned PP_CHUNK = 8;
+constexpr unsigned PP_TILES_MAX = 1u << 20;
+
+__device__ __forceinline__ fe shfl_up_fe(const fe &a, unsigned off) {
+  fe r;
 #pragma unroll
-  for (unsigned k = 0; k < SCAN_ITEMS; k++) {
-    v[k] = base + k < n ? load_fe(in + base + k) : fe_one<F>();
-    acc = k == 0 ? v[0] : mul<F>(acc, v[k]);
-    v[k] = acc; // local inclusive products
-  }
-  sh[threadIdx.x] = acc;
-  __syncthreads();
-  for (unsigned off = 1; off < SCAN_BLOCK; off <<= 1) {
-    fe t = sh[threadIdx.x];
-    if (threadIdx.x >= off)
-      t = mul<F>(sh[threadIdx.x - off], t);
-    __syncthreads();
-    sh[threadIdx.x] = t;
-    __syncthreads();
-  }
-  const bool has_prefix = threadIdx.x > 0;
-  const fe prefix = has_prefix ? sh[threadIdx.x - 1] : fe_one<F>();
-#pragma unroll
-  for (unsigned k = 0; k < SCAN_ITEMS; k++)
-    if (base + k < n)
-      store_fe(out + base + k, has_prefix ? mul<F>(prefix, v[k]) : v[k]);
-  if (threadIdx.x == SCAN_BLOCK - 1 && block_totals)
-    store_fe(block_totals + blockIdx.x, sh[SCAN_BLOCK - 1]);
+  for (int i = 0; i < 8; i++)
+    r.v[i] = __shfl_up(a.v[i], off, 64);
+  return r;
 }
 
-// multiplies block b >= 1 by the inclusive product of blocks [0, b)
-__global__ __launch_bounds__(SCAN_BLOCK) void prefix_product_fixup_kernel(fe *out, const fe *block_inclusive, size_t n) {
-  if (blockIdx.x == 0)
-    return;
-  const fe m = load_fe(block_inclusive + blockIdx.x - 1);
-  const size_t i = (size_t)blockIdx.x * SCAN_TILE + threadIdx.x;
+// Scans tiles of SCAN_BLOCK * K elements, K consecutive ones a thread; the
+// product of a whole tile goes to tile_products (if any).
+template <unsigned K>
+__global__ __launch_bounds__(SCAN_BLOCK) void prefix_product_tile_kernel(const fe *in, fe *out, fe *tile_products, size_t n) {
+  using F = FrParams;
+  __shared__ fe wave_product[PP_WAVES];
+  const unsigned lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const size_t first = ((size_t)blockIdx.x * SCAN_BLOCK + threadIdx.x) * K;
+  fe v[K];
 #pragma unroll
-  for (unsigned k = 0; k < SCAN_ITEMS; k++) {
+  for (unsigned k = 0; k < K; k++)
+    v[k] = first + k < n ? load_fe(in + first + k) : fe_one<F>();
+#pragma unroll
+  for (unsigned k = 1; k < K; k++)
+    v[k] = mul_lazy<F>(v[k - 1], v[k]);
+  fe incl = v[K - 1]; // of the wave's lanes up to this one
+  for (unsigned off = 1; off < 64; off <<= 1) {
+    const fe y = shfl_up_fe(incl, off);
+    const fe xy = mul_lazy<F>(y, incl);
+    if (lane >= off)
+      incl = xy;
+  }
+  if (lane == 63)
+    wave_product[wave] = incl;
+  __syncthreads();
+  // everything before the thread's elements: the waves before, then the lanes before
+  fe before = shfl_up_fe(incl, 1);
+  if (wave > 0) {
+    fe w = wave_product[0];
+    for (unsigned i = 1; i < wave; i++)
+      w = mul_lazy<F>(w, wave_product[i]);
+    before = lane > 0 ? mul_lazy<F>(w, before) : w;
+  }
+#pragma unroll
+  for (unsigned k = 0; k < K; k++) {
+    if (threadIdx.x > 0)
+      v[k] = mul_lazy<F>(before, v[k]);
+    v[k] = reduce<F>(v[k]);
+    if (first + k < n)
+      store_fe(out + first + k, v[k]);
+  }
+  if (tile_products && threadIdx.x == SCAN_BLOCK - 1)
+    store_fe(tile_products + blockIdx.x, v[K - 1]);
+}
+
+// multiplies tile t >= 1 by the product of the tiles [0, t)
+__global__ __launch_bounds__(SCAN_BLOCK) void prefix_product_fixup_kernel(fe *out, const fe *tiles_inclusive, size_t n) {
+  const fe m = load_fe(tiles_inclusive + blockIdx.x);
+  const size_t i = (size_t)(blockIdx.x + 1) * PP_TILE + threadIdx.x;
+#pragma unroll
+  for (unsigned k = 0; k < PP_TILE / SCAN_BLOCK; k++) {
     const size_t j = i + k * SCAN_BLOCK;
     if (j < n)
       store_fe(out + j, mul<FrParams>(m, load_fe(out + j)));
+  }
+}
+
+// The chunk's elements are all loaded before the first product: its lines are
+// then fetched once although neighbouring lanes are a chunk apart.
+__device__ __forceinline__ void load_chunk(const fe *in, size_t first, size_t n, fe (&v)[PP_CHUNK]) {
+#pragma unroll
+  for (unsigned k = 0; k < PP_CHUNK; k++)
+    v[k] = first + k < n ? load_fe(in + first + k) : fe_one<FrParams>();
+}
+
+__global__ __launch_bounds__(SCAN_BLOCK) void prefix_product_chunk_kernel(const fe *in, fe *products, size_t n) {
+  const size_t c = (size_t)blockIdx.x * SCAN_BLOCK + threadIdx.x, first = c * PP_CHUNK;
+  if (first >= n)
+    return;
+  fe v[PP_CHUNK];
+  load_chunk(in, first, n, v);
+  fe acc = v[0];
+#pragma unroll
+  for (unsigned k = 1; k < PP_CHUNK; k++)
+    acc = mul_lazy<FrParams>(acc, v[k]);
+  store_fe(products + c, acc);
+}
+
+// scanned[c]: the product of c's tile of chunks up to and including chunk c;
+// tiles[t]: the product of the tiles up to and including t
+__global__ __launch_bounds__(SCAN_BLOCK) void prefix_product_apply_kernel(const fe *in, fe *out, const fe *scanned, const fe *tiles, size_t n) {
+  using F = FrParams;
+  const size_t c = (size_t)blockIdx.x * SCAN_BLOCK + threadIdx.x, first = c * PP_CHUNK;
+  if (first >= n)
+    return;
+  fe v[PP_CHUNK];
+  load_chunk(in, first, n, v);
+  fe acc = v[0];
+  if (c > 0) {
+    const size_t tile = (c - 1) / PP_TILE;
+    fe before = load_fe(scanned + (c - 1));
+    if (tile > 0)
+      before = mul_lazy<F>(load_fe(tiles + (tile - 1)), before);
+    acc = mul_lazy<F>(before, acc);
+  }
+#pragma unroll
+  for (unsigned k = 0; k < PP_CHUNK; k++) {
+    if (k > 0)
+      acc = mul_lazy<F>(acc, v[k]);
+    if (first + k < n)
+      store_fe(out + first + k, reduce<F>(acc));
   }
 }
 
@@ -201,19 +283,32 @@ hipError_t prefix_product(const fe *in, fe *out, size_t n, arena &ar) {
   hipStream_t stream = ar.stream();
   if (n == 0)
     return hipSuccess;
-  const size_t blocks = (n + SCAN_TILE - 1) / SCAN_TILE;
-  if (blocks == 1) {
-    prefix_product_block_kernel<<<1, SCAN_BLOCK, 0, stream>>>(in, out, nullptr, n);
+  if (n <= PP_TILE) {
+    if (n <= SCAN_BLOCK)
+      prefix_product_tile_kernel<1><<<1, SCAN_BLOCK, 0, stream>>>(in, out, nullptr, n);
+    else
+      prefix_product_tile_kernel<4><<<1, SCAN_BLOCK, 0, stream>>>(in, out, nullptr, n);
     return hipGetLastError();
   }
-  fe *totals = nullptr;
-  BC_TRY(ar.get(&totals, blocks));
-  prefix_product_block_kernel<<<(unsigned)blocks, SCAN_BLOCK, 0, stream>>>(in, out, totals, n);
+  const bool chunked = n > PP_TILES_MAX;
+  const size_t items = chunked ? (n + PP_CHUNK - 1) / PP_CHUNK : n; // elements or chunk products to scan in tiles
+  const size_t tiles = (items + PP_TILE - 1) / PP_TILE;
+  fe *temp = nullptr;
+  BC_TRY(ar.get(&temp, tiles + (chunked ? items : 0)));
+  fe *tile_products = temp, *chunk_products = temp + tiles;
+  if (chunked) {
+    prefix_product_chunk_kernel<<<grid_for(items, SCAN_BLOCK), SCAN_BLOCK, 0, stream>>>(in, chunk_products, n);
+    BC_LAUNCH_CHECK();
+  }
+  prefix_product_tile_kernel<4><<<(unsigned)tiles, SCAN_BLOCK, 0, stream>>>(chunked ? chunk_products : in, chunked ? chunk_products : out, tile_products, items);
   BC_LAUNCH_CHECK();
-  BC_TRY(prefix_product(totals, totals, blocks, ar));
-  prefix_product_fixup_kernel<<<(unsigned)blocks, SCAN_BLOCK, 0, stream>>>(out, totals, n);
+  BC_TRY(prefix_product(tile_products, tile_products, tiles, ar));
+  if (chunked)
+    prefix_product_apply_kernel<<<grid_for(items, SCAN_BLOCK), SCAN_BLOCK, 0, stream>>>(in, out, chunk_products, tile_products, n);
+  else
+    prefix_product_fixup_kernel<<<(unsigned)(tiles - 1), SCAN_BLOCK, 0, stream>>>(out, tile_products, n);
   BC_LAUNCH_CHECK();
-  return ar.put(totals);
+  return ar.put(temp);
 }
 
 // ---------------- Fr sum ----------------
