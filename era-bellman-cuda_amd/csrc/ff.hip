@@ -6,6 +6,7 @@
 
 #include "common.h"
 #include "inverse.cuh"
+#include "powers.cuh"
 #include "scan.h"
 #include "sort.h"
 #include "tables.h"
@@ -308,6 +309,215 @@ void batch_inverse(const fe *in, fe *out, unsigned count, hipStream_t s) {
     batch_inverse_launch<4, 8>(in, out, count, s);
 }
 
+// ---------------------------------------------------------------- powers of one point
+// The digit table of a scalar in device memory is made there, one thread (a host
+// scalar's is made on the host and travels in the kernel arguments).  Table t + 1
+// belongs to the point^(4^step) of table t.
+__global__ void power_digits_kernel(const fe *point, power_digits *tables, unsigned count, unsigned digits, unsigned log_step) {
+  fe x = load_fe(point);
+  for (unsigned t = 0; t < count; t++) {
+    power_digits_fill(tables[t], x, digits);
+    for (unsigned i = 0; t + 1 < count && i < log_step; i++)
+      x = mul<FrParams>(x, x);
+  }
+}
+
+// out[i] = in[i] base^i.  Up to POWERS_DIRECT elements a thread forms its power
+// from the digits; above, from one entry each of two tables, POWERS_FINE low
+// powers and every POWERS_FINE-th one: two products an element.  65539 elements
+// 47 -> 14 us, 4194299 283 -> 85 us (a prefix product of the base before); at
+// 2^18 the tables' extra launch and memory cost as much as the powers save.
+constexpr unsigned POWERS_LOG_FINE = 10, POWERS_FINE = 1u << POWERS_LOG_FINE;
+constexpr unsigned POWERS_DIRECT = 1u << 17;
+
+template <bool REF>
+__global__ __launch_bounds__(256) void power_table_kernel(const power_digits arg, const power_digits *ref, fe *fine, fe *coarse, unsigned coarse_count,
+                                                          unsigned coarse_digits) {
+  const power_digits &t = REF ? *ref : arg;
+  const unsigned i = blockIdx.x * 256 + threadIdx.x;
+  if (i < POWERS_FINE)
+    store_fe(fine + i, power_of(t, i, POWERS_LOG_FINE / 2));
+  else if (i - POWERS_FINE < coarse_count)
+    store_fe(coarse + (i - POWERS_FINE), power_of(t, i - POWERS_FINE, coarse_digits, POWERS_LOG_FINE / 2));
+}
+
+template <bool REF>
+__global__ __launch_bounds__(256) void multiply_by_powers_direct_kernel(const power_digits arg, const power_digits *ref, const fe *in, fe *out,
+                                                                        unsigned count, unsigned digits) {
+  const power_digits &t = REF ? *ref : arg;
+  const unsigned i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= count)
+    return;
+  const fe v = load_fe(in + i);
+  store_fe(out + i, mul<FrParams>(v, power_of(t, i, digits)));
+}
+
+__global__ __launch_bounds__(256) void multiply_by_powers_kernel(const fe *fine, const fe *coarse, const fe *in, fe *out, unsigned count) {
+  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= count)
+    return;
+  const fe v = load_fe(in + i), w = mul_lazy<FrParams>(load_fe(fine + (i & (POWERS_FINE - 1))), load_fe(coarse + (i >> POWERS_LOG_FINE)));
+  store_fe(out + i, mul<FrParams>(v, w));
+}
+
+// sum_i values[i] x^i: block b writes its tile's sum_j values[b tile + j] x^j to
+// out[b], the values of a polynomial in x^tile for the next launch.  A thread
+// takes every EVAL_BLOCK-th element of the tile (coalesced), by Horner's rule in
+// x^EVAL_BLOCK: one product an element, beside 4 for the thread's own power of x.
+constexpr unsigned EVAL_BLOCK = 256, EVAL_DIGITS = 4; // 4^EVAL_DIGITS = EVAL_BLOCK
+template <unsigned K, bool REF>
+__global__ __launch_bounds__(EVAL_BLOCK) void poly_eval_kernel(const power_digits arg, const power_digits *ref, const fe *values, size_t n, fe *out) {
+  using F = FrParams;
+  __shared__ fe wave_sum[EVAL_BLOCK / 64];
+  const power_digits &t = REF ? *ref : arg;
+  constexpr unsigned G = K < 8 ? K : 8; // loads in flight
+  const size_t first = (size_t)blockIdx.x * (EVAL_BLOCK * K) + threadIdx.x;
+  fe acc = fe_zero();
+  for (unsigned g = K / G; g-- > 0;) {
+    fe v[G];
+#pragma unroll
+    for (unsigned k = 0; k < G; k++) {
+      const size_t i = first + (size_t)(g * G + k) * EVAL_BLOCK;
+      v[k] = i < n ? load_fe(values + i) : fe_zero();
+    }
+#pragma unroll
+    for (unsigned k = G; k-- > 0;) // acc < 3m, x^EVAL_BLOCK canonical: the product is below 2m
+      acc = K == 1 ? v[0] : add_raw(mul_lazy<F>(acc, t.p[EVAL_DIGITS][0]), v[k]);
+  }
+  acc = mul_lazy<F>(acc, power_of(t, threadIdx.x, EVAL_DIGITS));
+#pragma unroll
+  for (unsigned off = 32; off > 0; off >>= 1) {
+    fe o;
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+      o.v[i] = __shfl_xor(acc.v[i], off, 64);
+    acc = add2<F>(acc, o);
+  }
+  if ((threadIdx.x & 63) == 0)
+    wave_sum[threadIdx.x >> 6] = acc;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (unsigned w = 1; w < EVAL_BLOCK / 64; w++)
+      acc = add2<F>(acc, wave_sum[w]);
+    store_fe(out + blockIdx.x, reduce<F>(acc));
+  }
+}
+
+hipError_t poly_eval_launch(unsigned K, const power_digits &arg, const power_digits *ref, const fe *values, size_t n, fe *out, hipStream_t s) {
+  const unsigned blocks = n ? grid_for(n, EVAL_BLOCK * K) : 1;
+  auto launch = [&](auto kernel) { kernel<<<blocks, EVAL_BLOCK, 0, s>>>(arg, ref, values, n, out); };
+  switch (K) {
+  case 1:
+    ref ? launch(poly_eval_kernel<1, true>) : launch(poly_eval_kernel<1, false>);
+    break;
+  case 2:
+    ref ? launch(poly_eval_kernel<2, true>) : launch(poly_eval_kernel<2, false>);
+    break;
+  case 8:
+    ref ? launch(poly_eval_kernel<8, true>) : launch(poly_eval_kernel<8, false>);
+    break;
+  default:
+    ref ? launch(poly_eval_kernel<32, true>) : launch(poly_eval_kernel<32, false>);
+    break;
+  }
+  return hipGetLastError();
+}
+
+// A scalar argument: the value of a host scalar, or where a device one lies.
+const fe *scalar_argument(const void *p, fe *value) {
+  if (classify_pointer(p) == mem_kind::device)
+    return static_cast<const fe *>(p);
+  memcpy(value, p, sizeof(fe));
+  return nullptr;
+}
+
+hipError_t multiply_by_powers(const fe *in, const void *base, fe *out, unsigned n, hipMemPool_t pool, hipStream_t s) {
+  const unsigned digits = power_digits_for(n);
+  power_digits arg;
+  fe b;
+  const fe *base_ref = scalar_argument(base, &b);
+  call_resources res(pool, s);
+  power_digits *ref = nullptr;
+  if (base_ref) {
+    BC_TRY(res.get(&ref, 1));
+    power_digits_kernel<<<1, 1, 0, s>>>(base_ref, ref, 1, digits, 0);
+    BC_LAUNCH_CHECK();
+  } else {
+    power_digits_fill(arg, b, digits);
+  }
+  if (n <= POWERS_DIRECT) {
+    if (ref)
+      multiply_by_powers_direct_kernel<true><<<grid_for(n, 256), 256, 0, s>>>(arg, ref, in, out, n, digits);
+    else
+      multiply_by_powers_direct_kernel<false><<<grid_for(n, 256), 256, 0, s>>>(arg, ref, in, out, n, digits);
+    return hipGetLastError();
+  }
+  const unsigned coarse_count = (n - 1) / POWERS_FINE + 1, coarse_digits = digits - POWERS_LOG_FINE / 2;
+  fe *table = nullptr;
+  BC_TRY(res.get(&table, (size_t)POWERS_FINE + coarse_count));
+  const unsigned blocks = grid_for((size_t)POWERS_FINE + coarse_count, 256);
+  if (ref)
+    power_table_kernel<true><<<blocks, 256, 0, s>>>(arg, ref, table, table + POWERS_FINE, coarse_count, coarse_digits);
+  else
+    power_table_kernel<false><<<blocks, 256, 0, s>>>(arg, ref, table, table + POWERS_FINE, coarse_count, coarse_digits);
+  BC_LAUNCH_CHECK();
+  multiply_by_powers_kernel<<<grid_for(n, 256), 256, 0, s>>>(table, table + POWERS_FINE, in, out, n);
+  return hipGetLastError();
+}
+
+// Launches of poly_eval_kernel until one value is left: 32 elements a thread
+// where that fills the GPU, 8 below, and 2 where a thread's chain of products
+// would set the time (65539 elements: 10 us against 13 at 8); up to EVAL_BLOCK
+// * 8 elements one block does it.  65539 elements 93 -> 32 us (20 us of kernels,
+// the temporary's release most of the rest), 4194299 341 -> 64 us: before, the
+// powers were a prefix product, followed by an element-wise product and a sum.
+hipError_t poly_evaluate(const fe *values, const void *point, void *result, size_t n, hipMemPool_t pool, hipStream_t s) {
+  const unsigned K = n > (size_t)1 << 21 ? 32 : n > (size_t)1 << 17 ? 8 : 2;
+  const size_t tile = (size_t)EVAL_BLOCK * K, last_max = EVAL_BLOCK * 8;
+  unsigned levels = 1;
+  size_t partials = 0;
+  for (size_t m = n; m > last_max; levels++) {
+    m = (m + tile - 1) / tile;
+    partials += m;
+  }
+  fe x;
+  const fe *point_ref = scalar_argument(point, &x);
+  call_resources res(pool, s);
+  power_digits *tables = nullptr;
+  if (point_ref) {
+    unsigned log_tile = 0;
+    while ((size_t)1 << log_tile < tile)
+      log_tile++;
+    BC_TRY(res.get(&tables, levels));
+    power_digits_kernel<<<1, 1, 0, s>>>(point_ref, tables, levels, EVAL_DIGITS + 1, log_tile);
+    BC_LAUNCH_CHECK();
+  }
+  const bool to_device = classify_pointer(result) == mem_kind::device;
+  fe *sums = nullptr; // the partial sums of every level, then the result if it goes to the host
+  if (partials || !to_device)
+    BC_TRY(res.get(&sums, partials + 1));
+  fe *last = to_device ? static_cast<fe *>(result) : sums + partials;
+  for (unsigned level = 0; level < levels; level++) {
+    power_digits arg;
+    if (!tables)
+      power_digits_fill(arg, x, EVAL_DIGITS + 1);
+    const power_digits *ref = tables ? tables + level : nullptr;
+    if (level + 1 == levels) {
+      BC_TRY(poly_eval_launch(n > 2 * EVAL_BLOCK ? 8 : n > EVAL_BLOCK ? 2 : 1, arg, ref, values, n, last, s));
+      break;
+    }
+    BC_TRY(poly_eval_launch(K, arg, ref, values, n, sums, s));
+    values = sums;
+    n = (n + tile - 1) / tile;
+    sums += n;
+    for (size_t i = 1; !tables && i < tile; i <<= 1)
+      x = mul<FrParams>(x, x);
+  }
+  if (!to_device)
+    BC_TRY(hipMemcpyAsync(result, last, sizeof(fe), hipMemcpyDeviceToHost, s));
+  return hipSuccess;
+}
+
 // ---------------------------------------------------------------- packed bits / distribute (src/pn_kernels.cu:123-160)
 __global__ void set_values_from_packed_bits_kernel(fe *values, const unsigned *bits, unsigned count) {
   const unsigned i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -322,10 +532,6 @@ __global__ void distribute_values_kernel(const fe *src, fe *dst, unsigned count,
   if (i >= count)
     return;
   store_fe(dst + (size_t)i * stride, load_fe(src + i));
-}
-
-hipError_t copy_scalar_to_device(fe *dst, const void *src, hipStream_t stream) {
-  return hipMemcpyAsync(dst, src, sizeof(fe), hipMemcpyDefault, stream);
 }
 
 } // namespace bc
@@ -395,29 +601,12 @@ bc_error ff_grand_product(ff_grand_product_configuration cfg) {
   return as_bc(prefix_product(static_cast<const fe *>(cfg.inputs), static_cast<fe *>(cfg.outputs), cfg.count, ar));
 }
 
-// outputs[i] = inputs[i] * base^i via a prefix product of [1, base, base, ...] (src/ff.cu:136-163).
+// outputs[i] = inputs[i] * base^i (src/ff.cu:136-163).
 bc_error ff_multiply_by_powers(ff_multiply_by_powers_configuration cfg) {
-  hipStream_t s = to_stream(cfg.stream);
-  hipMemPool_t pool = to_pool(cfg.mem_pool);
-  const unsigned n = cfg.count;
-  if (n == 0)
+  if (cfg.count == 0)
     return bc_success;
-  fe *powers = nullptr;
-  const bool use_outputs = cfg.inputs != cfg.outputs;
-  if (use_outputs)
-    powers = static_cast<fe *>(cfg.outputs);
-  else
-    BC_TRY_BC(pool_alloc(&powers, n, pool, s));
-  BC_TRY_BC(ff_set_value_one(powers, 1, cfg.stream));
-  if (n > 1) {
-    BC_TRY_BC(ff_set_value(powers + 1, cfg.base, n - 1, cfg.stream));
-    arena ar = arena::pool_mode(pool, s);
-    BC_TRY_BC(prefix_product(powers + 1, powers + 1, n - 1, ar));
-  }
-  BC_TRY_BC(ff_x_mul_y(cfg.inputs, powers, cfg.outputs, n, cfg.stream));
-  if (!use_outputs)
-    BC_TRY_BC(pool_free(powers, s));
-  return bc_success;
+  return as_bc(multiply_by_powers(static_cast<const fe *>(cfg.inputs), cfg.base, static_cast<fe *>(cfg.outputs), cfg.count, to_pool(cfg.mem_pool),
+                                  to_stream(cfg.stream)));
 }
 
 bc_error ff_inverse(ff_inverse_configuration cfg) {
@@ -429,22 +618,7 @@ bc_error ff_inverse(ff_inverse_configuration cfg) {
 
 // sum_i values[i] * point^i (src/ff.cu:183-201); point and result may be host or device pointers.
 bc_error ff_poly_evaluate(ff_poly_evaluate_configuration cfg) {
-  hipStream_t s = to_stream(cfg.stream);
-  hipMemPool_t pool = to_pool(cfg.mem_pool);
-  const unsigned n = cfg.count;
-  fe *temp = nullptr, *sum = nullptr;
-  BC_TRY_BC(pool_alloc(&temp, n ? n : 1, pool, s));
-  BC_TRY_BC(pool_alloc(&sum, 1, pool, s));
-  if (n) {
-    ff_multiply_by_powers_configuration mp{cfg.mem_pool, cfg.stream, cfg.values, cfg.point, temp, n};
-    BC_TRY_BC(ff_multiply_by_powers(mp));
-  }
-  arena ar = arena::pool_mode(pool, s);
-  BC_TRY_BC(field_sum(temp, sum, n, ar));
-  BC_TRY_BC(hipMemcpyAsync(cfg.result, sum, sizeof(fe), hipMemcpyDefault, s));
-  BC_TRY_BC(pool_free(temp, s));
-  BC_TRY_BC(pool_free(sum, s));
-  return bc_success;
+  return as_bc(poly_evaluate(static_cast<const fe *>(cfg.values), cfg.point, cfg.result, cfg.count, to_pool(cfg.mem_pool), to_stream(cfg.stream)));
 }
 
 bc_error ff_get_powers_of_w(void *target, unsigned log_degree, unsigned offset, unsigned count, bool inverse, bool bit_reversed, bc_stream stream) {

@@ -14,7 +14,4 @@ hipError_t scan_u32_exclusive(const uint32_t *in, uint32_t *out, size_t n, arena
 // out[i] = prod_{j<=i} in[j] over Fr (canonical); in and out may alias.
 hipError_t prefix_product(const fe *in, fe *out, size_t n, arena &ar);
 
-// *out = sum of in[0..n) over Fr (zero for n = 0).
-hipError_t field_sum(const fe *in, fe *out, size_t n, arena &ar);
-
 } // namespace bc

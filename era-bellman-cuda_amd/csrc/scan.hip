@@ -1,14 +1,12 @@
 // Device-wide scans and reductions, replacing the reference's cub calls
-// (src/bellman-cuda-cub.cu:30-64): u32 exclusive sum, Fr inclusive prefix
-// product (grand product) and Fr sum.
+// (src/bellman-cuda-cub.cu:30-64): u32 exclusive sum and Fr inclusive prefix
+// product (grand product).
 #include "device.cuh"
 #include "scan.h"
 
 namespace bc {
 
 constexpr unsigned SCAN_BLOCK = 256;
-constexpr unsigned SCAN_ITEMS = 4;
-constexpr unsigned SCAN_TILE = SCAN_BLOCK * SCAN_ITEMS;
 
 // ---------------- u32 exclusive sum ----------------
 // Reduce-then-scan over tiles: one launch sums every tile, one block scans the
@@ -309,45 +307,6 @@ hipError_t prefix_product(const fe *in, fe *out, size_t n, arena &ar) {
     prefix_product_fixup_kernel<<<(unsigned)(tiles - 1), SCAN_BLOCK, 0, stream>>>(out, tile_products, n);
   BC_LAUNCH_CHECK();
   return ar.put(temp);
-}
-
-// ---------------- Fr sum ----------------
-__global__ __launch_bounds__(SCAN_BLOCK) void field_sum_kernel(const fe *in, fe *out, size_t n) {
-  using F = FrParams;
-  __shared__ fe sh[SCAN_BLOCK];
-  const size_t base = (size_t)blockIdx.x * SCAN_TILE + threadIdx.x;
-  fe acc = fe_zero();
-#pragma unroll
-  for (unsigned k = 0; k < SCAN_ITEMS; k++) {
-    const size_t j = base + k * SCAN_BLOCK;
-    if (j < n)
-      acc = add<F>(acc, load_fe(in + j));
-  }
-  sh[threadIdx.x] = acc;
-  __syncthreads();
-  for (unsigned off = SCAN_BLOCK / 2; off > 0; off >>= 1) {
-    if (threadIdx.x < off)
-      sh[threadIdx.x] = add<F>(sh[threadIdx.x], sh[threadIdx.x + off]);
-    __syncthreads();
-  }
-  if (threadIdx.x == 0)
-    store_fe(out + blockIdx.x, sh[0]);
-}
-
-// *out = sum of in[0..n) (zero for n = 0); in is not modified.
-hipError_t field_sum(const fe *in, fe *out, size_t n, arena &ar) {
-  hipStream_t stream = ar.stream();
-  const size_t blocks = n == 0 ? 1 : (n + SCAN_TILE - 1) / SCAN_TILE;
-  if (blocks == 1) {
-    field_sum_kernel<<<1, SCAN_BLOCK, 0, stream>>>(in, out, n);
-    return hipGetLastError();
-  }
-  fe *partial = nullptr;
-  BC_TRY(ar.get(&partial, blocks));
-  field_sum_kernel<<<(unsigned)blocks, SCAN_BLOCK, 0, stream>>>(in, partial, n);
-  BC_LAUNCH_CHECK();
-  BC_TRY(field_sum(partial, out, blocks, ar));
-  return ar.put(partial);
 }
 
 } // namespace bc

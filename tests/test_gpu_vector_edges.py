@@ -20,3 +20,44 @@ def test_grand_product_at_tile_edges(bellman, oracle, n, in_place):
     dev.free(dx)
     if not in_place:
         dev.free(dy)
+
+
+# a power per thread up to 2^17 elements, the two tables above; one evaluation
+# block up to 2048; tiles of 512 up to 2^17, 2048 up to 2^21, 8192 above, then one block
+@pytest.mark.parametrize("n", [0, 1, 2, 64, 65, 255, 256, 257, 511, 513, 2049, 65539, 1 << 17, (1 << 17) + 1, (1 << 20) + 3, (1 << 21) + 1])
+@pytest.mark.parametrize("on_device", [False, True])
+def test_powers_and_evaluation_at_tile_edges(bellman, oracle, n, on_device):
+    B, dev = bellman
+    x = oracle.random_fr(n + 13, max(n, 1))
+    base = oracle.random_fr(n + 17, 1)
+    dx, dy, db, dr = dev.upload(x), dev.malloc(max(n, 1) * 32), dev.upload(base), dev.malloc(32)
+    result = np.zeros((1, 8), dtype=np.uint32)
+    B.call("ff_poly_evaluate", B.ff_poly_evaluate_configuration(dev.pool, dev.stream, dx, db if on_device else base.ctypes.data,
+                                                                dr if on_device else result.ctypes.data, n))
+    B.call("ff_multiply_by_powers", B.ff_multiply_by_powers_configuration(dev.pool, dev.stream, dx, db if on_device else base.ctypes.data, dy, n))
+    dev.sync()
+    if on_device:
+        result = dev.download(dr, (1, 8))
+    assert np.array_equal(result, oracle.poly_evaluate(x[:n], base) if n else np.zeros((1, 8), dtype=np.uint32))
+    if n:
+        expected = oracle.multiply_by_powers(x, base)
+        assert np.array_equal(dev.download(dy, (n, 8)), expected)
+        B.call("ff_multiply_by_powers", B.ff_multiply_by_powers_configuration(dev.pool, dev.stream, dx, db if on_device else base.ctypes.data, dx, n))
+        dev.sync()
+        assert np.array_equal(dev.download(dx, (n, 8)), expected)
+    for p in (dx, dy, db, dr):
+        dev.free(p)
+
+
+@pytest.mark.parametrize("point", [0, 1, -1])
+def test_evaluation_at_special_points(bellman, oracle, point):
+    B, dev = bellman
+    n = 5001
+    x = oracle.random_fr(19, n)
+    base = oracle.to_mont([point % oracle.R])
+    dx = dev.upload(x)
+    result = np.zeros((1, 8), dtype=np.uint32)
+    B.call("ff_poly_evaluate", B.ff_poly_evaluate_configuration(dev.pool, dev.stream, dx, base.ctypes.data, result.ctypes.data, n))
+    dev.sync()
+    assert np.array_equal(result, oracle.poly_evaluate(x, base))
+    dev.free(dx)
