@@ -47,6 +47,7 @@
 #include "curve.cuh"
 #include "curve29.cuh"
 #include "msm.h"
+#include "quad29.cuh"
 #include "scan.h"
 #include "sort.h"
 
@@ -84,12 +85,19 @@ namespace {
 constexpr uint32_t SIGN = 0x80000000u;
 constexpr unsigned MSM_BLOCK = 256;
 constexpr unsigned ACC_BLOCK = 64;
+constexpr unsigned DIGITS_BLOCK = 1024; // threads of a block that also counts (4 points each)
 constexpr unsigned SPLIT_TERMS = 16; // most terms one split thread adds
 constexpr unsigned SMALL_PIECES = 32; // buckets of up to this many partial sums are summed by one thread
 // First-digit counters of one digits block.  Measured at 2^24: with 15 KiB of
 // counters (c = 17) counting in the digits kernel saved 0.18 ms over the
 // sort's own count; with 27 KiB (c = 20) it saved nothing.
 constexpr size_t DIGITS_MAX_LDS = 20 * 1024;
+// Counting takes a block per 4096 points, so it pays once the tiles give every
+// CU a block; below, one point a thread on all CUs and the sort's own count are
+// faster: 2^12 points 120 -> 9 us (and 5 us for the count), four chunks of 2^16
+// 402 -> 32 (and 17) us.  With DIGITS_BLOCK threads a tile instead of 256 the
+// counting form takes 61 us instead of 104 at 2^20.
+constexpr uint64_t DIGITS_MIN_TILES = 256;
 
 struct job_desc {
   const g1_affine *bases;
@@ -162,10 +170,10 @@ hipError_t fill_u32(uint32_t *p, size_t n, uint32_t v, hipStream_t s) {
 // `first_table`, block_points = SEG_TILE, so a block holds tile k of every
 // window's sort segment: it also counts the sort's first digit (key bits
 // [0, bits0)) per window in LDS and writes the tile's counts to the first-pass
-// table, and the sort need not read the entries to count them.  Without it a
-// block takes MSM_BLOCK points, one per thread.  A scalar is loaded one point
-// ahead of its digits.
-__global__ __launch_bounds__(MSM_BLOCK) void digits_kernel(const job_table jobs, uint64_t *__restrict__ entries, uint32_t *__restrict__ first_table,
+// table, and the sort need not read the entries to count them; DIGITS_BLOCK
+// threads share the tile.  Without it a block takes MSM_BLOCK points, one per
+// thread.  A scalar is loaded one point ahead of its digits.
+__global__ __launch_bounds__(DIGITS_BLOCK) void digits_kernel(const job_table jobs, uint64_t *__restrict__ entries, uint32_t *__restrict__ first_table,
                                                            unsigned bits0, uint32_t block_points) {
   using F = FrParams;
   // [Wd][2^min(c, bits0)] 16-bit counts (a tile has SEG_TILE entries), two per
@@ -186,17 +194,17 @@ __global__ __launch_bounds__(MSM_BLOCK) void digits_kernel(const job_table jobs,
     atomicAdd(&hist[slot >> 1], v << ((slot & 1) << 4));
   };
   if (first_table) {
-    for (uint32_t i = threadIdx.x; i < (Wd * nd + 1) / 2; i += MSM_BLOCK)
+    for (uint32_t i = threadIdx.x; i < (Wd * nd + 1) / 2; i += blockDim.x)
       hist[i] = 0;
     __syncthreads();
   }
   const uint32_t p1 = min(n, (k + 1) * block_points);
   uint32_t i = k * block_points + threadIdx.x;
   fe next = i < p1 ? load_fe(jd.scalars + i) : fe_zero();
-  for (; i < p1; i += MSM_BLOCK) {
+  for (; i < p1; i += blockDim.x) {
     const fe pos = from_mont<F>(next);
-    if (i + MSM_BLOCK < p1)
-      next = load_fe(jd.scalars + i + MSM_BLOCK);
+    if (i + blockDim.x < p1)
+      next = load_fe(jd.scalars + i + blockDim.x);
     fe neg;
     sub_limbs(neg, fe_const<F>(F::m), pos); // r - s (r for s = 0)
     const uint32_t global_sign = lt(pos, neg) ? 0u : SIGN;
@@ -233,7 +241,7 @@ __global__ __launch_bounds__(MSM_BLOCK) void digits_kernel(const job_table jobs,
     // fixed-base job's single segment (windows of whole tiles, n >= SEG_TILE),
     // [digit][w tiles + k]
     const uint32_t tiles = (n + SEG_TILE - 1) / SEG_TILE;
-    for (uint32_t j = threadIdx.x; j < (Wd << bits0); j += MSM_BLOCK) {
+    for (uint32_t j = threadIdx.x; j < (Wd << bits0); j += blockDim.x) {
       const uint32_t w = j >> bits0, d = j & ((1u << bits0) - 1), slot = w * nd + d;
       const uint64_t at = jd.stride ? (uint64_t)d * Wd * tiles + w * tiles + k : (uint64_t)j * tiles + k;
       first_table[jd.table_begin + at] = d < nd ? (hist[slot >> 1] >> ((slot & 1) << 4)) & 0xffffu : 0u;
@@ -866,7 +874,10 @@ hipError_t accumulate_phase(batch_layout &bl, unsigned count, arena &ar, g1_xyzz
     uint32_t *first_table = nullptr;
     // (the digits kernel counts per window tile: a fixed-base job's single
     // segment qualifies when its windows are whole tiles)
-    if (fp.bits > 0 && lds <= DIGITS_MAX_LDS && fp.table_entries < (1ull << 32) && !unaligned) {
+    uint64_t tiles = 0;
+    for (unsigned j = 0; j < count; j++)
+      tiles += ((1u << jt.job[j].log_n) + SEG_TILE - 1) / SEG_TILE;
+    if (fp.bits > 0 && lds <= DIGITS_MAX_LDS && fp.table_entries < (1ull << 32) && !unaligned && tiles >= DIGITS_MIN_TILES) {
       BC_TRY(ar.get(&first_table, fp.table_entries));
       for (unsigned j = 0; j < count; j++)
         jt.job[j].table_begin = (uint32_t)fp.table_begin[j];
@@ -877,7 +888,7 @@ hipError_t accumulate_phase(batch_layout &bl, unsigned count, arena &ar, g1_xyzz
       jt.job[j].digit_block = blocks;
       blocks += ((1u << jt.job[j].log_n) + block_points - 1) / block_points;
     }
-    digits_kernel<<<blocks, MSM_BLOCK, first_table ? lds : 0, s>>>(jt, digits, first_table, fp.bits, block_points);
+    digits_kernel<<<blocks, first_table ? DIGITS_BLOCK : MSM_BLOCK, first_table ? lds : 0, s>>>(jt, digits, first_table, fp.bits, block_points);
     BC_LAUNCH_CHECK();
     BC_TRY(segmented_sort_kv(digits, sorted, groups, count, key_bits, ar, first_table));
     if (first_table)

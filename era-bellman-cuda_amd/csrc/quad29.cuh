@@ -109,4 +109,35 @@ __device__ __forceinline__ f29 quad_from_jacobian(const g1_jacobian *p) {
   return select29(l < 2, c, select29(l == QUAD_ZZZ, zzz, zz));
 }
 
+// XYZZ points in memory hold x, y, zz, zzz: lane l's coordinate is number l ^ 1.
+// In the library's format (coordinates below 2p; infinity has ZZ = 0 mod p):
+__device__ __forceinline__ f29 quad_load_xyzz(const g1_xyzz *p) { return reduce_value29<Fq>(ext_to29(load_fe(&p->x + (quad_lane() ^ 1)))); }
+__device__ __forceinline__ void quad_store_xyzz(g1_xyzz *p, const f29 &c) { store_fe(&p->x + (quad_lane() ^ 1), to_ext<Fq>(c)); }
+
+// and as a partial sum on 29-bit limbs (the accumulators' bounds: X < 2m, the
+// other coordinates products, below 2^257.3, taken below 2m here)
+__device__ __forceinline__ f29 quad_load_xyzz29(const xyzz29 *p) {
+  const uint32_t *w = reinterpret_cast<const uint32_t *>(p) + 9 * (quad_lane() ^ 1);
+  f29 r;
+#pragma unroll
+  for (int i = 0; i < 9; i++)
+    r.v[i] = w[i];
+  return reduce_value29<Fq>(r);
+}
+__device__ __forceinline__ void quad_store_xyzz29(xyzz29 *p, const f29 &c) {
+  uint32_t *w = reinterpret_cast<uint32_t *>(p) + 9 * (quad_lane() ^ 1);
+#pragma unroll
+  for (int i = 0; i < 9; i++)
+    w[i] = c.v[i];
+}
+
+// the point of the quad `quads` quads away (a power of two): lane l ^ 4 quads
+__device__ __forceinline__ f29 quad_from_neighbour(const f29 &a, unsigned quads) {
+  f29 r;
+#pragma unroll
+  for (int i = 0; i < 9; i++)
+    r.v[i] = __shfl_xor(a.v[i], 4 * quads, 64);
+  return r;
+}
+
 } // namespace bc
