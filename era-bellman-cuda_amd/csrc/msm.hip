@@ -356,12 +356,35 @@ __global__ __launch_bounds__(ACC_BLOCK) void accumulate_kernel(const job_table j
 }
 
 // Heavy buckets are reduced in chunks of HEAVY_CHUNK partial sums, one block
-// per chunk: each thread sums HEAVY_PER_THREAD consecutive sums, then a tree in
-// LDS; the chunk's sum overwrites the chunk's first slot.  A second kernel adds
-// a bucket's chunk sums in order into its first slot.
-constexpr unsigned HEAVY_BLOCK = 64;
-constexpr unsigned HEAVY_PER_THREAD = 8;
-constexpr unsigned HEAVY_CHUNK = HEAVY_BLOCK * HEAVY_PER_THREAD;
+// per chunk: a quad of lanes (quad29.cuh) sums every HEAVY_QUADS-th sum, then a
+// tree in LDS; the chunk's sum overwrites the chunk's first slot.  A second
+// kernel adds a bucket's chunk sums into its first slot.  There are few such
+// buckets, so the additions in sequence set the time: 13 by quads, at 2.7 us
+// each, where a thread per point takes 14 at 7 us (2^12 points, 512 sums: 98 -> 41 us).
+constexpr unsigned HEAVY_BLOCK = 256;
+constexpr unsigned HEAVY_QUADS = HEAVY_BLOCK / 4;
+constexpr unsigned HEAVY_CHUNK = HEAVY_QUADS * 8;
+
+// the sum of `n` points (not 0), `stride` apart, in every quad's lanes of quad 0
+__device__ __forceinline__ f29 heavy_block_sum(const xyzz29 *base, uint32_t n, uint32_t stride, f29 (&sh)[HEAVY_QUADS][4]) {
+  const unsigned q = threadIdx.x >> 2, l = quad_lane();
+  f29 acc = f29{}; // infinity
+  if (q < n)
+    acc = quad_load_xyzz29(base + (size_t)q * stride);
+  for (uint32_t i = q + HEAVY_QUADS; i < n; i += HEAVY_QUADS)
+    acc = quad_add(acc, quad_load_xyzz29(base + (size_t)i * stride));
+  unsigned half = HEAVY_QUADS / 2;
+  while (half >= n && half > 0) // the upper halves hold nothing
+    half >>= 1;
+  for (; half > 0; half >>= 1) {
+    sh[q][l] = acc;
+    __syncthreads();
+    if (q < half && q + half < n)
+      acc = quad_add(acc, sh[q + half][l]);
+    __syncthreads();
+  }
+  return acc;
+}
 
 // exclusive prefix of the heavy buckets' chunk counts (one block, chunked)
 __global__ __launch_bounds__(256) void heavy_prefix_kernel(const uint32_t *heavy, const uint32_t *heavy_count, const uint32_t *piece_count,
@@ -393,7 +416,7 @@ __global__ __launch_bounds__(256) void heavy_prefix_kernel(const uint32_t *heavy
 __global__ __launch_bounds__(HEAVY_BLOCK) void heavy_chunk_kernel(xyzz29 *partials, const uint32_t *heavy, const uint32_t *heavy_count,
                                                                   const uint32_t *chunk_offset, const uint32_t *chunk_total,
                                                                   const uint32_t *piece_offset, const uint32_t *piece_count) {
-  __shared__ xyzz29 sh[HEAVY_BLOCK];
+  __shared__ f29 sh[HEAVY_QUADS][4];
   const uint32_t total = *chunk_total, count = *heavy_count;
   for (uint32_t c = blockIdx.x; c < total; c += gridDim.x) {
     uint32_t lo = 0, hi = count; // heavy bucket of chunk c
@@ -405,61 +428,28 @@ __global__ __launch_bounds__(HEAVY_BLOCK) void heavy_chunk_kernel(xyzz29 *partia
         hi = mid;
     }
     const uint32_t b = heavy[lo];
-    const uint32_t np = piece_count[b];
-    xyzz29 *base = partials + piece_offset[b] + (size_t)(c - chunk_offset[lo]) * HEAVY_CHUNK;
-    const uint32_t left = np - (c - chunk_offset[lo]) * HEAVY_CHUNK; // sums from the chunk start
-    xyzz29 acc;
-    bool empty = true;
-    for (uint32_t k = 0; k < HEAVY_PER_THREAD; k++) {
-      const uint32_t q = threadIdx.x * HEAVY_PER_THREAD + k;
-      if (q < left)
-        xyzz29_accumulate29(acc, empty, load_xyzz29(base + q));
-    }
-    sh[threadIdx.x] = empty ? xyzz29_infinity() : acc;
-    __syncthreads();
-    for (unsigned half = HEAVY_BLOCK / 2; half > 0; half >>= 1) {
-      if (threadIdx.x < half) {
-        xyzz29 a = sh[threadIdx.x];
-        bool e = xyzz29_is_infinity(a);
-        xyzz29_accumulate29(a, e, sh[threadIdx.x + half]);
-        sh[threadIdx.x] = e ? xyzz29_infinity() : a;
-      }
-      __syncthreads();
-    }
-    if (threadIdx.x == 0)
-      store_xyzz29_raw(base, sh[0]);
-    __syncthreads();
+    const uint32_t first = (c - chunk_offset[lo]) * HEAVY_CHUNK, left = piece_count[b] - first; // sums from the chunk start
+    xyzz29 *base = partials + piece_offset[b] + first;
+    const f29 sum = heavy_block_sum(base, left < HEAVY_CHUNK ? left : HEAVY_CHUNK, 1, sh);
+    if (threadIdx.x < 4)
+      quad_store_xyzz29(base, sum);
   }
 }
 
-// 4b. one block per heavy bucket (grid-stride): its chunk sums, strided over
-// the threads, then an LDS tree, into the first slot
+// 4b. one block per heavy bucket (grid-stride): its chunk sums into the first slot
 __global__ __launch_bounds__(HEAVY_BLOCK) void heavy_final_kernel(xyzz29 *partials, const uint32_t *heavy, const uint32_t *heavy_count,
                                                                   const uint32_t *piece_offset, const uint32_t *piece_count) {
-  __shared__ xyzz29 sh[HEAVY_BLOCK];
+  __shared__ f29 sh[HEAVY_QUADS][4];
   const uint32_t count = *heavy_count;
   for (uint32_t h = blockIdx.x; h < count; h += gridDim.x) {
     const uint32_t b = heavy[h];
-    xyzz29 *base = partials + piece_offset[b];
     const uint32_t chunks = (piece_count[b] + HEAVY_CHUNK - 1) / HEAVY_CHUNK;
-    xyzz29 acc;
-    bool empty = true;
-    for (uint32_t q = threadIdx.x; q < chunks; q += HEAVY_BLOCK)
-      xyzz29_accumulate29(acc, empty, load_xyzz29(base + (size_t)q * HEAVY_CHUNK));
-    sh[threadIdx.x] = empty ? xyzz29_infinity() : acc;
-    __syncthreads();
-    for (unsigned half = HEAVY_BLOCK / 2; half > 0; half >>= 1) {
-      if (threadIdx.x < half) {
-        xyzz29 a = sh[threadIdx.x];
-        bool e = xyzz29_is_infinity(a);
-        xyzz29_accumulate29(a, e, sh[threadIdx.x + half]);
-        sh[threadIdx.x] = e ? xyzz29_infinity() : a;
-      }
-      __syncthreads();
-    }
-    if (threadIdx.x == 0)
-      store_xyzz29_raw(base, sh[0]);
-    __syncthreads();
+    if (chunks == 1)
+      continue; // the chunk's sum is the bucket's
+    xyzz29 *base = partials + piece_offset[b];
+    const f29 sum = heavy_block_sum(base, chunks, HEAVY_CHUNK, sh);
+    if (threadIdx.x < 4)
+      quad_store_xyzz29(base, sum);
   }
 }
 
@@ -920,7 +910,7 @@ hipError_t accumulate_phase(batch_layout &bl, unsigned count, arena &ar, g1_xyzz
     BC_TRY(ar.get(&chunk_offset, nb));
     heavy_prefix_kernel<<<1, 256, 0, s>>>(heavy, meta, piece_count, chunk_offset, meta + 1);
     BC_LAUNCH_CHECK();
-    heavy_chunk_kernel<<<1024, HEAVY_BLOCK, 0, s>>>(partials, heavy, meta, chunk_offset, meta + 1, piece_offset, piece_count);
+    heavy_chunk_kernel<<<512, HEAVY_BLOCK, 0, s>>>(partials, heavy, meta, chunk_offset, meta + 1, piece_offset, piece_count);
     BC_LAUNCH_CHECK();
     heavy_final_kernel<<<256, HEAVY_BLOCK, 0, s>>>(partials, heavy, meta, piece_offset, piece_count);
     BC_LAUNCH_CHECK();
