@@ -39,9 +39,9 @@ struct msm_job {
 // temporaries come from `ar`, everything is ordered on ar.stream().
 hipError_t msm_batch_device(const msm_job *jobs, unsigned count, arena &ar);
 
-// Threads (one XYZZ point of scratch each) over all bucket-split levels of one
-// job with `windows` bucket windows of width c.
-uint64_t msm_split_threads(unsigned c, unsigned windows);
+// XYZZ points of scratch of one job's bucket reduction (`windows` bucket windows
+// of width c).
+uint64_t msm_split_points(unsigned c, unsigned windows);
 
 // table[w * 2^log_n + i] = [2^(c w)] bases[i], affine Montgomery, for the
 // ceil(254 / c) windows w; bases are valid points (not the affine (0, 0)).

@@ -34,8 +34,9 @@
 //                  of 512 sums: serial sums of 8, then an LDS tree); smaller
 //                  ones are summed as the buckets are gathered into windows;
 //   5. per-bit reduction: windows are split recursively into low/high halves
-//                  of their index bits until each holds one bit (sums split
-//                  across threads, then folded pairwise);
+//                  of their index bits (sums split across threads, then folded,
+//                  or by quads of lanes) until they hold at most 8 bits; then a
+//                  block per window forms its per-bit sums;
 //   6. gather:     254 Jacobian results per job.
 #include <algorithm>
 #include <functional>
@@ -86,7 +87,7 @@ constexpr uint32_t SIGN = 0x80000000u;
 constexpr unsigned MSM_BLOCK = 256;
 constexpr unsigned ACC_BLOCK = 64;
 constexpr unsigned DIGITS_BLOCK = 1024; // threads of a block that also counts (4 points each)
-constexpr unsigned SPLIT_TERMS = 16; // most terms one split thread adds
+constexpr uint64_t SPLIT_THREADS = 1u << 17; // two waves per SIMD
 constexpr unsigned SMALL_PIECES = 32; // buckets of up to this many partial sums are summed by one thread
 // First-digit counters of one digits block.  Measured at 2^24: with 15 KiB of
 // counters (c = 17) counting in the digits kernel saved 0.18 ms over the
@@ -649,7 +650,12 @@ template <bool PREFETCH> __global__ __launch_bounds__(ACC_BLOCK) void split_kern
   store_xyzz29(sg.out + (size_t)part * per_part + ((2 * x + half) << t) + j, acc, empty);
 }
 
-// out[i] += out[i + half] for i < half, per segment
+// out[i] += out[i + half] for i < half, per segment, while that is
+// FOLD_THREADS_MIN additions or more; quads take over below, FOLD_QUADS_MAX of
+// them (a wave per SIMD) where the parts allow.
+constexpr uint64_t FOLD_THREADS_MIN = 1u << 17;
+constexpr uint32_t FOLD_QUADS_MAX = 1u << 14;
+
 struct fold_seg {
   g1_xyzz *out;
   uint32_t half;
@@ -675,13 +681,133 @@ __global__ __launch_bounds__(ACC_BLOCK) void fold_kernel(const fold_table segs, 
   store_xyzz29(sg.out + i, acc, empty);
 }
 
+// The rest of a level's parts, by quads of lanes (quad29.cuh): Q quads share an
+// output, a quad adds every Q-th of its D parts, then the quads' sums meet in a
+// tree over the wave.  A level's fold has few outputs (2816 at 2^12 points), so
+// additions in sequence set its time: one launch of D / Q + log2 Q additions by
+// quads, at 2.7 us, replaces log2 D launches of one at 7 us each.
+struct quad_fold_seg {
+  g1_xyzz *out;
+  uint32_t outputs, D, Q;
+  uint32_t thread_begin; // a multiple of 64
+};
+
+struct quad_fold_table {
+  uint32_t count;
+  quad_fold_seg seg[MSM_MAX_JOBS];
+};
+
+__global__ __launch_bounds__(ACC_BLOCK) void quad_fold_kernel(const quad_fold_table segs) {
+  const uint32_t id_all = blockIdx.x * ACC_BLOCK + threadIdx.x;
+  const quad_fold_seg &sg = segs.seg[find_seg(segs, id_all)];
+  const uint32_t quad = (id_all - sg.thread_begin) >> 2;
+  const uint32_t i = quad / sg.Q, q = quad % sg.Q;
+  if (i >= sg.outputs)
+    return; // padding; a wave serves one segment, an output's quads leave together
+  f29 acc = quad_load_xyzz(sg.out + (size_t)q * sg.outputs + i);
+  for (uint32_t part = q + sg.Q; part < sg.D; part += sg.Q)
+    acc = quad_add(acc, quad_load_xyzz(sg.out + (size_t)part * sg.outputs + i));
+  for (uint32_t off = sg.Q >> 1; off > 0; off >>= 1)
+    acc = quad_add(acc, quad_from_neighbour(acc, off));
+  if (q == 0)
+    quad_store_xyzz(sg.out + i, acc);
+}
+
+// A whole split level by quads, for small levels: Q quads share an output sum
+// (Q << (t - hs) in the high half, whose sums are longer), a quad adds every Q-th
+// term, and the quads' sums meet in a tree over the wave, so the level needs no
+// parts and no folds.  A thread per part adds in half the SIMD time, a quad in
+// under half the latency: at 2^12 points (90 K terms) 34 us against 51 us for
+// parts and their fold, at 2^18 (557 K terms) 167 us against 115 us.
+constexpr uint64_t QUAD_SPLIT_TERMS = 1u << 18; // levels of fewer terms
+struct quad_split_seg {
+  const g1_xyzz *A;
+  g1_xyzz *out;
+  uint32_t X, s, Q;
+  uint32_t thread_begin; // a multiple of 64
+};
+
+struct quad_split_table {
+  uint32_t count;
+  quad_split_seg seg[MSM_MAX_JOBS];
+};
+
+__global__ __launch_bounds__(ACC_BLOCK) void quad_split_kernel(const quad_split_table segs) {
+  const uint32_t id_all = blockIdx.x * ACC_BLOCK + threadIdx.x;
+  const quad_split_seg &sg = segs.seg[find_seg(segs, id_all)];
+  const unsigned s = sg.s, t = (s + 1) >> 1, hs = s - t;
+  // a window's half takes Q << t quads (a multiple of 16: a wave has one half)
+  const uint32_t quad = (id_all - sg.thread_begin) >> 2, per_half = sg.Q << t;
+  const uint32_t x = quad / (2 * per_half), half = (quad / per_half) & 1, in_half = quad % per_half;
+  const uint32_t Q = half ? sg.Q << (t - hs) : sg.Q, j = in_half / Q, q = in_half % Q;
+  const g1_xyzz *src = sg.A + ((size_t)x << s);
+  // terms q, q + Q, ... at src[(term << t) | j] (low half, 2^hs of them) or src[(j << t) | term] (high half, 2^t)
+  const uint32_t terms = half ? 1u << t : 1u << hs;
+  auto term = [&](uint32_t i) { return src + (half ? (j << t) | i : (i << t) | j); };
+  f29 acc = quad_load_xyzz(term(q));
+  for (uint32_t i = q + Q; i < terms; i += Q)
+    acc = quad_add(acc, quad_load_xyzz(term(i)));
+  for (uint32_t off = Q >> 1; off > 0; off >>= 1)
+    acc = quad_add(acc, quad_from_neighbour(acc, off));
+  if (q == 0) {
+    g1_xyzz *out = sg.out + ((size_t)(2 * x + half) << t) + j;
+    quad_store_xyzz(out, acc);
+    if (half && hs < t) // the high child has one bit less: its upper half is infinity
+      quad_store_xyzz(out + (1u << hs), f29{});
+  }
+}
+
+// Windows of s <= BITS_WIDTH bits, a block each, down to their per-bit sums:
+// bits[x s + j] = the sum of the points of window x whose index has bit j set.
+// In round r the lists of 2^(s - r) points at offsets 0 and 2^j, j >= s - r, are
+// halved, L[i] += L[i + half]; the upper half of the list at 0 becomes the list
+// at 2^(s - r - 1), the sum of bit s - r - 1.  About 2 2^s additions by quads, in
+// s rounds of one LDS barrier, replace the splits and folds of the last three
+// levels (nine launches).
+constexpr unsigned BITS_WIDTH = 8;
+constexpr unsigned BITS_BLOCK = 256, BITS_QUADS = BITS_BLOCK / 4;
+
+struct bits_seg {
+  const g1_xyzz *A;
+  g1_xyzz *bits;
+  uint32_t s;
+  uint32_t thread_begin; // first window (block) of the job
+};
+
+struct bits_table {
+  uint32_t count;
+  bits_seg seg[MSM_MAX_JOBS];
+};
+
+__global__ __launch_bounds__(BITS_BLOCK) void bits_kernel(const bits_table segs) {
+  __shared__ f29 pts[1u << BITS_WIDTH][4];
+  const bits_seg &sg = segs.seg[find_seg(segs, blockIdx.x)];
+  const uint32_t x = blockIdx.x - sg.thread_begin, s = sg.s;
+  const unsigned quad = threadIdx.x >> 2, l = quad_lane();
+  for (uint32_t i = quad; i < (1u << s); i += BITS_QUADS)
+    pts[i][l] = quad_load_xyzz(sg.A + ((size_t)x << s) + i);
+  __syncthreads();
+  for (uint32_t r = 0; r < s; r++) {
+    const uint32_t log_half = s - 1 - r;
+    for (uint32_t k = quad; k < ((r + 1) << log_half); k += BITS_QUADS) {
+      const uint32_t list = k >> log_half, i = k & ((1u << log_half) - 1);
+      const uint32_t at = (list == 0 ? 0u : 1u << (s - list)) + i;
+      pts[at][l] = quad_add(pts[at][l], pts[at + (1u << log_half)][l]);
+    }
+    __syncthreads();
+  }
+  if (quad < s)
+    quad_store_xyzz(sg.bits + (size_t)x * s + quad, pts[1u << quad][l]);
+}
+
 // 6. bit i = w*c + j of a job is its window's top bucket (j == c-1 or i == 253),
-// else bucket 1 of the one-bit window reached by following the splits: a width-s
-// window x holds bits [0, t) in child 2x and [t, s) in child 2x+1, t = ceil(s/2).
+// else the bit's sum in the window reached by following the splits: a width-s
+// window x holds bits [0, t) in child 2x and [t, s) in child 2x+1, t = ceil(s/2),
+// down to the BITS_WIDTH bits whose sums bits_kernel left.
 // A job over a fixed-base table has one window: bits [0, c) as above, the
 // bits above are infinity (its fold is the same point).
 struct result_desc {
-  const g1_xyzz *A_final;
+  const g1_xyzz *bits;
   const g1_xyzz *tops;
   g1_jacobian *out;
   uint32_t c;
@@ -712,7 +838,7 @@ __global__ void result_kernel(const result_table jobs) {
     v = load_xyzz(rd.tops + w);
   } else {
     uint32_t x = w, s = c - 1;
-    while (s > 1) {
+    while (s > BITS_WIDTH) {
       const uint32_t half = (s + 1) >> 1;
       if (j < half) {
         x = 2 * x;
@@ -722,7 +848,7 @@ __global__ void result_kernel(const result_table jobs) {
       }
       s = half;
     }
-    v = load_xyzz(rd.A_final + 2 * (size_t)x + 1);
+    v = load_xyzz(rd.bits + (size_t)x * s + j);
   }
   const g1_jacobian r = xyzz_to_jacobian(v);
   store_fe(&rd.out[i].x, r.x);
@@ -732,32 +858,47 @@ __global__ void result_kernel(const result_table jobs) {
 
 } // namespace
 
-// Parts D_lo of the low half of a split level (X windows of `width` bits):
-// each split thread adds 2^hs / D_lo terms, SPLIT_TERMS where the level has
-// work enough for 2^16 threads and fewer (down to 2) on small levels, whose
-// serial chains would otherwise set the time.  A function of the job alone,
-// so a job's sums are the same alone and in any batch.
 namespace {
 
+// Both are functions of the job alone, so a job's sums are the same alone and in
+// any batch.
+//
+// Parts D_lo of the low half of a split level (X windows of `width` bits): each
+// split thread adds 2^hs / D_lo terms: 16 where that leaves SPLIT_THREADS
+// threads, else 8 (2^20 points: 187 -> 109 us of splits for 28 us more of folds;
+// at 2^18 four terms cost 49 us more of folds than they save of splits).
 uint32_t split_parts(uint32_t X, unsigned width) {
   const unsigned hs = width - (width + 1) / 2;
   const uint64_t level_terms = (uint64_t)(2 * X) << width;
-  unsigned terms = SPLIT_TERMS;
-  while (terms > 2 && level_terms / terms < (1u << 16))
-    terms >>= 1;
+  const unsigned terms = level_terms / 16 >= SPLIT_THREADS ? 16 : 8;
   return (1u << hs) > terms ? (1u << hs) / terms : 1u;
+}
+
+bool split_by_quads(uint32_t X, unsigned width) { return (uint64_t)(2 * X) << width < QUAD_SPLIT_TERMS; }
+
+// Quads per low-half sum of such a level: up to a wave per SIMD, and no more
+// than 4, whose tree is a small part of the additions.
+uint32_t split_quads(uint32_t X, unsigned width) {
+  uint32_t Q = 1;
+  while (Q < 4 && ((uint64_t)(2 * X) * 2 * Q << ((width + 1) / 2)) <= FOLD_QUADS_MAX)
+    Q *= 2;
+  return Q;
 }
 
 } // namespace
 
-uint64_t msm_split_threads(unsigned c, unsigned windows) {
+// Points (of 128 bytes) the reduction of one job's windows keeps: the windows
+// (in parts) of every split level and the per-bit sums.
+uint64_t msm_split_points(unsigned c, unsigned windows) {
   uint64_t total = 0;
   uint32_t X = windows;
-  for (unsigned width = c - 1; width > 1; width = (width + 1) / 2, X *= 2) {
+  unsigned width = c - 1;
+  for (; width > BITS_WIDTH; width = (width + 1) / 2, X *= 2) {
     const unsigned t = (width + 1) / 2, hs = width - t;
-    total += ((uint64_t)split_parts(X, width) << (t - hs)) * ((uint64_t)(2 * X) << t);
+    const uint64_t D = split_by_quads(X, width) ? 1 : (uint64_t)split_parts(X, width) << (t - hs);
+    total += D * (2 * (uint64_t)X << t);
   }
-  return total;
+  return total + (uint64_t)X * width;
 }
 
 namespace {
@@ -838,8 +979,10 @@ hipError_t accumulate_phase(batch_layout &bl, unsigned count, arena &ar, g1_xyzz
   // 1-2. digits, sort, bucket runs
   uint32_t *offsets = nullptr, *counts = nullptr;
   uint64_t *sorted = nullptr; // (key, point reference) pairs, sorted by key within each window
-  BC_TRY(ar.get(&offsets, nb));
-  BC_TRY(ar.get(&counts, nb));
+  // offsets, counts and meta = {heavy count, heavy chunk total} are cleared together
+  BC_TRY(ar.get(&offsets, 2 * (uint64_t)nb + 2));
+  counts = offsets + nb;
+  uint32_t *const meta = counts + nb;
   BC_TRY(ar.get(&sorted, entries));
   {
     uint64_t *digits = nullptr;
@@ -887,18 +1030,14 @@ hipError_t accumulate_phase(batch_layout &bl, unsigned count, arena &ar, g1_xyzz
   }
 
   // 3. accumulation over chunks of the sorted entries, which also records each
-  // bucket's run [offsets[b], counts[b]) (empty buckets keep [0, 0));
-  // meta = {heavy count, heavy chunk total}
-  uint32_t *piece_count = nullptr, *piece_offset = nullptr, *meta = nullptr, *heavy = nullptr;
+  // bucket's run [offsets[b], counts[b]) (empty buckets keep [0, 0))
+  uint32_t *piece_count = nullptr, *piece_offset = nullptr, *heavy = nullptr;
   xyzz29 *partials = nullptr; // on 29-bit limbs, 144 B each
   BC_TRY(ar.get(&piece_count, nb));
   BC_TRY(ar.get(&piece_offset, nb));
-  BC_TRY(ar.get(&meta, 2));
   BC_TRY(ar.get(&partials, slots));
   BC_TRY(ar.get(&heavy, nb));
-  BC_TRY(fill_u32(offsets, nb, 0, s));
-  BC_TRY(fill_u32(counts, nb, 0, s));
-  BC_TRY(fill_u32(meta, 2, 0, s));
+  BC_TRY(fill_u32(offsets, 2 * (uint64_t)nb + 2, 0, s));
   accumulate_kernel<<<grid_for(chunks, ACC_BLOCK), ACC_BLOCK, 0, s>>>(jt, sorted, (uint32_t)chunks, partials, offsets, counts);
   BC_LAUNCH_CHECK();
   bucket_slots_kernel<<<grid_for(nb, MSM_BLOCK), MSM_BLOCK, 0, s>>>(jt, offsets, counts, piece_offset, piece_count, nb, heavy, meta);
@@ -933,8 +1072,7 @@ hipError_t accumulate_phase(batch_layout &bl, unsigned count, arena &ar, g1_xyzz
   else
     bucket_gather_kernel<false><<<grid_for(nb, MSM_BLOCK), MSM_BLOCK, 0, s>>>(jt, nb, partials, piece_offset, piece_count, A, tops, add);
   BC_LAUNCH_CHECK();
-  for (void *p : {(void *)partials, (void *)piece_offset, (void *)piece_count, (void *)meta, (void *)offsets, (void *)counts,
-                  (void *)sorted})
+  for (void *p : {(void *)partials, (void *)piece_offset, (void *)piece_count, (void *)sorted, (void *)offsets})
     BC_TRY(ar.put(p));
   return hipSuccess;
 }
@@ -953,65 +1091,122 @@ hipError_t reduce_phase(const batch_layout &bl, const msm_job *jobs, unsigned co
   }
   for (;;) {
     split_table st{};
-    std::vector<unsigned> active;
-    std::vector<uint32_t> per_part;
-    uint64_t threads = 0;
+    quad_split_table qs{};
+    std::vector<uint32_t> per_part, parts;
+    uint64_t points = 0, threads = 0, quad_threads = 0;
+    unsigned wide = 0;
     for (unsigned j = 0; j < count; j++) {
-      if (width[j] <= 1)
+      if (width[j] <= BITS_WIDTH)
         continue;
+      wide++;
       const unsigned t = (width[j] + 1) / 2, hs = width[j] - t;
-      const uint32_t D_lo = split_parts(X[j], width[j]);
-      split_seg &sg = st.seg[st.count++];
-      sg.A = cur[j];
-      sg.X = X[j];
-      sg.s = width[j];
-      sg.D_lo = D_lo;
-      sg.D = D_lo << (t - hs);
-      sg.thread_begin = (uint32_t)threads;
-      per_part.push_back((2 * X[j]) << t);
-      threads += (uint64_t)sg.D * per_part.back();
-      active.push_back(j);
+      const uint32_t sums = (2 * X[j]) << t;
+      if (split_by_quads(X[j], width[j])) {
+        const uint32_t Q = split_quads(X[j], width[j]);
+        qs.seg[qs.count++] = {cur[j], nullptr, X[j], width[j], Q, (uint32_t)quad_threads};
+        quad_threads += 4ull * Q * sums;
+        points += sums;
+      } else {
+        const uint32_t D_lo = split_parts(X[j], width[j]), D = D_lo << (t - hs);
+        st.seg[st.count++] = {cur[j], nullptr, X[j], width[j], D_lo, D, (uint32_t)threads};
+        per_part.push_back(sums);
+        parts.push_back(D);
+        threads += (uint64_t)D * sums;
+        points += (uint64_t)D * sums;
+      }
     }
-    if (active.empty())
+    if (wide == 0)
       break;
-    if (threads >= (1ull << 32))
+    if (threads >= (1ull << 32) || quad_threads >= (1ull << 32))
       return hipErrorInvalidValue;
     g1_xyzz *next = nullptr;
-    BC_TRY(ar.get(&next, threads));
+    BC_TRY(ar.get(&next, points));
     level_buffers.push_back(next);
-    for (unsigned k = 0; k < st.count; k++)
-      st.seg[k].out = next + st.seg[k].thread_begin;
+    for (unsigned j = 0, k = 0, q = 0; j < count; j++) {
+      if (width[j] <= BITS_WIDTH)
+        continue;
+      const unsigned t = (width[j] + 1) / 2;
+      const uint32_t sums = (2 * X[j]) << t;
+      const bool quads = split_by_quads(X[j], width[j]);
+      cur[j] = next;
+      if (quads)
+        qs.seg[q++].out = next;
+      else
+        st.seg[k].out = next;
+      next += quads ? sums : (uint64_t)sums * st.seg[k++].D;
+      X[j] *= 2;
+      width[j] = t;
+    }
+    if (qs.count) {
+      quad_split_kernel<<<(unsigned)(quad_threads / ACC_BLOCK), ACC_BLOCK, 0, s>>>(qs);
+      BC_LAUNCH_CHECK();
+    }
+    if (st.count == 0)
+      continue;
     if (threads < SPLIT_PREFETCH_BELOW)
       split_kernel<true><<<grid_for(threads, ACC_BLOCK), ACC_BLOCK, 0, s>>>(st, (uint32_t)threads);
     else
       split_kernel<false><<<grid_for(threads, ACC_BLOCK), ACC_BLOCK, 0, s>>>(st, (uint32_t)threads);
     BC_LAUNCH_CHECK();
-    // fold round r halves every segment that still holds more than one part
-    for (unsigned r = 0;; r++) {
+    // rounds that halve the parts, a thread per sum, while they fill the GPU
+    // (again a rule on the job alone), then quads
+    for (;;) {
       fold_table ft{};
       uint32_t fthreads = 0;
       for (unsigned k = 0; k < st.count; k++) {
-        const uint32_t d = st.seg[k].D >> (r + 1);
-        if (d == 0)
+        const uint64_t half = (uint64_t)(parts[k] / 2) * per_part[k];
+        if (half < FOLD_THREADS_MIN)
           continue;
         fold_seg &fs = ft.seg[ft.count++];
         fs.out = st.seg[k].out;
-        fs.half = d * per_part[k];
+        fs.half = (uint32_t)half;
         fs.thread_begin = fthreads;
         fthreads += fs.half;
+        parts[k] /= 2;
       }
       if (ft.count == 0)
         break;
       fold_kernel<<<grid_for(fthreads, ACC_BLOCK), ACC_BLOCK, 0, s>>>(ft, fthreads);
       BC_LAUNCH_CHECK();
     }
+    quad_fold_table qt{};
+    uint32_t qthreads = 0;
     for (unsigned k = 0; k < st.count; k++) {
-      const unsigned j = active[k];
-      cur[j] = st.seg[k].out;
-      X[j] *= 2;
-      width[j] = (width[j] + 1) / 2;
+      if (parts[k] < 2)
+        continue;
+      quad_fold_seg &qf = qt.seg[qt.count++];
+      qf.out = st.seg[k].out;
+      qf.outputs = per_part[k];
+      qf.D = parts[k];
+      qf.Q = 1;
+      while (qf.Q < 8 && 2 * qf.Q < qf.D && 2 * qf.Q * qf.outputs <= FOLD_QUADS_MAX)
+        qf.Q *= 2;
+      qf.thread_begin = qthreads;
+      qthreads += (4 * qf.Q * qf.outputs + 63) & ~63u;
+    }
+    if (qt.count) {
+      quad_fold_kernel<<<qthreads / ACC_BLOCK, ACC_BLOCK, 0, s>>>(qt);
+      BC_LAUNCH_CHECK();
     }
   }
+
+  bits_table bt{};
+  uint32_t windows = 0;
+  uint64_t sums = 0;
+  for (unsigned j = 0; j < count; j++)
+    sums += (uint64_t)X[j] * width[j];
+  g1_xyzz *bits = nullptr;
+  BC_TRY(ar.get(&bits, sums));
+  level_buffers.push_back(bits);
+  bt.count = count;
+  for (unsigned j = 0; j < count; j++) {
+    bt.seg[j] = {cur[j], bits, width[j], windows};
+    cur[j] = bits;
+    bits += X[j] * width[j];
+    windows += X[j];
+  }
+  bits_kernel<<<windows, BITS_BLOCK, 0, s>>>(bt);
+  BC_LAUNCH_CHECK();
 
   // 6. results
   result_table rt{};
@@ -1020,8 +1215,10 @@ hipError_t reduce_phase(const batch_layout &bl, const msm_job *jobs, unsigned co
     rt.job[j] = {cur[j], tops + jt.job[j].top_begin, jobs[j].results, jt.job[j].c, jt.job[j].stride ? 1u : 0u};
   result_kernel<<<grid_for(254 * count, 256), 256, 0, s>>>(rt);
   BC_LAUNCH_CHECK();
-  for (g1_xyzz *p : level_buffers)
-    BC_TRY(ar.put(p));
+  while (!level_buffers.empty()) {
+    BC_TRY(ar.put(level_buffers.back()));
+    level_buffers.pop_back();
+  }
   return hipSuccess;
 }
 

@@ -88,17 +88,15 @@ __device__ __forceinline__ f29 quad_add(const f29 &p, const f29 &q) {
   const f29 r4 = mul29<Fq>(select29(l == 0, r1, select29(l == 1, R, r2)), select29(l == 1, QX, PPP)); // S1 PPP, R (Q - X3), ZZZ3
   const f29 Y3 = norm29(sub29(quad_broadcast<QUAD_X>(r4), r4, P::c2));
   f29 s = select29(l == QUAD_Y, Y3, select29(l == QUAD_X, X3, select29(l == QUAD_ZZZ, r4, r3)));
-  if (p_inf)
-    s = q;
-  else if (q_inf)
-    s = p;
-  else if (same_x) {
-    if (same_y)
-      s = quad_dbl(p);
-    else
-      s = f29{}; // q = -p: infinity
+  // infinities by selects, equal and opposite points behind a branch of the
+  // whole wave: as lanes' branches the doubling was executed by every addition
+  const bool special = same_x && !p_inf && !q_inf;
+  if (__any(special)) {
+    const f29 twice = quad_dbl(p);
+    if (special)
+      s = same_y ? twice : f29{}; // q = -p: infinity
   }
-  return s;
+  return select29(p_inf, q, select29(q_inf, p, s));
 }
 
 // A Jacobian point of the library's format (coordinates below 2p); infinity has Z = 0.
