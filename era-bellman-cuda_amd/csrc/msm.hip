@@ -88,7 +88,6 @@ constexpr unsigned MSM_BLOCK = 256;
 constexpr unsigned ACC_BLOCK = 64;
 constexpr unsigned DIGITS_BLOCK = 1024; // threads of a block that also counts (4 points each)
 constexpr uint64_t SPLIT_THREADS = 1u << 17; // two waves per SIMD
-constexpr unsigned SMALL_PIECES = 32; // buckets of up to this many partial sums are summed by one thread
 // First-digit counters of one digits block.  Measured at 2^24: with 15 KiB of
 // counters (c = 17) counting in the digits kernel saved 0.18 ms over the
 // sort's own count; with 27 KiB (c = 20) it saved nothing.
@@ -116,6 +115,7 @@ struct job_desc {
   uint8_t c;             // window bits
   uint8_t Wd;            // digit windows of a scalar, ceil(254 / c)
   uint8_t W;             // bucket windows: Wd, or 1 over a fixed-base table
+  uint8_t small;         // partial sums of a bucket that one thread of the gather adds
 };
 
 static_assert(MSM_MAX_JOBS <= SEG_MAX_GROUPS, "one sort segment group per job");
@@ -263,11 +263,36 @@ __global__ __launch_bounds__(DIGITS_BLOCK) void digits_kernel(const job_table jo
 // starts (ends), from the keys before and after it, so no separate pass over
 // the sorted entries is needed.
 
+// Buckets of up to d.small partial sums are summed by one thread of the gather,
+// those of up to MEDIUM_PIECES by a wave of quads, larger ones by blocks of quads
+// in chunks of HEAVY_CHUNK.  The additions of a thread take 7 us each in
+// sequence, so the line (a rule on the job alone) lies at twice the sums of an
+// average bucket, where few buckets are left to the waves; a witness has some:
+// the window where its small scalars end (13 sums at 2^12 points), the top
+// window (9 at 2^20, 15 at 2^24).  At 2^12 points the gather takes 23 us instead
+// of 112 for 12 us more of waves.
+uint8_t small_pieces(const job_desc &d) {
+  const uint64_t entries_per_bucket = ((uint64_t)(d.stride ? d.Wd : 1u) << d.log_n) >> (d.c - 1);
+  return (uint8_t)std::min<uint64_t>(4 + 2 * (entries_per_bucket / d.piece), 32);
+}
+constexpr uint32_t MEDIUM_PIECES = 64;
+constexpr unsigned HEAVY_BLOCK = 256;
+constexpr unsigned HEAVY_QUADS = HEAVY_BLOCK / 4;
+constexpr unsigned HEAVY_CHUNK = HEAVY_QUADS * 8;
+
+// Work lists of the buckets that the gather does not sum itself: medium buckets,
+// (bucket, chunk) pairs of heavy ones, and heavy buckets of several chunks.
+// count[0..2] are their lengths.  Their order varies from run to run; what is
+// summed in which order does not.
+struct piece_lists {
+  uint32_t *count, *medium, *several;
+  uint2 *chunks;
+};
+
 // piece_offset[b], piece_count[b]: the slots of bucket b's sums, from its run
-// [start, end) of sorted entries (empty buckets have none).  Buckets of more
-// than SMALL_PIECES sums (a few at most) are listed for the heavy fix-up.
+// [start, end) of sorted entries (empty buckets have none).
 __global__ void bucket_slots_kernel(const job_table jobs, const uint32_t *start, const uint32_t *end, uint32_t *piece_offset, uint32_t *piece_count,
-                                    unsigned nb, uint32_t *heavy, uint32_t *heavy_count) {
+                                    unsigned nb, const piece_lists lists) {
   const unsigned b = blockIdx.x * blockDim.x + threadIdx.x;
   if (b >= nb)
     return;
@@ -281,8 +306,24 @@ __global__ void bucket_slots_kernel(const job_table jobs, const uint32_t *start,
   }
   piece_offset[b] = off;
   piece_count[b] = np;
-  if (np > SMALL_PIECES)
-    heavy[atomicAdd(heavy_count, 1u)] = b;
+  if (np > MEDIUM_PIECES) {
+    const uint32_t chunks = (np + HEAVY_CHUNK - 1) / HEAVY_CHUNK;
+    const uint32_t at = atomicAdd(lists.count + 1, chunks);
+    for (uint32_t k = 0; k < chunks; k++)
+      lists.chunks[at + k] = make_uint2(b, k);
+    if (chunks > 1)
+      lists.several[atomicAdd(lists.count + 2, 1u)] = b;
+  }
+  // one atomic per wave: the top window's buckets are all medium, side by side
+  const bool medium = np > jd.small && np <= MEDIUM_PIECES;
+  const uint64_t mask = __ballot(medium);
+  if (medium) {
+    const unsigned lane = threadIdx.x & 63, before = __popcll(mask & ((1ull << lane) - 1)), leader = (unsigned)__ffsll((unsigned long long)mask) - 1;
+    uint32_t at = 0;
+    if (before == 0)
+      at = atomicAdd(lists.count, (uint32_t)__popcll(mask));
+    lists.medium[__shfl(at, leader, 64) + before] = b;
+  }
 }
 
 __global__ __launch_bounds__(ACC_BLOCK) void accumulate_kernel(const job_table jobs, const uint64_t *__restrict__ sorted, uint32_t chunks,
@@ -362,9 +403,6 @@ __global__ __launch_bounds__(ACC_BLOCK) void accumulate_kernel(const job_table j
 // kernel adds a bucket's chunk sums into its first slot.  There are few such
 // buckets, so the additions in sequence set the time: 13 by quads, at 2.7 us
 // each, where a thread per point takes 14 at 7 us (2^12 points, 512 sums: 98 -> 41 us).
-constexpr unsigned HEAVY_BLOCK = 256;
-constexpr unsigned HEAVY_QUADS = HEAVY_BLOCK / 4;
-constexpr unsigned HEAVY_CHUNK = HEAVY_QUADS * 8;
 
 // the sum of `n` points (not 0), `stride` apart, in every quad's lanes of quad 0
 __device__ __forceinline__ f29 heavy_block_sum(const xyzz29 *base, uint32_t n, uint32_t stride, f29 (&sh)[HEAVY_QUADS][4]) {
@@ -387,68 +425,47 @@ __device__ __forceinline__ f29 heavy_block_sum(const xyzz29 *base, uint32_t n, u
   return acc;
 }
 
-// exclusive prefix of the heavy buckets' chunk counts (one block, chunked)
-__global__ __launch_bounds__(256) void heavy_prefix_kernel(const uint32_t *heavy, const uint32_t *heavy_count, const uint32_t *piece_count,
-                                                           uint32_t *chunk_offset, uint32_t *chunk_total) {
-  __shared__ uint32_t sh[256];
-  const uint32_t count = *heavy_count;
-  uint32_t carry = 0;
-  for (uint32_t base = 0; base < count; base += 256) {
-    const uint32_t i = base + threadIdx.x;
-    const uint32_t v = i < count ? (piece_count[heavy[i]] + HEAVY_CHUNK - 1) / HEAVY_CHUNK : 0;
-    sh[threadIdx.x] = v;
-    __syncthreads();
-    for (unsigned off = 1; off < 256; off <<= 1) {
-      const uint32_t t = threadIdx.x >= off ? sh[threadIdx.x - off] : 0;
-      __syncthreads();
-      sh[threadIdx.x] += t;
-      __syncthreads();
-    }
-    if (i < count)
-      chunk_offset[i] = carry + sh[threadIdx.x] - v;
-    carry += sh[255];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0)
-    *chunk_total = carry;
-}
-
-// 4a. one block per chunk (grid-stride over all chunks of all heavy buckets)
-__global__ __launch_bounds__(HEAVY_BLOCK) void heavy_chunk_kernel(xyzz29 *partials, const uint32_t *heavy, const uint32_t *heavy_count,
-                                                                  const uint32_t *chunk_offset, const uint32_t *chunk_total,
-                                                                  const uint32_t *piece_offset, const uint32_t *piece_count) {
+// 4a. one block per chunk of a heavy bucket, then one wave per medium bucket: a
+// quad sums every 16th partial sum and the quads' sums meet in a tree over the
+// wave, in the bucket's first slot (grid-stride over both lists)
+__global__ __launch_bounds__(HEAVY_BLOCK) void heavy_chunk_kernel(xyzz29 *partials, const piece_lists lists, const uint32_t *piece_offset,
+                                                                  const uint32_t *piece_count) {
   __shared__ f29 sh[HEAVY_QUADS][4];
-  const uint32_t total = *chunk_total, count = *heavy_count;
-  for (uint32_t c = blockIdx.x; c < total; c += gridDim.x) {
-    uint32_t lo = 0, hi = count; // heavy bucket of chunk c
-    while (hi - lo > 1) {
-      const uint32_t mid = (lo + hi) >> 1;
-      if (chunk_offset[mid] <= c)
-        lo = mid;
-      else
-        hi = mid;
-    }
-    const uint32_t b = heavy[lo];
-    const uint32_t first = (c - chunk_offset[lo]) * HEAVY_CHUNK, left = piece_count[b] - first; // sums from the chunk start
-    xyzz29 *base = partials + piece_offset[b] + first;
+  const uint32_t chunks = lists.count[1], medium = lists.count[0];
+  for (uint32_t c = blockIdx.x; c < chunks; c += gridDim.x) {
+    const uint2 ch = lists.chunks[c];
+    const uint32_t first = ch.y * HEAVY_CHUNK, left = piece_count[ch.x] - first; // sums from the chunk start
+    xyzz29 *base = partials + piece_offset[ch.x] + first;
     const f29 sum = heavy_block_sum(base, left < HEAVY_CHUNK ? left : HEAVY_CHUNK, 1, sh);
     if (threadIdx.x < 4)
       quad_store_xyzz29(base, sum);
   }
+  const unsigned q = (threadIdx.x & 63) >> 2;
+  for (uint32_t m = blockIdx.x * (HEAVY_BLOCK / 64) + (threadIdx.x >> 6); m < medium; m += gridDim.x * (HEAVY_BLOCK / 64)) {
+    const uint32_t b = lists.medium[m], np = piece_count[b];
+    xyzz29 *base = partials + piece_offset[b];
+    f29 acc = f29{};
+    if (q < np)
+      acc = quad_load_xyzz29(base + q);
+    for (uint32_t i = q + 16; i < np; i += 16)
+      acc = quad_add(acc, quad_load_xyzz29(base + i));
+    for (uint32_t off = 8; off > 0; off >>= 1)
+      if (off < np) // the sums off.. of a smaller bucket are infinity
+        acc = quad_add(acc, quad_from_neighbour(acc, off));
+    if (q == 0)
+      quad_store_xyzz29(base, acc);
+  }
 }
 
-// 4b. one block per heavy bucket (grid-stride): its chunk sums into the first slot
-__global__ __launch_bounds__(HEAVY_BLOCK) void heavy_final_kernel(xyzz29 *partials, const uint32_t *heavy, const uint32_t *heavy_count,
-                                                                  const uint32_t *piece_offset, const uint32_t *piece_count) {
+// 4b. one block per heavy bucket of several chunks (grid-stride): its chunk sums into the first slot
+__global__ __launch_bounds__(HEAVY_BLOCK) void heavy_final_kernel(xyzz29 *partials, const piece_lists lists, const uint32_t *piece_offset,
+                                                                  const uint32_t *piece_count) {
   __shared__ f29 sh[HEAVY_QUADS][4];
-  const uint32_t count = *heavy_count;
+  const uint32_t count = lists.count[2];
   for (uint32_t h = blockIdx.x; h < count; h += gridDim.x) {
-    const uint32_t b = heavy[h];
-    const uint32_t chunks = (piece_count[b] + HEAVY_CHUNK - 1) / HEAVY_CHUNK;
-    if (chunks == 1)
-      continue; // the chunk's sum is the bucket's
+    const uint32_t b = lists.several[h];
     xyzz29 *base = partials + piece_offset[b];
-    const f29 sum = heavy_block_sum(base, chunks, HEAVY_CHUNK, sh);
+    const f29 sum = heavy_block_sum(base, (piece_count[b] + HEAVY_CHUNK - 1) / HEAVY_CHUNK, HEAVY_CHUNK, sh);
     if (threadIdx.x < 4)
       quad_store_xyzz29(base, sum);
   }
@@ -463,8 +480,8 @@ __global__ __launch_bounds__(HEAVY_BLOCK) void heavy_final_kernel(xyzz29 *partia
 // it.  With `first`, the window's infinity stores are made here.
 struct gather_item {
   g1_xyzz *dst;
-  uint32_t off, np;
-  bool live; // false: nothing to store for this bucket
+  uint32_t off, np; // np: the sums to add here, 1 when they were added before
+  bool live;        // false: nothing to store for this bucket
 };
 
 __device__ __forceinline__ gather_item gather_prepare(const job_table &jobs, uint32_t t, const uint32_t *__restrict__ piece_offset,
@@ -490,15 +507,17 @@ __device__ __forceinline__ gather_item gather_prepare(const job_table &jobs, uin
   const uint32_t d = k == 0 ? B : k;
   const uint32_t b = jd.bucket_begin + w * B + d - 1;
   g.np = piece_count[b];
+  if (g.np > jd.small)
+    g.np = 1;
   g.off = piece_offset[b];
   g.dst = to_top ? tops + jd.top_begin + w : A + t;
   g.live = !(add && g.np == 0); // nothing of this launch to add
   return g;
 }
 
-// buckets of 2..SMALL_PIECES sums are summed here, a heavy bucket's sum is
+// buckets of 2..jd.small sums are summed here; the sum of a larger one is
 // already in its first slot
-__device__ __forceinline__ bool gather_sums(const gather_item &g) { return g.live && g.np >= 2 && g.np <= SMALL_PIECES; }
+__device__ __forceinline__ bool gather_sums(const gather_item &g) { return g.live && g.np >= 2; }
 
 __device__ __forceinline__ void gather_finish(const gather_item &g, const xyzz29 *__restrict__ partials, bool add) {
   // the partial sums are on 29-bit limbs; the window arrays take the library's format
@@ -507,9 +526,8 @@ __device__ __forceinline__ void gather_finish(const gather_item &g, const xyzz29
   if (g.np != 0) {
     acc = load_xyzz29(partials + g.off);
     empty = xyzz29_is_infinity(acc);
-    if (g.np <= SMALL_PIECES)
-      for (uint32_t q = 1; q < g.np; q++)
-        xyzz29_accumulate29(acc, empty, load_xyzz29(partials + g.off + q));
+    for (uint32_t q = 1; q < g.np; q++)
+      xyzz29_accumulate29(acc, empty, load_xyzz29(partials + g.off + q));
   }
   if (add)
     xyzz29_accumulate(acc, empty, load_xyzz(g.dst));
@@ -938,6 +956,7 @@ hipError_t layout_batch(const msm_job *jobs, unsigned count, batch_layout *out) 
     d.W = jobs[j].stride ? 1 : d.Wd;
     d.stride = jobs[j].stride;
     d.piece = (uint16_t)jobs[j].piece;
+    d.small = small_pieces(d);
     if (entries + (uint64_t)d.Wd * n >= (1ull << 31))
       return hipErrorInvalidValue;
     d.entry_begin = (uint32_t)entries;
@@ -979,10 +998,9 @@ hipError_t accumulate_phase(batch_layout &bl, unsigned count, arena &ar, g1_xyzz
   // 1-2. digits, sort, bucket runs
   uint32_t *offsets = nullptr, *counts = nullptr;
   uint64_t *sorted = nullptr; // (key, point reference) pairs, sorted by key within each window
-  // offsets, counts and meta = {heavy count, heavy chunk total} are cleared together
-  BC_TRY(ar.get(&offsets, 2 * (uint64_t)nb + 2));
+  // offsets, counts and the lists' lengths are cleared together
+  BC_TRY(ar.get(&offsets, 2 * (uint64_t)nb + 3));
   counts = offsets + nb;
-  uint32_t *const meta = counts + nb;
   BC_TRY(ar.get(&sorted, entries));
   {
     uint64_t *digits = nullptr;
@@ -1031,31 +1049,33 @@ hipError_t accumulate_phase(batch_layout &bl, unsigned count, arena &ar, g1_xyzz
 
   // 3. accumulation over chunks of the sorted entries, which also records each
   // bucket's run [offsets[b], counts[b]) (empty buckets keep [0, 0))
-  uint32_t *piece_count = nullptr, *piece_offset = nullptr, *heavy = nullptr;
+  uint32_t *piece_count = nullptr, *piece_offset = nullptr;
+  piece_lists lists{counts + nb, nullptr, nullptr, nullptr};
   xyzz29 *partials = nullptr; // on 29-bit limbs, 144 B each
   BC_TRY(ar.get(&piece_count, nb));
   BC_TRY(ar.get(&piece_offset, nb));
   BC_TRY(ar.get(&partials, slots));
-  BC_TRY(ar.get(&heavy, nb));
-  BC_TRY(fill_u32(offsets, 2 * (uint64_t)nb + 2, 0, s));
+  // a chunk has more than MEDIUM_PIECES of the sums, a bucket of several HEAVY_CHUNK
+  BC_TRY(ar.get(&lists.medium, nb));
+  BC_TRY(ar.get(&lists.chunks, slots / MEDIUM_PIECES + 1));
+  BC_TRY(ar.get(&lists.several, slots / HEAVY_CHUNK + 1));
+  BC_TRY(fill_u32(offsets, 2 * (uint64_t)nb + 3, 0, s));
   accumulate_kernel<<<grid_for(chunks, ACC_BLOCK), ACC_BLOCK, 0, s>>>(jt, sorted, (uint32_t)chunks, partials, offsets, counts);
   BC_LAUNCH_CHECK();
-  bucket_slots_kernel<<<grid_for(nb, MSM_BLOCK), MSM_BLOCK, 0, s>>>(jt, offsets, counts, piece_offset, piece_count, nb, heavy, meta);
+  bucket_slots_kernel<<<grid_for(nb, MSM_BLOCK), MSM_BLOCK, 0, s>>>(jt, offsets, counts, piece_offset, piece_count, nb, lists);
   BC_LAUNCH_CHECK();
 
-  // 4. buckets of more than SMALL_PIECES sums; smaller ones are summed by the gather
-  if (max_np > SMALL_PIECES) {
-    uint32_t *chunk_offset = nullptr;
-    BC_TRY(ar.get(&chunk_offset, nb));
-    heavy_prefix_kernel<<<1, 256, 0, s>>>(heavy, meta, piece_count, chunk_offset, meta + 1);
+  // 4. buckets of more than a job's `small` sums; smaller ones are summed by the gather
+  if (max_np > 4) {
+    heavy_chunk_kernel<<<512, HEAVY_BLOCK, 0, s>>>(partials, lists, piece_offset, piece_count);
     BC_LAUNCH_CHECK();
-    heavy_chunk_kernel<<<512, HEAVY_BLOCK, 0, s>>>(partials, heavy, meta, chunk_offset, meta + 1, piece_offset, piece_count);
-    BC_LAUNCH_CHECK();
-    heavy_final_kernel<<<256, HEAVY_BLOCK, 0, s>>>(partials, heavy, meta, piece_offset, piece_count);
-    BC_LAUNCH_CHECK();
-    BC_TRY(ar.put(chunk_offset));
+    if (max_np > HEAVY_CHUNK) {
+      heavy_final_kernel<<<256, HEAVY_BLOCK, 0, s>>>(partials, lists, piece_offset, piece_count);
+      BC_LAUNCH_CHECK();
+    }
   }
-  BC_TRY(ar.put(heavy));
+  for (void *p : {(void *)lists.several, (void *)lists.chunks, (void *)lists.medium})
+    BC_TRY(ar.put(p));
 
   // the listing gather when most buckets lie in jobs whose buckets average at
   // most a quarter of a chunk
