@@ -147,7 +147,9 @@ public:
     return hipSuccess;
   }
   hipError_t stream(hipStream_t *t) {
-    BC_TRY(hipStreamCreate(t)); // default priority
+    // default priority; not ordered with the null stream, which a caller may pass
+    // as its stream: work moves between the two by events only
+    BC_TRY(hipStreamCreateWithFlags(t, hipStreamNonBlocking));
     streams_.push_back(*t);
     return hipSuccess;
   }

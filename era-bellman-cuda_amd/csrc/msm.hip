@@ -1295,10 +1295,13 @@ hipError_t msm_batch_device(const msm_job *jobs, unsigned count, arena &ar) {
 
 namespace {
 
-// Host inputs are copied in four chunks from 2^18 points up: chunk k+1 moves
-// over PCIe while chunk k is accumulated (src/msm.cu:160-195 copies growing
-// chunks on side streams for the same purpose).
-unsigned host_chunk_log(unsigned L) { return L >= 18 ? L - 2 : L; }
+// Host inputs are copied in chunks: chunk k+1 moves over PCIe while chunk k is
+// accumulated (src/msm.cu:160-195 copies growing chunks on side streams for the
+// same purpose).  Every chunk pays for the sort and the bucket sums again, so
+// chunks pay once the copy they hide is longer: pinned scalars in one, two and
+// four chunks take 0.91 / 1.05 / 1.60 ms at 2^18, 2.29 / 2.23 / 2.64 at 2^20,
+// 4.17 / 3.70 / 4.02 at 2^21, 7.79 / 6.78 / 6.53 at 2^22.
+unsigned host_chunk_log(unsigned L) { return L >= 22 ? L - 2 : L >= 20 ? L - 1 : L; }
 // Out-of-memory back-off: at most this many halvings of the chunk.
 constexpr unsigned MSM_BACKOFF_HALVINGS = 8;
 
@@ -1360,10 +1363,12 @@ hipError_t msm_execute_chunks(const msm_configuration &cfg, unsigned chunk_log, 
   BC_TRY(res.get(&block, bytes));
   arena ar = arena::bump_mode(block, bytes, s);
 
-  // Copies run on their own stream: chunk k's copy is enqueued right after
-  // chunk k - 1's kernels (so a pageable copy, which holds the host thread,
-  // overlaps them), into slot k % 2 once chunk k - 2 has been consumed.
-  hipStream_t cs = nullptr;
+  // Several chunks' copies run on their own stream: chunk k's copy is enqueued
+  // right after chunk k - 1's kernels (so a pageable copy, which holds the host
+  // thread, overlaps them), into slot k % 2 once chunk k - 2 has been consumed.
+  // A single copy runs on the call's stream.
+  const bool own_stream = copying && K > 1;
+  hipStream_t cs = s;
   std::vector<hipEvent_t> loaded(K), freed(2);
   auto enqueue_copy = [&](unsigned k) -> hipError_t {
     if (k >= 2)
@@ -1373,7 +1378,8 @@ hipError_t msm_execute_chunks(const msm_configuration &cfg, unsigned chunk_log, 
       BC_TRY(hipMemcpyAsync(s_slot[k % 2], static_cast<const fe *>(cfg.scalars) + off, sizeof(fe) * chunk_n, hipMemcpyHostToDevice, cs));
     if (bases_host)
       BC_TRY(hipMemcpyAsync(b_slot[k % 2], static_cast<const g1_affine *>(cfg.bases) + off, sizeof(g1_affine) * chunk_n, hipMemcpyHostToDevice, cs));
-    BC_TRY(hipEventRecord(loaded[k], cs));
+    if (own_stream)
+      BC_TRY(hipEventRecord(loaded[k], cs));
     if (k + 1 == K) {
       // after the last copy, on the copy stream (src/msm.cu:183-191)
       if (cfg.h2d_copy_finished.handle)
@@ -1383,7 +1389,7 @@ hipError_t msm_execute_chunks(const msm_configuration &cfg, unsigned chunk_log, 
     }
     return hipSuccess;
   };
-  if (copying) {
+  if (own_stream) {
     BC_TRY(res.stream(&cs));
     for (auto &e : loaded)
       BC_TRY(res.event(&e));
@@ -1394,18 +1400,19 @@ hipError_t msm_execute_chunks(const msm_configuration &cfg, unsigned chunk_log, 
     BC_TRY(res.event(&ready));
     BC_TRY(hipEventRecord(ready, s));
     BC_TRY(hipStreamWaitEvent(cs, ready, 0));
-    BC_TRY(enqueue_copy(0));
   }
+  if (copying)
+    BC_TRY(enqueue_copy(0));
   auto inputs_of = [&](unsigned k, const g1_affine **b, const fe **sc) -> hipError_t {
     const size_t off = (size_t)k * chunk_n;
-    if (copying)
+    if (own_stream)
       BC_TRY(hipStreamWaitEvent(s, loaded[k], 0));
     *b = bases_host ? b_slot[k % 2] : full.bases + off;
     *sc = scalars_host ? s_slot[k % 2] : full.scalars + off;
     return hipSuccess;
   };
   auto consumed = [&](unsigned k) -> hipError_t {
-    if (!copying || k + 1 >= K)
+    if (!own_stream || k + 1 >= K)
       return hipSuccess;
     BC_TRY(hipEventRecord(freed[k % 2], s));
     return enqueue_copy(k + 1);
