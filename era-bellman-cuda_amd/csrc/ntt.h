@@ -16,6 +16,11 @@ constexpr unsigned NTT_MAX_JOBS = 64;
 // against 2.27 ms in two passes of 2^12-element tiles).
 constexpr unsigned NTT_LOG_TILE = 10;
 
+// Smallest natural-order transform whose first twelve stages run on the matrix
+// cores (two passes of six).  Against the VALU passes alone: 2^24 1.73 -> 1.46 ms,
+// 2^20 120 -> 95 us, 2^18 47 -> 43 us; at 2^17 the third pass costs what they save.
+constexpr unsigned NTT_MFMA_MIN_LOG = 18;
+
 inline unsigned ntt_passes(unsigned log_n) { return (log_n + NTT_LOG_TILE - 1) / NTT_LOG_TILE; }
 
 // A first pass of `first` stages is valid for a size of two or more passes
@@ -46,6 +51,7 @@ inline bool ntt_job_valid(const ntt_job &q) { return ntt_shape_valid(q.log_n, q.
 
 struct ntt_tables {
   const fe *fwd, *inv, *inv_sizes;
+  const int8_t *mfma_fwd, *mfma_inv;
   unsigned log_size;
 };
 

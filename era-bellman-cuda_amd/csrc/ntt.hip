@@ -22,7 +22,10 @@
 // butterflies stay inside groups of 2^(s_hi-s_lo) elements, strided by
 // 2^(L-s_hi), so a transform of 2^L takes ceil(L / 10) HBM passes (three at
 // 2^24).  Tiles are mapped XCD-major so that neighbouring strided columns run
-// on the same XCD and share its L2 lines.
+// on the same XCD and share its L2 lines.  The first twelve stages of a natural-
+// order transform of 2^NTT_MFMA_MIN_LOG or more are two passes of six stages on
+// the matrix cores instead (ntt_mfma.cuh): their few twiddles are shared by 32
+// columns and more.
 #include <algorithm>
 #include <mutex>
 #include <vector>
@@ -31,6 +34,7 @@
 #include "common.h"
 #include "inverse.cuh"
 #include "ntt.h"
+#include "ntt_mfma.cuh"
 #include "powers.cuh"
 #include "tables.h"
 #include "tuning.h"
@@ -46,6 +50,7 @@ struct twiddle_state {
   fe *fwd = nullptr;       // TW[2^s + b] = omega_{2^(s+1)}^brev_s(b), index 0 unused
   fe *inv = nullptr;       // inverse powers, same layout
   fe *inv_sizes = nullptr; // 2^-i, i <= NTT_MAX_LOG
+  int8_t *mfma_fwd = nullptr, *mfma_inv = nullptr; // twiddle matrices (ntt_mfma.cuh)
   unsigned log_size = 0;
   bool attributes = false;
   std::vector<fe *> retired;
@@ -280,6 +285,112 @@ template <bool GS> __global__ __launch_bounds__(NTT_BLOCK) void ntt_pass_kernel(
   }
 }
 
+// A pass of six stages on the matrix cores, natural to bit-reversed order: tiles
+// of 64 rows x 32 columns, a quad of rows a thread and step, three radix-4 steps.
+// A wave's quads share their twiddles (its two halves in the last step), whose
+// matrices depend on the pass's block hi alone, so they come from L2.  The first
+// step takes its quads from memory and the last returns them there; in between
+// they change hands through LDS, in two arrays of 16-byte halves (lanes on
+// consecutive columns then meet no bank conflict).
+// Bound by memory at 2^24: 0.29 ms for 1.07 GB (3.7 TB/s, where a copy reaches
+// 5.2), where six stages of VALU butterflies take 0.56-0.60 ms; at 2^20 23 us,
+// one round of blocks, so its loads, steps and stores follow one another.
+__global__ __launch_bounds__(mf::BLOCK, 4) void ntt_mfma_kernel(const pass_table pt, const int8_t *mfma_fwd, const int8_t *mfma_inv, int two16) {
+  using F = FrParams;
+  extern __shared__ fe tile[];
+  u32x4 *lds = reinterpret_cast<u32x4 *>(tile); // [2][mf::TILE]
+  fe *multiples = tile + mf::TILE;
+  unsigned jl = 0, jh = pt.count; // job of this block
+  while (jh - jl > 1) {
+    const unsigned mid = (jl + jh) >> 1;
+    if (pt.job[mid].tile_begin <= blockIdx.x)
+      jl = mid;
+    else
+      jh = mid;
+  }
+  const pass_job &a = pt.job[jl];
+  const unsigned L = a.log_n, s_lo = a.s_lo, log_lo = L - s_lo - mf::STAGES;
+  const unsigned tiles = 1u << (L - mf::STAGES - mf::LOG_COLS);
+  unsigned t = blockIdx.x - a.tile_begin;
+  if (t >= tiles)
+    return; // alignment padding
+  if ((tiles & 7) == 0)
+    t = (t & 7) * (tiles >> 3) + (t >> 3);
+  if (threadIdx.x < 8) { // (4 - e) r
+    const int64_t k = 4 - (int)threadIdx.x;
+    int64_t acc = 0;
+    fe v;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      acc += k * (int64_t)F::m[i];
+      v.v[i] = (uint32_t)acc;
+      acc >>= 32;
+    }
+    multiples[threadIdx.x] = v;
+  }
+  const unsigned hi = t >> (log_lo - mf::LOG_COLS), lo0 = (t << mf::LOG_COLS) & ((1u << log_lo) - 1);
+  const unsigned c = threadIdx.x & (mf::COLS - 1), u = threadIdx.x >> mf::LOG_COLS, lane = threadIdx.x & 63;
+  const size_t base = ((size_t)hi << (L - s_lo)) + lo0 + c;
+  const unsigned group = s_lo == 0 ? 0 : 1 + hi;
+  const v4i *matrices = reinterpret_cast<const v4i *>((a.inverse ? mfma_inv : mfma_fwd) +
+                                                      (size_t)group * mf::GROUP_BLOCKS * mf::PER_BLOCK * mf::MATRIX_BYTES) + lane;
+  auto block_matrices = [&](unsigned block) { return matrices + block * (mf::PER_BLOCK * mf::MATRIX_BYTES / sizeof(v4i)); };
+  auto put = [&](unsigned row, const fe &v) {
+    lds[row * mf::COLS + c] = u32x4{v.v[0], v.v[1], v.v[2], v.v[3]};
+    lds[mf::TILE + row * mf::COLS + c] = u32x4{v.v[4], v.v[5], v.v[6], v.v[7]};
+  };
+  auto take = [&](unsigned row) {
+    const u32x4 p = lds[row * mf::COLS + c], q = lds[mf::TILE + row * mf::COLS + c];
+    fe v;
+    v.v[0] = p.x, v.v[1] = p.y, v.v[2] = p.z, v.v[3] = p.w;
+    v.v[4] = q.x, v.v[5] = q.y, v.v[6] = q.z, v.v[7] = q.w;
+    return v;
+  };
+  fe x[4];
+#pragma unroll
+  for (unsigned i = 0; i < 4; i++)
+    x[i] = load_fe(a.in + base + ((size_t)(u + 16 * i) << log_lo));
+  if (a.pre_table) {
+#pragma unroll
+    for (unsigned i = 0; i < 4; i++)
+      x[i] = mul_lazy<F>(x[i], twist_pow(a.aux, (unsigned)(base + ((size_t)(u + 16 * i) << log_lo))));
+  }
+  // inputs below 2r (the transform's), or below 4r as this kernel leaves them: 2r off
+  if (s_lo == 0) {
+#pragma unroll
+    for (unsigned i = 0; i < 4; i++)
+      x[i] = mf::add_offset(x[i], mf::offset(0, 1));
+  } else {
+#pragma unroll
+    for (unsigned i = 0; i < 4; i++)
+      x[i] = mf::add_offset(x[i], mf::offset(-2, 1));
+  }
+  __syncthreads(); // `multiples`
+  mf::radix4(x, block_matrices(0), block_matrices(0), multiples, two16);
+#pragma unroll
+  for (unsigned i = 0; i < 4; i++)
+    put(u + 16 * i, x[i]);
+  __syncthreads();
+  const unsigned row2 = (u >> 2) * 16 + (u & 3);
+#pragma unroll
+  for (unsigned i = 0; i < 4; i++)
+    x[i] = take(row2 + 4 * i);
+  const unsigned block2 = __builtin_amdgcn_readfirstlane(1 + (u >> 2));
+  mf::radix4(x, block_matrices(block2), block_matrices(block2), multiples, two16);
+#pragma unroll
+  for (unsigned i = 0; i < 4; i++)
+    put(row2 + 4 * i, x[i]); // the rows this thread took
+  __syncthreads();
+#pragma unroll
+  for (unsigned i = 0; i < 4; i++)
+    x[i] = take(4 * u + i);
+  const unsigned block3 = __builtin_amdgcn_readfirstlane(5 + (u & ~1u));
+  mf::radix4(x, block_matrices(block3), block_matrices(block3 + 1), multiples, two16);
+#pragma unroll
+  for (unsigned i = 0; i < 4; i++)
+    store_fe(a.out + base + ((size_t)(4 * u + i) << log_lo), mf::add_offset(x[i], mf::offset(2, -1)));
+}
+
 // fine[j] = alpha^j (j < 2^12), coarse[j] = scale * alpha^(j << 12), so that
 // twist(i) = fine[i mod 2^12] * coarse[i >> 12] = scale * alpha^i (fine[0] is
 // skipped).  The digit table of alpha comes from the host, so an entry is a chain
@@ -296,24 +407,29 @@ __global__ void twist_table_kernel(fe *fine, fe *coarse, const power_digits alph
 
 struct pass_plan {
   unsigned s_lo, s_hi;
+  bool mfma; // ntt_mfma_kernel
 };
 
 // Stage runs of the HBM passes: ceil(L / NTT_LOG_TILE) passes, balanced;
 // the tuning table may name the first pass's stage count, and the rest are
 // then balanced over the remaining passes.
-std::vector<pass_plan> plan_passes(unsigned L) {
+std::vector<pass_plan> plan_passes(unsigned L, bool bitrev_in) {
   std::vector<pass_plan> p;
   unsigned passes = ntt_passes(L), s = 0;
   const unsigned first = passes >= 2 ? ntt_first_pass(L) : 0;
   if (first && ntt_split_valid(L, first)) {
-    p.push_back({0, first});
+    p.push_back({0, first, false});
     s = first;
     passes--;
+  } else if (!bitrev_in && L >= NTT_MFMA_MIN_LOG) {
+    for (; s < 2 * mf::STAGES; s += mf::STAGES)
+      p.push_back({s, s + mf::STAGES, true});
+    passes = ntt_passes(L - s);
   }
   const unsigned rest = L - s;
   for (unsigned i = 0; i < passes; i++) {
     const unsigned len = rest / passes + (i < rest % passes ? 1 : 0);
-    p.push_back({s, s + len});
+    p.push_back({s, s + len, false});
     s += len;
   }
   return p;
@@ -343,6 +459,7 @@ hipError_t ntt_prepare(unsigned max_log_n, hipStream_t stream, ntt_tables *out) 
     const int bytes = (int)(sizeof(fe) << NTT_LOG_TILE);
     BC_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&ntt_pass_kernel<false>), hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
     BC_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&ntt_pass_kernel<true>), hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
+    BC_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&ntt_mfma_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)mf::LDS_BYTES));
     t.attributes = true;
   }
   if (!t.inv_sizes) {
@@ -374,8 +491,20 @@ hipError_t ntt_prepare(unsigned max_log_n, hipStream_t stream, ntt_tables *out) 
     t.inv = i;
     t.log_size = log_size;
   }
+  if (!t.mfma_fwd && max_log_n >= NTT_MFMA_MIN_LOG) {
+    int8_t *m = nullptr;
+    BC_TRY(hipMalloc(&m, 2 * mf::TABLE_BYTES));
+    const unsigned rows = mf::TABLE_BYTES / 32;
+    mf::matrix_kernel<<<grid_for(rows, 256), 256, 0, stream>>>(t.fwd, m);
+    BC_LAUNCH_CHECK();
+    mf::matrix_kernel<<<grid_for(rows, 256), 256, 0, stream>>>(t.inv, m + mf::TABLE_BYTES);
+    BC_LAUNCH_CHECK();
+    BC_TRY(hipStreamSynchronize(stream));
+    t.mfma_fwd = m;
+    t.mfma_inv = m + mf::TABLE_BYTES;
+  }
   if (out)
-    *out = ntt_tables{t.fwd, t.inv, t.inv_sizes, t.log_size};
+    *out = ntt_tables{t.fwd, t.inv, t.inv_sizes, t.mfma_fwd, t.mfma_inv, t.log_size};
   return hipSuccess;
 }
 
@@ -424,11 +553,14 @@ hipError_t ntt_batch_device(const ntt_job *jobs, unsigned count, arena &ar) {
   std::vector<std::vector<pass_plan>> plans(count);
   unsigned max_passes = 0;
   for (unsigned j = 0; j < count; j++) {
-    plans[j] = plan_passes(jobs[j].log_n);
+    plans[j] = plan_passes(jobs[j].log_n, jobs[j].bitrev_in);
     max_passes = std::max(max_passes, (unsigned)plans[j].size());
   }
   for (unsigned k = 0; k < max_passes; k++) {
-    for (int gs = 0; gs < 2; gs++) {
+    // butterfly order and kernel: Cooley-Tukey, Gentleman-Sande, Cooley-Tukey on the matrix cores
+    for (int form = 0; form < 3; form++) {
+      const int gs = form == 1;
+      const bool mfma = form == 2;
       pass_table pt{};
       pt.tw_fwd = tt.fwd;
       pt.tw_inv = tt.inv;
@@ -440,6 +572,8 @@ hipError_t ntt_batch_device(const ntt_job *jobs, unsigned count, arena &ar) {
         if ((int)q.bitrev_in != gs || k >= np)
           continue;
         const pass_plan pp = q.bitrev_in ? plans[j][np - 1 - k] : plans[j][k];
+        if (pp.mfma != mfma)
+          continue;
         const unsigned L = q.log_n;
         const unsigned log_t = pp.s_hi - pp.s_lo;
         const unsigned log_lo = L - pp.s_hi, log_hi = pp.s_lo;
@@ -470,13 +604,15 @@ hipError_t ntt_batch_device(const ntt_job *jobs, unsigned count, arena &ar) {
           a.post = POST_LAZY;
         }
         a.tile_begin = blocks;
-        const uint32_t tiles = 1u << (L - log_t - log_c - log_g);
+        const uint32_t tiles = mfma ? 1u << (L - mf::STAGES - mf::LOG_COLS) : 1u << (L - log_t - log_c - log_g);
         blocks += (tiles + 7) & ~7u;
         lds = std::max(lds, sizeof(fe) << (log_g + log_t + log_c));
       }
       if (pt.count == 0)
         continue;
-      if (gs)
+      if (mfma)
+        ntt_mfma_kernel<<<blocks, mf::BLOCK, mf::LDS_BYTES, stream>>>(pt, tt.mfma_fwd, tt.mfma_inv, 1 << 16);
+      else if (gs)
         ntt_pass_kernel<true><<<blocks, NTT_BLOCK, lds, stream>>>(pt);
       else
         ntt_pass_kernel<false><<<blocks, NTT_BLOCK, lds, stream>>>(pt);
@@ -504,6 +640,8 @@ hipError_t ntt_tear_down_impl() {
   }
   if (t.inv_sizes)
     BC_TRY(hipFree(t.inv_sizes));
+  if (t.mfma_fwd)
+    BC_TRY(hipFree(t.mfma_fwd));
   t = twiddle_state{};
   return hipSuccess;
 }

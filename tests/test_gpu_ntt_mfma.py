@@ -1,0 +1,48 @@
+"""Transforms around the size where the first twelve stages move to the matrix
+cores (2^18, natural order in), with inputs at the ends of the value range: the
+signed digit sums there are the largest."""
+import numpy as np
+import pytest
+
+from gpu_helpers import ntt, ntt_batch
+
+pytestmark = pytest.mark.gpu
+
+
+def inputs(oracle, kind, log_n):
+    n = 1 << log_n
+    if kind == "random":
+        return oracle.random_fr(0xBC0000B1 + log_n, n)
+    x = np.zeros((n, 8), dtype=np.uint32)
+    top = oracle.to_limbs([oracle.R - 1])[0]  # the largest stored value
+    if kind == "largest":
+        x[:] = top
+    elif kind == "alternating":
+        x[::2] = top
+    else:  # bytes 0x80 and 0x7f, where the signed digits change sign
+        x[:] = 0x80808080
+        x[:, 7] = 0x007F807F
+        x[1::3] = 0x7F7F7F7F
+        x[1::3, 7] = 0x2F7F807F
+    return x
+
+
+@pytest.mark.parametrize("log_n", [17, 18, 19, 21])
+@pytest.mark.parametrize("inverse", [False, True])
+@pytest.mark.parametrize("kind", ["random", "largest", "alternating", "sign bytes"])
+def test_natural_order_transforms(bellman, oracle, log_n, inverse, kind):
+    _, dev = bellman
+    x = inputs(oracle, kind, log_n)
+    assert np.array_equal(ntt(dev, x, log_n, inverse=inverse), oracle.ntt(x, log_n, False, inverse))
+
+
+@pytest.mark.parametrize("inverse", [False, True])
+def test_cosets_in_place_and_in_a_batch(bellman, oracle, inverse):
+    B, dev = bellman
+    logs = [18, 10, 20, 19]
+    xs = [inputs(oracle, "random", l) for l in logs]
+    bufs = [dev.upload(x) for x in xs]
+    ntt_batch(dev, [B.ntt_job(p, p, l, bitrev=i == 3, inverse=inverse, log_ext=2, coset=i) for i, (p, l) in enumerate(zip(bufs, logs))])
+    for i, (p, x, l) in enumerate(zip(bufs, xs, logs)):
+        assert np.array_equal(dev.download(p, (1 << l, 8)), oracle.ntt(x, l, i == 3, inverse, 2, i)), i
+        dev.free(p)
