@@ -121,6 +121,8 @@ template <class F> struct P29 {
   static constexpr c29::limbs one = c29::pow2_mod(n, 261);       // 1 in the 2^261 radix
   static constexpr c29::limbs c2 = c29::borrowed(c29::times(n, 2), 0);
   static constexpr c29::limbs c16 = c29::borrowed(c29::times(n, 16), 0);
+  static constexpr c29::limbs c16e2 = c29::borrowed(c29::times(n, 16), 2);
+  static constexpr c29::limbs c32 = c29::borrowed(c29::times(n, 32), 0);
   static constexpr c29::limbs c48e2 = c29::borrowed(c29::times(n, 48), 2);
   static constexpr c29::limbs c64 = c29::borrowed(c29::times(n, 64), 1);
   // floor(x8 * div_magic / 2^52) <= floor(x8 / (n8 + 1)) for x8 < 2^31

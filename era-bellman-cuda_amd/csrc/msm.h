@@ -9,11 +9,11 @@ namespace bc {
 
 // Sorted (digit, point) entries per accumulating thread of the plain call at
 // the reference window widths, measured on MI355X: short chunks keep small
-// MSMs parallel (up to 2^15 the call is latency-bound and 4 entries per thread
-// was fastest in two sweeps of three sizes), long ones cut the partial sums of
-// large MSMs (2^24: 128 entries 2 % faster than 64, 8 % faster than 16).
+// MSMs parallel (2^12 points: 219 us at 4 entries, 233 at 8, 277 at 16), long
+// ones cut the partial sums of large MSMs (2^14: 258 us at 8 entries, 275 at 4;
+// 2^18: 647 at 16, 666 at 8; 2^24: 128 entries 4 % faster than 16).
 constexpr unsigned msm_plain_piece(unsigned log_n) {
-  return log_n >= 24 ? 128u : log_n == 23 ? 64u : log_n >= 21 ? 32u : log_n >= 19 ? 16u : log_n >= 16 ? 8u : 4u;
+  return log_n >= 24 ? 128u : log_n == 23 ? 64u : log_n >= 21 ? 32u : log_n >= 18 ? 16u : log_n >= 14 ? 8u : 4u;
 }
 // The most entries per accumulating thread a job may ask for.
 constexpr unsigned MSM_MAX_PIECE = 0xffff;

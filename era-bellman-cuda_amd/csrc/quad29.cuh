@@ -13,9 +13,11 @@
 // are the same in the four lanes.
 //
 // Bounds, in multiples of m (a product of a m and b m is below (a b / 164 + 1) m,
-// since m / 2^261 < 1 / 164): X < 2, Y < 4, ZZ < 2, ZZZ < 2, all normalized.
-// Every product below has operands of at most 8 m and 4 m, so it is below
-// 1.2 m, and differences of products take 2 m.
+// since m / 2^261 < 1 / 164): X < 18, Y < 6, ZZ < 2, ZZZ < 2; the values in
+// between are given in the functions.  X, ZZ and ZZZ are normalized, Y is not
+// (lower limbs below 2^31: the wide operand of a product).  Leaving X above 2 m
+// and Y and the second factor of Y3 unnormalized takes 100 of the 930
+// instructions of a doubling; a lone wave takes 5 cycles for one.
 #pragma once
 
 #include "curve29.cuh"
@@ -56,16 +58,17 @@ __device__ __forceinline__ bool quad_is_infinity(const f29 &p) { return quad_fla
 __device__ __forceinline__ f29 quad_dbl(const f29 &p) {
   using P = P29<Fq>;
   const unsigned l = quad_lane();
-  const f29 a = select29(l == QUAD_Y, norm29(add29(p, p)), p); // U = 2 Y, X, ZZZ, ZZ
-  const f29 r1 = sqr29<Fq>(a);                                 // V = U^2, X^2
+  const f29 a = select29(l == QUAD_Y, norm29(add29(p, p)), p); // U = 2 Y < 12, X, ZZZ, ZZ
+  const f29 r1 = sqr29<Fq>(a);                                 // V = U^2 < 1.9, X^2 < 3
   const f29 V = quad_broadcast<QUAD_Y>(r1), XX = quad_broadcast<QUAD_X>(r1);
-  const f29 M = norm29(add29(XX, add29(XX, XX)));
-  const f29 r2 = mul29<Fq>(select29(l == QUAD_ZZZ, M, a), select29(l == QUAD_ZZZ, M, V)); // W = U V, S = X V, M^2, V ZZ
-  const f29 W = quad_broadcast<QUAD_Y>(r2), S = quad_broadcast<QUAD_X>(r2), MM = quad_broadcast<QUAD_ZZZ>(r2);
-  const f29 X3 = reduce_value29<Fq>(norm29(sub29(MM, add29(S, S), P::c48e2)));
-  const f29 SX = norm29(sub29(S, X3, P::c2));
-  const f29 r3 = mul29<Fq>(select29(l == QUAD_X, M, W), select29(l == QUAD_X, SX, p)); // W Y, M (S - X3), W ZZZ
-  const f29 Y3 = norm29(sub29(quad_broadcast<QUAD_X>(r3), r3, P::c2));
+  const f29 M = norm29(add29(XX, add29(XX, XX))); // < 9
+  const f29 r2 = mul29<Fq>(select29(l == QUAD_ZZZ, M, a), select29(l == QUAD_ZZZ, M, V)); // W = U V, S = X V < 1.3, M^2 < 1.5, V ZZ
+  const f29 W = quad_broadcast<QUAD_Y>(r2), MM = quad_broadcast<QUAD_ZZZ>(r2);
+  // lane X
+  const f29 X3 = norm29(sub29(MM, add29(r2, r2), P::c16e2)); // M^2 - 2 S < 17.5
+  const f29 SX = sub29(r2, X3, P::c32);                      // S - X3 < 34, limbs below 2^31
+  const f29 r3 = mul29<Fq>(select29(l == QUAD_X, M, W), select29(l == QUAD_X, SX, p)); // W Y < 1.1, M (S - X3) < 2.9, W ZZZ
+  const f29 Y3 = sub29(quad_broadcast<QUAD_X>(r3), r3, P::c2);                         // < 4.9
   return select29(l == QUAD_Y, Y3, select29(l == QUAD_X, X3, select29(l == QUAD_ZZZ, r3, r2)));
 }
 
@@ -82,11 +85,11 @@ __device__ __forceinline__ f29 quad_add(const f29 &p, const f29 &q) {
   const f29 r2 = mul29<Fq>(select29(low, d, p), select29(low, d, q)); // R^2, PP = Pd^2, ZZZ1 ZZZ2, ZZ1 ZZ2
   const f29 RR = quad_broadcast<0>(r2), PP = quad_broadcast<1>(r2), U1 = quad_broadcast<1>(r1);
   const f29 r3 = mul29<Fq>(select29(l == 0, U1, select29(l == 1, d, r2)), PP); // Q = U1 PP, PPP = Pd PP, -, ZZ3
-  const f29 Q = quad_broadcast<0>(r3), PPP = quad_broadcast<1>(r3), R = quad_broadcast<0>(d);
-  const f29 X3 = reduce_value29<Fq>(norm29(sub29(RR, add29(PPP, add29(Q, Q)), P::c48e2)));
-  const f29 QX = norm29(sub29(Q, X3, P::c2));
+  const f29 Q = quad_broadcast<0>(r3), PPP = quad_broadcast<1>(r3), R = quad_broadcast<0>(d); // < 1.1, 1.1, 3.3
+  const f29 X3 = norm29(sub29(RR, add29(PPP, add29(Q, Q)), P::c16e2));                        // R^2 - PPP - 2 Q < 17.1
+  const f29 QX = sub29(Q, X3, P::c32);                                                        // Q - X3 < 34, limbs below 2^31
   const f29 r4 = mul29<Fq>(select29(l == 0, r1, select29(l == 1, R, r2)), select29(l == 1, QX, PPP)); // S1 PPP, R (Q - X3), ZZZ3
-  const f29 Y3 = norm29(sub29(quad_broadcast<QUAD_X>(r4), r4, P::c2));
+  const f29 Y3 = sub29(quad_broadcast<QUAD_X>(r4), r4, P::c2); // < 4
   f29 s = select29(l == QUAD_Y, Y3, select29(l == QUAD_X, X3, select29(l == QUAD_ZZZ, r4, r3)));
   // infinities by selects, equal and opposite points behind a branch of the
   // whole wave: as lanes' branches the doubling was executed by every addition
@@ -110,7 +113,7 @@ __device__ __forceinline__ f29 quad_from_jacobian(const g1_jacobian *p) {
 // XYZZ points in memory hold x, y, zz, zzz: lane l's coordinate is number l ^ 1.
 // In the library's format (coordinates below 2p; infinity has ZZ = 0 mod p):
 __device__ __forceinline__ f29 quad_load_xyzz(const g1_xyzz *p) { return reduce_value29<Fq>(ext_to29(load_fe(&p->x + (quad_lane() ^ 1)))); }
-__device__ __forceinline__ void quad_store_xyzz(g1_xyzz *p, const f29 &c) { store_fe(&p->x + (quad_lane() ^ 1), to_ext<Fq>(c)); }
+__device__ __forceinline__ void quad_store_xyzz(g1_xyzz *p, const f29 &c) { store_fe(&p->x + (quad_lane() ^ 1), to_ext<Fq>(norm29(c))); }
 
 // and as a partial sum on 29-bit limbs (the accumulators' bounds: X < 2m, the
 // other coordinates products, below 2^257.3, taken below 2m here)
@@ -124,9 +127,10 @@ __device__ __forceinline__ f29 quad_load_xyzz29(const xyzz29 *p) {
 }
 __device__ __forceinline__ void quad_store_xyzz29(xyzz29 *p, const f29 &c) {
   uint32_t *w = reinterpret_cast<uint32_t *>(p) + 9 * (quad_lane() ^ 1);
+  const f29 r = reduce_value29<Fq>(norm29(c)); // X < 2 m again
 #pragma unroll
   for (int i = 0; i < 9; i++)
-    w[i] = c.v[i];
+    w[i] = r.v[i];
 }
 
 // the point of the quad `quads` quads away (a power of two): lane l ^ 4 quads
