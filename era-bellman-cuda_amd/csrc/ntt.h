@@ -20,6 +20,10 @@ constexpr unsigned NTT_LOG_TILE = 10;
 // cores (two passes of six).  Against the VALU passes alone: 2^24 1.73 -> 1.46 ms,
 // 2^20 120 -> 95 us, 2^18 47 -> 43 us; at 2^17 the third pass costs what they save.
 constexpr unsigned NTT_MFMA_MIN_LOG = 18;
+// Smallest one with a third such pass (five to ten stages are then left for one
+// VALU pass; below, the one VALU pass takes them all): 2^23 731 -> 688 us, 2^24
+// 1.46 -> 1.38 ms.
+constexpr unsigned NTT_MFMA_ROWS_MIN_LOG = 23;
 
 inline unsigned ntt_passes(unsigned log_n) { return (log_n + NTT_LOG_TILE - 1) / NTT_LOG_TILE; }
 
@@ -52,6 +56,7 @@ inline bool ntt_job_valid(const ntt_job &q) { return ntt_shape_valid(q.log_n, q.
 struct ntt_tables {
   const fe *fwd, *inv, *inv_sizes;
   const int8_t *mfma_fwd, *mfma_inv;
+  const fe *rows_fwd, *rows_inv;
   unsigned log_size;
 };
 

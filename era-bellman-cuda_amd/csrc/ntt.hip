@@ -51,6 +51,7 @@ struct twiddle_state {
   fe *inv = nullptr;       // inverse powers, same layout
   fe *inv_sizes = nullptr; // 2^-i, i <= NTT_MAX_LOG
   int8_t *mfma_fwd = nullptr, *mfma_inv = nullptr; // twiddle matrices (ntt_mfma.cuh)
+  fe *rows_fwd = nullptr, *rows_inv = nullptr;     // [hi][t] = omega_{2^18}^(+-brev_12(hi) t), t < 64
   unsigned log_size = 0;
   bool attributes = false;
   std::vector<fe *> retired;
@@ -76,6 +77,17 @@ __global__ void twiddle_build_kernel(power_table w, fe *fwd, fe *inv, unsigned l
   store_fe(inv + m, table_pow(w, inverse_exponent(e)));
 }
 
+__global__ void row_factor_kernel(power_table w, fe *fwd, fe *inv) {
+  const unsigned i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= mf::ROW_FACTORS)
+    return;
+  const unsigned hi = i / mf::ROWS, t = i % mf::ROWS;
+  const unsigned e = brev_bits(hi, mf::ROWS_STAGE) * t << (POW_LOG_RANGE - mf::ROWS_STAGE - mf::STAGES);
+  store_fe(fwd + i, table_pow(w, e));
+  store_fe(inv + i, table_pow(w, inverse_exponent(e)));
+}
+
+enum : uint8_t { PRE_NONE = 0, PRE_COSET = 1, PRE_ROWS = 2 };
 enum : uint8_t { POST_LAZY = 0, POST_REDUCE = 1, POST_SCALE = 2, POST_TABLE = 3 };
 
 // One transform's share of a pass launch.
@@ -292,6 +304,9 @@ template <bool GS> __global__ __launch_bounds__(NTT_BLOCK) void ntt_pass_kernel(
 // step takes its quads from memory and the last returns them there; in between
 // they change hands through LDS, in two arrays of 16-byte halves (lanes on
 // consecutive columns then meet no bank conflict).
+// The blocks of stages 12..17 are too many for matrices of their own.  Scaling
+// row t of block hi by omega_{2^18}^(brev(hi) t) first makes every block's
+// network that of block 0 (PRE_ROWS; a row's 32 columns share the factor).
 // Bound by memory at 2^24: 0.29 ms for 1.07 GB (3.7 TB/s, where a copy reaches
 // 5.2), where six stages of VALU butterflies take 0.56-0.60 ms; at 2^20 23 us,
 // one round of blocks, so its loads, steps and stores follow one another.
@@ -331,7 +346,7 @@ __global__ __launch_bounds__(mf::BLOCK, 4) void ntt_mfma_kernel(const pass_table
   const unsigned hi = t >> (log_lo - mf::LOG_COLS), lo0 = (t << mf::LOG_COLS) & ((1u << log_lo) - 1);
   const unsigned c = threadIdx.x & (mf::COLS - 1), u = threadIdx.x >> mf::LOG_COLS, lane = threadIdx.x & 63;
   const size_t base = ((size_t)hi << (L - s_lo)) + lo0 + c;
-  const unsigned group = s_lo == 0 ? 0 : 1 + hi;
+  const unsigned group = s_lo == mf::STAGES ? 1 + hi : 0;
   const v4i *matrices = reinterpret_cast<const v4i *>((a.inverse ? mfma_inv : mfma_fwd) +
                                                       (size_t)group * mf::GROUP_BLOCKS * mf::PER_BLOCK * mf::MATRIX_BYTES) + lane;
   auto block_matrices = [&](unsigned block) { return matrices + block * (mf::PER_BLOCK * mf::MATRIX_BYTES / sizeof(v4i)); };
@@ -350,13 +365,21 @@ __global__ __launch_bounds__(mf::BLOCK, 4) void ntt_mfma_kernel(const pass_table
 #pragma unroll
   for (unsigned i = 0; i < 4; i++)
     x[i] = load_fe(a.in + base + ((size_t)(u + 16 * i) << log_lo));
-  if (a.pre_table) {
+  if (a.pre_table == PRE_COSET) {
 #pragma unroll
     for (unsigned i = 0; i < 4; i++)
       x[i] = mul_lazy<F>(x[i], twist_pow(a.aux, (unsigned)(base + ((size_t)(u + 16 * i) << log_lo))));
+  } else if (a.pre_table == PRE_ROWS) {
+    fe w[4];
+#pragma unroll
+    for (unsigned i = 0; i < 4; i++)
+      w[i] = load_fe(a.aux + hi * mf::ROWS + u + 16 * i);
+#pragma unroll
+    for (unsigned i = 0; i < 4; i++)
+      x[i] = mul_lazy<F>(x[i], w[i]);
   }
-  // inputs below 2r (the transform's), or below 4r as this kernel leaves them: 2r off
-  if (s_lo == 0) {
+  // inputs below 2r (the transform's, products), or below 4r as this kernel leaves them: 2r off
+  if (s_lo == 0 || a.pre_table) {
 #pragma unroll
     for (unsigned i = 0; i < 4; i++)
       x[i] = mf::add_offset(x[i], mf::offset(0, 1));
@@ -422,7 +445,9 @@ std::vector<pass_plan> plan_passes(unsigned L, bool bitrev_in) {
     s = first;
     passes--;
   } else if (!bitrev_in && L >= NTT_MFMA_MIN_LOG) {
-    for (; s < 2 * mf::STAGES; s += mf::STAGES)
+    // a third pass where a pass of VALU butterflies would follow it anyway
+    const unsigned mfma_stages = L >= NTT_MFMA_ROWS_MIN_LOG ? mf::ROWS_STAGE + mf::STAGES : mf::ROWS_STAGE;
+    for (; s < mfma_stages; s += mf::STAGES)
       p.push_back({s, s + mf::STAGES, true});
     passes = ntt_passes(L - s);
   }
@@ -503,8 +528,20 @@ hipError_t ntt_prepare(unsigned max_log_n, hipStream_t stream, ntt_tables *out) 
     t.mfma_fwd = m;
     t.mfma_inv = m + mf::TABLE_BYTES;
   }
+  if (!t.rows_fwd && max_log_n >= NTT_MFMA_ROWS_MIN_LOG) {
+    const ff_state *ff = ff_current();
+    if (!ff)
+      return hipErrorNotInitialized;
+    fe *f = nullptr;
+    BC_TRY(hipMalloc(&f, 2 * sizeof(fe) * mf::ROW_FACTORS));
+    row_factor_kernel<<<grid_for(mf::ROW_FACTORS, 256), 256, 0, stream>>>(ff->w, f, f + mf::ROW_FACTORS);
+    BC_LAUNCH_CHECK();
+    BC_TRY(hipStreamSynchronize(stream));
+    t.rows_fwd = f;
+    t.rows_inv = f + mf::ROW_FACTORS;
+  }
   if (out)
-    *out = ntt_tables{t.fwd, t.inv, t.inv_sizes, t.mfma_fwd, t.mfma_inv, t.log_size};
+    *out = ntt_tables{t.fwd, t.inv, t.inv_sizes, t.mfma_fwd, t.mfma_inv, t.rows_fwd, t.rows_inv, t.log_size};
   return hipSuccess;
 }
 
@@ -589,8 +626,12 @@ hipError_t ntt_batch_device(const ntt_job *jobs, unsigned count, arena &ar) {
         a.log_c = (uint8_t)log_c;
         a.log_g = (uint8_t)log_g;
         a.inverse = q.inverse ? 1 : 0;
-        a.pre_table = (k == 0 && q.log_ext && !q.inverse) ? 1 : 0;
+        a.pre_table = (k == 0 && q.log_ext && !q.inverse) ? PRE_COSET : PRE_NONE;
         a.aux = twist[j];
+        if (mfma && pp.s_lo == mf::ROWS_STAGE) {
+          a.pre_table = PRE_ROWS;
+          a.aux = q.inverse ? tt.rows_inv : tt.rows_fwd;
+        }
         if (k == np - 1) {
           if (!q.inverse)
             a.post = POST_REDUCE;
@@ -642,6 +683,8 @@ hipError_t ntt_tear_down_impl() {
     BC_TRY(hipFree(t.inv_sizes));
   if (t.mfma_fwd)
     BC_TRY(hipFree(t.mfma_fwd));
+  if (t.rows_fwd)
+    BC_TRY(hipFree(t.rows_fwd));
   t = twiddle_state{};
   return hipSuccess;
 }

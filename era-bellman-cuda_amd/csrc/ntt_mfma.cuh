@@ -49,6 +49,9 @@ constexpr unsigned PER_BLOCK = 5, GROUP_BLOCKS = 21, MATRIX_BYTES = 1024;
 constexpr unsigned GROUPS = 1 + ROWS; // position 0: one group; position 6: 64
 constexpr size_t TABLE_BYTES = (size_t)GROUPS * GROUP_BLOCKS * PER_BLOCK * MATRIX_BYTES; // 6.8 MB a direction
 
+// Row factors of the pass over stages ROWS_STAGE..: 64 rows of 2^12 blocks (8 MB)
+constexpr unsigned ROWS_STAGE = 12, ROW_FACTORS = ROWS << ROWS_STAGE;
+
 constexpr uint32_t BIAS[8] = {0x80808080, 0x80808080, 0x80808080, 0x80808080, 0x80808080, 0x80808080, 0x80808080, 0x00808080};
 
 // r as signed 32-bit limbs

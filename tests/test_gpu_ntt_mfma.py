@@ -46,3 +46,11 @@ def test_cosets_in_place_and_in_a_batch(bellman, oracle, inverse):
     for i, (p, x, l) in enumerate(zip(bufs, xs, logs)):
         assert np.array_equal(dev.download(p, (1 << l, 8)), oracle.ntt(x, l, i == 3, inverse, 2, i)), i
         dev.free(p)
+
+
+@pytest.mark.parametrize("inverse", [False, True])
+def test_third_pass(bellman, oracle, inverse):
+    _, dev = bellman
+    x = inputs(oracle, "random", 23)
+    x[5::7] = oracle.to_limbs([oracle.R - 1])[0]
+    assert np.array_equal(ntt(dev, x, 23, inverse=inverse), oracle.ntt(x, 23, False, inverse))
