@@ -25,6 +25,10 @@ constexpr unsigned NTT_MFMA_MIN_LOG = 18;
 // 1.46 -> 1.38 ms.
 constexpr unsigned NTT_MFMA_ROWS_MIN_LOG = 23;
 
+// Launches of at most this many elements run one butterfly per thread and stage
+// (a wave per SIMD); at 2^18 that takes 46 us, the larger passes 43 to 47 us.
+constexpr uint64_t NTT_SMALL_ELEMENTS = 1u << 17;
+
 inline unsigned ntt_passes(unsigned log_n) { return (log_n + NTT_LOG_TILE - 1) / NTT_LOG_TILE; }
 
 // A first pass of `first` stages is valid for a size of two or more passes

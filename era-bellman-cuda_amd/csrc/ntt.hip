@@ -44,6 +44,7 @@ namespace bc {
 namespace {
 
 constexpr unsigned NTT_BLOCK = (1u << NTT_LOG_TILE) / 4; // one radix-4 group per thread and step
+constexpr unsigned NTT_SMALL_LOG_TILE = 9, NTT_SMALL_BLOCK = (1u << NTT_SMALL_LOG_TILE) / 2; // one butterfly per thread and stage
 constexpr unsigned TWIST_FINE_BITS = 12;
 
 struct twiddle_state {
@@ -297,6 +298,98 @@ template <bool GS> __global__ __launch_bounds__(NTT_BLOCK) void ntt_pass_kernel(
   }
 }
 
+// A pass of a launch too small to fill the GPU.  Its time is the chain of one
+// thread's products, barriers and loads, so a thread forms one radix-2 butterfly
+// a stage (tiles of at most 512 elements for 256 threads, one wave per SIMD)
+// where a radix-4 step of the kernel above has four products in a row, and the
+// next stage's twiddle is loaded during the current one.  2^12 elements 29 ->
+// 21 us, 2^17 41 -> 31 us (34 bit-reversed to natural).
+template <bool GS> __global__ __launch_bounds__(NTT_SMALL_BLOCK) void ntt_small_pass_kernel(const pass_table pt) {
+  using F = FrParams;
+  __shared__ fe tile[2 * NTT_SMALL_BLOCK];
+  unsigned jl = 0, jh = pt.count; // job of this block
+  while (jh - jl > 1) {
+    const unsigned mid = (jl + jh) >> 1;
+    if (pt.job[mid].tile_begin <= blockIdx.x)
+      jl = mid;
+    else
+      jh = mid;
+  }
+  const pass_job &a = pt.job[jl];
+  const unsigned L = a.log_n, s_lo = a.s_lo, s_hi = a.s_hi, log_c = a.log_c, log_g = a.log_g;
+  const unsigned log_t = s_hi - s_lo, log_lo = L - s_hi;
+  const unsigned t = blockIdx.x - a.tile_begin;
+  if (t >= 1u << (L - log_t - log_c - log_g))
+    return; // alignment padding
+  const fe *__restrict__ tw = a.inverse ? pt.tw_inv : pt.tw_fwd;
+  const unsigned lo0 = (t & ((1u << (log_lo - log_c)) - 1)) << log_c, hi0 = (t >> (log_lo - log_c)) << log_g;
+  const unsigned elems = 1u << (log_g + log_t + log_c), cmask = (1u << log_c) - 1, tmask = (1u << log_t) - 1;
+  auto index_of = [&](unsigned e) {
+    const unsigned c = e & cmask, row = (e >> log_c) & tmask, g = e >> (log_c + log_t);
+    return ((hi0 + g) << (L - s_lo)) | (row << log_lo) | (lo0 + c);
+  };
+  // the thread's butterfly of stage s: elements i0, i1 and its block b
+  const unsigned q = threadIdx.x, c = q & cmask, r = (q >> log_c) & (tmask >> 1), g = q >> (log_c + log_t - 1);
+  const bool active = q < (elems >> 1);
+  auto twiddle = [&](unsigned s) {
+    const unsigned log_h = s_hi - s - 1, b = ((hi0 + g) << (s - s_lo)) | (r >> log_h);
+    return active ? load_fe(tw + (1u << s) + b) : fe_zero();
+  };
+  fe w = twiddle(GS ? s_hi - 1 : s_lo);
+#pragma unroll
+  for (unsigned k = 0; k < 2; k++) {
+    const unsigned e = threadIdx.x + k * NTT_SMALL_BLOCK;
+    if (e < elems) {
+      const unsigned idx = index_of(e);
+      fe v = load_fe(a.in + idx);
+      if (a.pre_table)
+        v = mul_lazy<F>(v, twist_pow(a.aux, GS ? brev_bits(idx, L) : idx));
+      tile[e] = v;
+    }
+  }
+  __syncthreads();
+  for (unsigned k = 0; k < log_t; k++) {
+    const unsigned s = GS ? s_hi - 1 - k : s_lo + k;
+    const fe next = k + 1 < log_t ? twiddle(GS ? s - 1 : s + 1) : w;
+    if (active) {
+      const unsigned log_h = s_hi - s - 1;
+      const unsigned t0 = ((r >> log_h) << (log_h + 1)) | (r & ((1u << log_h) - 1));
+      const unsigned i0 = (((g << log_t) | t0) << log_c) | c, i1 = i0 + (1u << (log_h + log_c));
+      const fe E = tile[i0], O = tile[i1];
+      if (!GS) {
+        // CT tile values are < 4m; each output is < 4m again
+        const fe wo = s != 0 ? mul_lazy<F>(O, w) : reduce2<F>(O);
+        const fe e = reduce2<F>(E);
+        tile[i0] = add_raw(e, wo);
+        tile[i1] = sub_raw2<F>(e, wo);
+      } else {
+        // GS tile values stay < 2m
+        tile[i0] = add2<F>(E, O);
+        tile[i1] = s != 0 ? mul_lazy<F>(sub_raw2<F>(E, O), w) : sub2<F>(E, O);
+      }
+    }
+    w = next;
+    __syncthreads();
+  }
+  const unsigned post = a.post;
+  const fe scale = post == POST_SCALE ? load_fe(a.aux) : fe_zero();
+#pragma unroll
+  for (unsigned k = 0; k < 2; k++) {
+    const unsigned e = threadIdx.x + k * NTT_SMALL_BLOCK;
+    if (e >= elems)
+      continue;
+    const unsigned idx = index_of(e);
+    fe v = tile[e];
+    if (post == POST_REDUCE)
+      v = reduce4<F>(v);
+    else if (post == POST_SCALE)
+      v = mul<F>(v, scale);
+    else if (post == POST_TABLE)
+      v = mul<F>(v, twist_pow(a.aux, GS ? idx : brev_bits(idx, L)));
+    store_fe(a.out + idx, v);
+  }
+}
+
 // A pass of six stages on the matrix cores, natural to bit-reversed order: tiles
 // of 64 rows x 32 columns, a quad of rows a thread and step, three radix-4 steps.
 // A wave's quads share their twiddles (its two halves in the last step), whose
@@ -432,6 +525,18 @@ struct pass_plan {
   unsigned s_lo, s_hi;
   bool mfma; // ntt_mfma_kernel
 };
+
+// Passes of a launch of ntt_small_pass_kernel: as few as its tiles allow, balanced.
+std::vector<pass_plan> plan_small_passes(unsigned L) {
+  std::vector<pass_plan> p;
+  const unsigned passes = (L + NTT_SMALL_LOG_TILE - 1) / NTT_SMALL_LOG_TILE;
+  for (unsigned i = 0, s = 0; i < passes; i++) {
+    const unsigned len = L / passes + (i < L % passes ? 1 : 0);
+    p.push_back({s, s + len, false});
+    s += len;
+  }
+  return p;
+}
 
 // Stage runs of the HBM passes: ceil(L / NTT_LOG_TILE) passes, balanced;
 // the tuning table may name the first pass's stage count, and the rest are
@@ -587,10 +692,20 @@ hipError_t ntt_batch_device(const ntt_job *jobs, unsigned count, arena &ar) {
     BC_LAUNCH_CHECK();
   }
 
+  // a launch that cannot fill the GPU (a named first pass asks for the large one's passes)
+  uint64_t elements = 0;
+  bool small = max_log <= 2 * NTT_SMALL_LOG_TILE;
+  for (unsigned j = 0; j < count; j++) {
+    elements += 1ull << jobs[j].log_n;
+    small = small && !(ntt_passes(jobs[j].log_n) >= 2 && ntt_first_pass(jobs[j].log_n));
+  }
+  small = small && elements <= NTT_SMALL_ELEMENTS;
+  const unsigned log_tile = small ? NTT_SMALL_LOG_TILE : NTT_LOG_TILE;
+
   std::vector<std::vector<pass_plan>> plans(count);
   unsigned max_passes = 0;
   for (unsigned j = 0; j < count; j++) {
-    plans[j] = plan_passes(jobs[j].log_n, jobs[j].bitrev_in);
+    plans[j] = small ? plan_small_passes(jobs[j].log_n) : plan_passes(jobs[j].log_n, jobs[j].bitrev_in);
     max_passes = std::max(max_passes, (unsigned)plans[j].size());
   }
   for (unsigned k = 0; k < max_passes; k++) {
@@ -614,7 +729,7 @@ hipError_t ntt_batch_device(const ntt_job *jobs, unsigned count, arena &ar) {
         const unsigned L = q.log_n;
         const unsigned log_t = pp.s_hi - pp.s_lo;
         const unsigned log_lo = L - pp.s_hi, log_hi = pp.s_lo;
-        const unsigned room = NTT_LOG_TILE - log_t;
+        const unsigned room = log_tile - log_t;
         const unsigned log_c = std::min(log_lo, room);
         const unsigned log_g = log_c == log_lo ? std::min(room - log_c, log_hi) : 0;
         pass_job &a = pt.job[pt.count++];
@@ -653,6 +768,10 @@ hipError_t ntt_batch_device(const ntt_job *jobs, unsigned count, arena &ar) {
         continue;
       if (mfma)
         ntt_mfma_kernel<<<blocks, mf::BLOCK, mf::LDS_BYTES, stream>>>(pt, tt.mfma_fwd, tt.mfma_inv, 1 << 16);
+      else if (small && gs)
+        ntt_small_pass_kernel<true><<<blocks, NTT_SMALL_BLOCK, 0, stream>>>(pt);
+      else if (small)
+        ntt_small_pass_kernel<false><<<blocks, NTT_SMALL_BLOCK, 0, stream>>>(pt);
       else if (gs)
         ntt_pass_kernel<true><<<blocks, NTT_BLOCK, lds, stream>>>(pt);
       else
@@ -717,9 +836,12 @@ hipError_t ntt_execute(const ntt_configuration &c) {
   if (out_host && !in_host && !c.can_overwrite_inputs)
     BC_TRY(res.get(&d_out, (size_t)1 << L));
   const ntt_job probe{d_in, d_out, L, c.bit_reversed_inputs, c.inverse, c.log_extension_degree, c.coset_index};
-  const size_t block_bytes = ntt_footprint(probe);
+  // only a coset transform has temporaries (releasing an unused block costs the
+  // host 8 us, a third of a small transform)
+  const size_t block_bytes = c.log_extension_degree ? ntt_footprint(probe) : 0;
   char *block = nullptr;
-  BC_TRY(res.get(&block, block_bytes));
+  if (block_bytes)
+    BC_TRY(res.get(&block, block_bytes));
   if (in_host) {
     BC_TRY(hipMemcpyAsync(staged_in, c.inputs, bytes, hipMemcpyHostToDevice, s));
     if (c.h2d_copy_finished.handle)
