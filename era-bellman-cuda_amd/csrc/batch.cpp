@@ -452,14 +452,11 @@ hipError_t capture(const plan_state &p, hipStream_t s, hipStream_t s2, hipGraph_
 }
 
 hipError_t plan_create(plan_state *p) {
-  unsigned max_log = 0;
-  for (const ntt_job &j : p->ntt)
-    max_log = std::max(max_log, j.log_n);
   hipStream_t s = nullptr, s2 = nullptr;
   BC_TRY(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
   hipError_t e = hipStreamCreateWithFlags(&s2, hipStreamNonBlocking);
-  if (e == hipSuccess && max_log)
-    e = ntt_prepare(max_log, s, nullptr);
+  if (e == hipSuccess)
+    e = ntt_prepare_jobs(p->ntt.data(), (unsigned)p->ntt.size(), s);
   // The sizing captures see placeholder addresses; their graphs are destroyed
   // without being launched.
   size_t ntt_bytes = 0;

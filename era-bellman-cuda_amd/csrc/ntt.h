@@ -29,6 +29,14 @@ constexpr unsigned NTT_MFMA_ROWS_MIN_LOG = 23;
 // (a wave per SIMD); at 2^18 that takes 46 us, the larger passes 43 to 47 us.
 constexpr uint64_t NTT_SMALL_ELEMENTS = 1u << 17;
 
+// Transforms whose last pass (6..10 stages, one launch) starts on the matrix
+// cores.  Its row factors are a table of 2^log_n elements per direction, so it is
+// kept to tables of 512 MB.
+constexpr unsigned NTT_MFMA_LAST_MAX_LOG = 24;
+inline bool ntt_mfma_last(unsigned log_n) {
+  return log_n >= NTT_MFMA_MIN_LOG && log_n <= NTT_MFMA_LAST_MAX_LOG && log_n != NTT_MFMA_ROWS_MIN_LOG;
+}
+
 inline unsigned ntt_passes(unsigned log_n) { return (log_n + NTT_LOG_TILE - 1) / NTT_LOG_TILE; }
 
 // A first pass of `first` stages is valid for a size of two or more passes
@@ -68,6 +76,9 @@ struct ntt_tables {
 // current device.  May allocate and synchronise `stream` (not capturable);
 // afterwards every batch of transforms up to that size is capturable.
 hipError_t ntt_prepare(unsigned max_log_n, hipStream_t stream, ntt_tables *out);
+
+// The same for these jobs, with the tables that are made per size and direction.
+hipError_t ntt_prepare_jobs(const ntt_job *jobs, unsigned count, hipStream_t stream);
 
 // Up to NTT_MAX_JOBS transforms, one launch per pass index and butterfly
 // order; temporaries (coset twist tables) come from `ar`.

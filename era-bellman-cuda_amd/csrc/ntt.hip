@@ -53,6 +53,7 @@ struct twiddle_state {
   fe *inv_sizes = nullptr; // 2^-i, i <= NTT_MAX_LOG
   int8_t *mfma_fwd = nullptr, *mfma_inv = nullptr; // twiddle matrices (ntt_mfma.cuh)
   fe *rows_fwd = nullptr, *rows_inv = nullptr;     // [hi][t] = omega_{2^18}^(+-brev_12(hi) t), t < 64
+  fe *last_rows[2][NTT_MFMA_LAST_MAX_LOG + 1] = {}; // of the last pass, by direction and size (ntt_last_rows)
   unsigned log_size = 0;
   bool attributes = false;
   std::vector<fe *> retired;
@@ -78,14 +79,14 @@ __global__ void twiddle_build_kernel(power_table w, fe *fwd, fe *inv, unsigned l
   store_fe(inv + m, table_pow(w, inverse_exponent(e)));
 }
 
-__global__ void row_factor_kernel(power_table w, fe *fwd, fe *inv) {
+// rows[hi][t] = omega_{2^(s_lo + log_rows)}^(+-brev(hi) t), hi < 2^s_lo, t < 2^log_rows
+__global__ void row_factor_kernel(power_table w, fe *rows, unsigned s_lo, unsigned log_rows, bool inverse) {
   const unsigned i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= mf::ROW_FACTORS)
+  if (i >= 1u << (s_lo + log_rows))
     return;
-  const unsigned hi = i / mf::ROWS, t = i % mf::ROWS;
-  const unsigned e = brev_bits(hi, mf::ROWS_STAGE) * t << (POW_LOG_RANGE - mf::ROWS_STAGE - mf::STAGES);
-  store_fe(fwd + i, table_pow(w, e));
-  store_fe(inv + i, table_pow(w, inverse_exponent(e)));
+  const unsigned hi = i >> log_rows, t = i & ((1u << log_rows) - 1);
+  const unsigned e = brev_bits(hi, s_lo) * t << (POW_LOG_RANGE - s_lo - log_rows);
+  store_fe(rows + i, table_pow(w, inverse ? inverse_exponent(e) : e));
 }
 
 enum : uint8_t { PRE_NONE = 0, PRE_COSET = 1, PRE_ROWS = 2 };
@@ -95,7 +96,8 @@ enum : uint8_t { POST_LAZY = 0, POST_REDUCE = 1, POST_SCALE = 2, POST_TABLE = 3 
 struct pass_job {
   const fe *in;
   fe *out;
-  const fe *aux; // POST_SCALE: n^-1; twists: fine table, coarse table 2^12 entries later
+  const fe *aux;  // POST_SCALE: n^-1; twists: fine table, coarse table 2^12 entries later
+  const fe *rows; // PRE_ROWS: [hi][row] factors
   uint32_t tile_begin; // first block of the job (a multiple of 8)
   uint8_t log_n, s_lo, s_hi;
   uint8_t log_c, log_g; // tile = 2^log_g groups x 2^(s_hi-s_lo) rows x 2^log_c columns
@@ -424,18 +426,7 @@ __global__ __launch_bounds__(mf::BLOCK, 4) void ntt_mfma_kernel(const pass_table
     return; // alignment padding
   if ((tiles & 7) == 0)
     t = (t & 7) * (tiles >> 3) + (t >> 3);
-  if (threadIdx.x < 8) { // (4 - e) r
-    const int64_t k = 4 - (int)threadIdx.x;
-    int64_t acc = 0;
-    fe v;
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-      acc += k * (int64_t)F::m[i];
-      v.v[i] = (uint32_t)acc;
-      acc >>= 32;
-    }
-    multiples[threadIdx.x] = v;
-  }
+  mf::make_multiples(multiples);
   const unsigned hi = t >> (log_lo - mf::LOG_COLS), lo0 = (t << mf::LOG_COLS) & ((1u << log_lo) - 1);
   const unsigned c = threadIdx.x & (mf::COLS - 1), u = threadIdx.x >> mf::LOG_COLS, lane = threadIdx.x & 63;
   const size_t base = ((size_t)hi << (L - s_lo)) + lo0 + c;
@@ -466,7 +457,7 @@ __global__ __launch_bounds__(mf::BLOCK, 4) void ntt_mfma_kernel(const pass_table
     fe w[4];
 #pragma unroll
     for (unsigned i = 0; i < 4; i++)
-      w[i] = load_fe(a.aux + hi * mf::ROWS + u + 16 * i);
+      w[i] = load_fe(a.rows + hi * mf::ROWS + u + 16 * i);
 #pragma unroll
     for (unsigned i = 0; i < 4; i++)
       x[i] = mul_lazy<F>(x[i], w[i]);
@@ -507,6 +498,150 @@ __global__ __launch_bounds__(mf::BLOCK, 4) void ntt_mfma_kernel(const pass_table
     store_fe(a.out + base + ((size_t)(4 * u + i) << log_lo), mf::add_offset(x[i], mf::offset(2, -1)));
 }
 
+// The last pass of 6..10 stages, natural to bit-reversed order: tiles of 2048
+// neighbouring elements, whole blocks hi of the pass.  Scaling element t of block
+// hi by omega_n^(brev(hi) t) first (a table as large as the transform, read
+// once) makes every block's network that of block 0, so the first six stages run
+// on the matrix cores as above (rows: the top six bits of t, columns: the lower
+// bits and the blocks); the rest are VALU butterflies with the first few
+// twiddles of the table.  Against the VALU pass: 2^20 94 -> 82 us for the whole
+// transform, 2^22 352 -> 324, 2^24 1.38 -> 1.30 ms; its time is a product an
+// element, half the bytes again for the factors, and at 2^20 one round of blocks.
+__global__ __launch_bounds__(mf::BLOCK, 4) void ntt_mfma_last_kernel(const pass_table pt, const int8_t *mfma_fwd, const int8_t *mfma_inv, int two16) {
+  using F = FrParams;
+  extern __shared__ fe tile[];
+  u32x4 *lds = reinterpret_cast<u32x4 *>(tile); // [2][mf::LAST_HALF]
+  fe *multiples = tile + mf::LAST_HALF;
+  unsigned jl = 0, jh = pt.count; // job of this block
+  while (jh - jl > 1) {
+    const unsigned mid = (jl + jh) >> 1;
+    if (pt.job[mid].tile_begin <= blockIdx.x)
+      jl = mid;
+    else
+      jh = mid;
+  }
+  const pass_job &a = pt.job[jl];
+  const unsigned L = a.log_n, rest = L - a.s_lo - mf::STAGES; // VALU stages
+  const unsigned t = blockIdx.x - a.tile_begin;
+  if (t >= 1u << (L - mf::STAGES - mf::LOG_COLS))
+    return; // alignment padding
+  mf::make_multiples(multiples);
+  const unsigned c = threadIdx.x & (mf::COLS - 1), u = threadIdx.x >> mf::LOG_COLS, lane = threadIdx.x & 63;
+  const size_t base = (size_t)t * mf::TILE;
+  const v4i *matrices = reinterpret_cast<const v4i *>(a.inverse ? mfma_inv : mfma_fwd) + lane;
+  auto block_matrices = [&](unsigned block) { return matrices + block * (mf::PER_BLOCK * mf::MATRIX_BYTES / sizeof(v4i)); };
+  auto put = [&](unsigned slot, const fe &v) {
+    lds[slot] = u32x4{v.v[0], v.v[1], v.v[2], v.v[3]};
+    lds[mf::LAST_HALF + slot] = u32x4{v.v[4], v.v[5], v.v[6], v.v[7]};
+  };
+  auto take = [&](unsigned slot) {
+    const u32x4 p = lds[slot], q = lds[mf::LAST_HALF + slot];
+    fe v;
+    v.v[0] = p.x, v.v[1] = p.y, v.v[2] = p.z, v.v[3] = p.w;
+    v.v[4] = q.x, v.v[5] = q.y, v.v[6] = q.z, v.v[7] = q.w;
+    return v;
+  };
+  // element e of the tile: block e >> (6 + rest), row, low bits
+  auto slot_of = [&](unsigned e) {
+    const unsigned low = e & ((1u << rest) - 1), row = (e >> rest) & (mf::ROWS - 1), g = e >> (mf::STAGES + rest);
+    return row * mf::LAST_ROW + (g << rest | low);
+  };
+  fe x[4];
+  {
+    fe w[4];
+#pragma unroll
+    for (unsigned i = 0; i < 4; i++) {
+      const size_t idx = base + threadIdx.x + i * mf::BLOCK;
+      x[i] = load_fe(a.in + idx);
+      w[i] = load_fe(a.rows + idx);
+    }
+#pragma unroll
+    for (unsigned i = 0; i < 4; i++)
+      put(slot_of(threadIdx.x + i * mf::BLOCK), mf::add_offset(mul_lazy<F>(x[i], w[i]), mf::offset(0, 1)));
+  }
+  __syncthreads();
+#pragma unroll
+  for (unsigned i = 0; i < 4; i++)
+    x[i] = take((u + 16 * i) * mf::LAST_ROW + c);
+  mf::radix4(x, block_matrices(0), block_matrices(0), multiples, two16);
+#pragma unroll
+  for (unsigned i = 0; i < 4; i++)
+    put((u + 16 * i) * mf::LAST_ROW + c, x[i]);
+  __syncthreads();
+  const unsigned row2 = (u >> 2) * 16 + (u & 3);
+#pragma unroll
+  for (unsigned i = 0; i < 4; i++)
+    x[i] = take((row2 + 4 * i) * mf::LAST_ROW + c);
+  const unsigned block2 = __builtin_amdgcn_readfirstlane(1 + (u >> 2));
+  mf::radix4(x, block_matrices(block2), block_matrices(block2), multiples, two16);
+#pragma unroll
+  for (unsigned i = 0; i < 4; i++)
+    put((row2 + 4 * i) * mf::LAST_ROW + c, x[i]);
+  __syncthreads();
+#pragma unroll
+  for (unsigned i = 0; i < 4; i++)
+    x[i] = take((4 * u + i) * mf::LAST_ROW + c);
+  const unsigned block3 = __builtin_amdgcn_readfirstlane(5 + (u & ~1u));
+  mf::radix4(x, block_matrices(block3), block_matrices(block3 + 1), multiples, two16);
+#pragma unroll
+  for (unsigned i = 0; i < 4; i++) // below 4r again
+    put((4 * u + i) * mf::LAST_ROW + c, mf::add_offset(x[i], mf::offset(2, -1)));
+  __syncthreads();
+
+  // stages 6..: a lane per row, the column pairs and quads of its row by wave
+  const fe *__restrict__ tw = a.inverse ? pt.tw_inv : pt.tw_fwd;
+  const unsigned slot0 = lane * mf::LAST_ROW, wave = threadIdx.x >> 6;
+  unsigned k = 0;
+  if (rest & 1) {
+    const unsigned log_h = rest - 1;
+    const unsigned b = lane;
+    const fe w = load_fe(tw + mf::ROWS + b);
+#pragma unroll
+    for (unsigned i = 0; i < 2; i++) {
+      const unsigned v = wave + 8 * i; // of 16 pairs
+      const unsigned i0 = slot0 + (((v >> log_h) << (log_h + 1)) | (v & ((1u << log_h) - 1))), i1 = i0 + (1u << log_h);
+      const fe e = reduce2<F>(take(i0)), wo = mul_lazy<F>(take(i1), w);
+      put(i0, add_raw(e, wo));
+      put(i1, sub_raw2<F>(e, wo));
+    }
+    __syncthreads();
+    k = 1;
+  }
+  for (; k < rest; k += 2) {
+    const unsigned log_hh = rest - 2 - k, hh = 1u << log_hh; // distance at stage 6 + k + 1
+    const unsigned low0 = ((wave >> log_hh) << (log_hh + 2)) | (wave & (hh - 1));
+    const unsigned b = lane << k | ((low0 & ((1u << rest) - 1)) >> (rest - k));
+    const unsigned i0 = slot0 + low0, i1 = i0 + hh, i2 = i1 + hh, i3 = i2 + hh;
+    const fe *tw_s1 = tw + (2u << (mf::STAGES + k)) + 2 * b;
+    const fe wa = load_fe(tw + (1u << (mf::STAGES + k)) + b), wb0 = load_fe(tw_s1), wb1 = load_fe(tw_s1 + 1);
+    // as the radix-4 step of ntt_pass_kernel<false>
+    const fe x0 = reduce2<F>(take(i0)), x1 = reduce2<F>(take(i1)), x2 = mul_lazy<F>(take(i2), wa), x3 = mul_lazy<F>(take(i3), wa);
+    const fe y0 = reduce2<F>(add_raw(x0, x2)), y2 = reduce2<F>(sub_raw2<F>(x0, x2));
+    const fe y1 = mul_lazy<F>(add_raw(x1, x3), wb0);
+    const fe y3 = mul_lazy<F>(sub_raw2<F>(x1, x3), wb1);
+    put(i0, add_raw(y0, y1));
+    put(i1, sub_raw2<F>(y0, y1));
+    put(i2, add_raw(y2, y3));
+    put(i3, sub_raw2<F>(y2, y3));
+    __syncthreads();
+  }
+  const unsigned post = a.post;
+  const fe scale = post == POST_SCALE ? load_fe(a.aux) : fe_zero();
+#pragma unroll
+  for (unsigned i = 0; i < 4; i++) {
+    const unsigned e = threadIdx.x + i * mf::BLOCK;
+    const size_t idx = base + e;
+    fe v = take(slot_of(e));
+    if (post == POST_REDUCE)
+      v = reduce4<F>(v);
+    else if (post == POST_SCALE)
+      v = mul<F>(v, scale);
+    else
+      v = mul<F>(v, twist_pow(a.aux, brev_bits((unsigned)idx, L)));
+    store_fe(a.out + idx, v);
+  }
+}
+
 // fine[j] = alpha^j (j < 2^12), coarse[j] = scale * alpha^(j << 12), so that
 // twist(i) = fine[i mod 2^12] * coarse[i >> 12] = scale * alpha^i (fine[0] is
 // skipped).  The digit table of alpha comes from the host, so an entry is a chain
@@ -523,7 +658,8 @@ __global__ void twist_table_kernel(fe *fine, fe *coarse, const power_digits alph
 
 struct pass_plan {
   unsigned s_lo, s_hi;
-  bool mfma; // ntt_mfma_kernel
+  bool mfma;               // ntt_mfma_kernel, or ntt_mfma_last_kernel with
+  const fe *last = nullptr; // its row factors
 };
 
 // Passes of a launch of ntt_small_pass_kernel: as few as its tiles allow, balanced.
@@ -541,7 +677,7 @@ std::vector<pass_plan> plan_small_passes(unsigned L) {
 // Stage runs of the HBM passes: ceil(L / NTT_LOG_TILE) passes, balanced;
 // the tuning table may name the first pass's stage count, and the rest are
 // then balanced over the remaining passes.
-std::vector<pass_plan> plan_passes(unsigned L, bool bitrev_in) {
+std::vector<pass_plan> plan_passes(unsigned L, bool bitrev_in, const fe *last_rows) {
   std::vector<pass_plan> p;
   unsigned passes = ntt_passes(L), s = 0;
   const unsigned first = passes >= 2 ? ntt_first_pass(L) : 0;
@@ -555,6 +691,10 @@ std::vector<pass_plan> plan_passes(unsigned L, bool bitrev_in) {
     for (; s < mfma_stages; s += mf::STAGES)
       p.push_back({s, s + mf::STAGES, true});
     passes = ntt_passes(L - s);
+    if (last_rows) {
+      p.push_back({s, L, true, last_rows});
+      return p;
+    }
   }
   const unsigned rest = L - s;
   for (unsigned i = 0; i < passes; i++) {
@@ -590,6 +730,7 @@ hipError_t ntt_prepare(unsigned max_log_n, hipStream_t stream, ntt_tables *out) 
     BC_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&ntt_pass_kernel<false>), hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
     BC_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&ntt_pass_kernel<true>), hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
     BC_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&ntt_mfma_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)mf::LDS_BYTES));
+    BC_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&ntt_mfma_last_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)mf::LAST_LDS_BYTES));
     t.attributes = true;
   }
   if (!t.inv_sizes) {
@@ -639,14 +780,65 @@ hipError_t ntt_prepare(unsigned max_log_n, hipStream_t stream, ntt_tables *out) 
       return hipErrorNotInitialized;
     fe *f = nullptr;
     BC_TRY(hipMalloc(&f, 2 * sizeof(fe) * mf::ROW_FACTORS));
-    row_factor_kernel<<<grid_for(mf::ROW_FACTORS, 256), 256, 0, stream>>>(ff->w, f, f + mf::ROW_FACTORS);
-    BC_LAUNCH_CHECK();
+    for (int inv = 0; inv < 2; inv++) {
+      row_factor_kernel<<<grid_for(mf::ROW_FACTORS, 256), 256, 0, stream>>>(ff->w, f + inv * mf::ROW_FACTORS, mf::ROWS_STAGE, mf::STAGES, inv != 0);
+      BC_LAUNCH_CHECK();
+    }
     BC_TRY(hipStreamSynchronize(stream));
     t.rows_fwd = f;
     t.rows_inv = f + mf::ROW_FACTORS;
   }
   if (out)
     *out = ntt_tables{t.fwd, t.inv, t.inv_sizes, t.mfma_fwd, t.mfma_inv, t.rows_fwd, t.rows_inv, t.log_size};
+  return hipSuccess;
+}
+
+// The row factors of a transform's last pass (nullptr: its stages are left to
+// VALU passes).  Made on the first transform of a size and direction, except
+// while `stream` is captured; ntt_prepare_jobs makes them ahead of a capture.
+// Results do not depend on which passes run.
+hipError_t ntt_last_rows(const ntt_job &q, hipStream_t stream, const fe **rows) {
+  *rows = nullptr;
+  const unsigned L = q.log_n;
+  if (q.bitrev_in || !ntt_mfma_last(L) || ntt_first_pass(L))
+    return hipSuccess;
+  std::lock_guard<std::mutex> lock(g_tw_mutex);
+  const int d = device_slot();
+  const ff_state *ff = ff_current();
+  if (d < 0 || !ff)
+    return hipErrorInvalidDevice;
+  fe *&slot = g_tw[d].last_rows[q.inverse][L];
+  if (!slot) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (stream)
+      BC_TRY(hipStreamIsCapturing(stream, &status));
+    if (status != hipStreamCaptureStatusNone)
+      return hipSuccess;
+    fe *f = nullptr;
+    if (hipMalloc(&f, sizeof(fe) << L) != hipSuccess) {
+      (void)hipGetLastError();
+      return hipSuccess; // no memory to spare
+    }
+    const unsigned s_lo = L >= NTT_MFMA_ROWS_MIN_LOG ? mf::ROWS_STAGE + mf::STAGES : mf::ROWS_STAGE;
+    row_factor_kernel<<<grid_for((size_t)1 << L, 256), 256, 0, stream>>>(ff->w, f, s_lo, L - s_lo, q.inverse);
+    BC_LAUNCH_CHECK();
+    BC_TRY(hipStreamSynchronize(stream)); // other streams may use the table as soon as it is published
+    slot = f;
+  }
+  *rows = slot;
+  return hipSuccess;
+}
+
+hipError_t ntt_prepare_jobs(const ntt_job *jobs, unsigned count, hipStream_t stream) {
+  unsigned max_log = 0;
+  for (unsigned j = 0; j < count; j++)
+    max_log = std::max(max_log, jobs[j].log_n);
+  if (max_log == 0)
+    return hipSuccess;
+  BC_TRY(ntt_prepare(max_log, stream, nullptr));
+  const fe *rows = nullptr;
+  for (unsigned j = 0; j < count; j++)
+    BC_TRY(ntt_last_rows(jobs[j], stream, &rows));
   return hipSuccess;
 }
 
@@ -705,14 +897,20 @@ hipError_t ntt_batch_device(const ntt_job *jobs, unsigned count, arena &ar) {
   std::vector<std::vector<pass_plan>> plans(count);
   unsigned max_passes = 0;
   for (unsigned j = 0; j < count; j++) {
-    plans[j] = small ? plan_small_passes(jobs[j].log_n) : plan_passes(jobs[j].log_n, jobs[j].bitrev_in);
+    if (small) {
+      plans[j] = plan_small_passes(jobs[j].log_n);
+    } else {
+      const fe *last_rows = nullptr;
+      BC_TRY(ntt_last_rows(jobs[j], stream, &last_rows));
+      plans[j] = plan_passes(jobs[j].log_n, jobs[j].bitrev_in, last_rows);
+    }
     max_passes = std::max(max_passes, (unsigned)plans[j].size());
   }
   for (unsigned k = 0; k < max_passes; k++) {
-    // butterfly order and kernel: Cooley-Tukey, Gentleman-Sande, Cooley-Tukey on the matrix cores
-    for (int form = 0; form < 3; form++) {
+    // butterfly order and kernel: Cooley-Tukey, Gentleman-Sande, Cooley-Tukey on the matrix cores (and its last pass)
+    for (int form = 0; form < 4; form++) {
       const int gs = form == 1;
-      const bool mfma = form == 2;
+      const bool mfma = form >= 2, last = form == 3;
       pass_table pt{};
       pt.tw_fwd = tt.fwd;
       pt.tw_inv = tt.inv;
@@ -724,7 +922,7 @@ hipError_t ntt_batch_device(const ntt_job *jobs, unsigned count, arena &ar) {
         if ((int)q.bitrev_in != gs || k >= np)
           continue;
         const pass_plan pp = q.bitrev_in ? plans[j][np - 1 - k] : plans[j][k];
-        if (pp.mfma != mfma)
+        if (pp.mfma != mfma || (pp.last != nullptr) != last)
           continue;
         const unsigned L = q.log_n;
         const unsigned log_t = pp.s_hi - pp.s_lo;
@@ -743,9 +941,11 @@ hipError_t ntt_batch_device(const ntt_job *jobs, unsigned count, arena &ar) {
         a.inverse = q.inverse ? 1 : 0;
         a.pre_table = (k == 0 && q.log_ext && !q.inverse) ? PRE_COSET : PRE_NONE;
         a.aux = twist[j];
-        if (mfma && pp.s_lo == mf::ROWS_STAGE) {
+        if (last) {
+          a.rows = pp.last;
+        } else if (mfma && pp.s_lo == mf::ROWS_STAGE) {
           a.pre_table = PRE_ROWS;
-          a.aux = q.inverse ? tt.rows_inv : tt.rows_fwd;
+          a.rows = q.inverse ? tt.rows_inv : tt.rows_fwd;
         }
         if (k == np - 1) {
           if (!q.inverse)
@@ -766,7 +966,9 @@ hipError_t ntt_batch_device(const ntt_job *jobs, unsigned count, arena &ar) {
       }
       if (pt.count == 0)
         continue;
-      if (mfma)
+      if (last)
+        ntt_mfma_last_kernel<<<blocks, mf::BLOCK, mf::LAST_LDS_BYTES, stream>>>(pt, tt.mfma_fwd, tt.mfma_inv, 1 << 16);
+      else if (mfma)
         ntt_mfma_kernel<<<blocks, mf::BLOCK, mf::LDS_BYTES, stream>>>(pt, tt.mfma_fwd, tt.mfma_inv, 1 << 16);
       else if (small && gs)
         ntt_small_pass_kernel<true><<<blocks, NTT_SMALL_BLOCK, 0, stream>>>(pt);
@@ -804,6 +1006,10 @@ hipError_t ntt_tear_down_impl() {
     BC_TRY(hipFree(t.mfma_fwd));
   if (t.rows_fwd)
     BC_TRY(hipFree(t.rows_fwd));
+  for (auto &direction : t.last_rows)
+    for (fe *p : direction)
+      if (p)
+        BC_TRY(hipFree(p));
   t = twiddle_state{};
   return hipSuccess;
 }

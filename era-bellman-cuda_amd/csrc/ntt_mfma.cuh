@@ -42,6 +42,10 @@ namespace mf {
 constexpr unsigned STAGES = 6, ROWS = 1u << STAGES, LOG_COLS = 5, COLS = 1u << LOG_COLS;
 constexpr unsigned TILE = ROWS * COLS, BLOCK = TILE / 4; // a quad of elements a thread
 constexpr unsigned LDS_BYTES = TILE * sizeof(fe) + 8 * sizeof(fe);
+// the last pass's tile has rows of 33 16-byte slots: lanes on consecutive rows
+// then meet no bank conflict either
+constexpr unsigned LAST_ROW = COLS + 1, LAST_HALF = ROWS * LAST_ROW;
+constexpr unsigned LAST_LDS_BYTES = LAST_HALF * sizeof(fe) + 8 * sizeof(fe);
 
 // Matrices of a group of blocks (one pass position): per radix-4 block a, b0,
 // a b0, b1, -a b1; one block at stage 0, four at stage 2, sixteen at stage 4.
@@ -148,6 +152,22 @@ __device__ __forceinline__ fe centre(const fe &x, const fe *multiples) {
   fe r;
   add_limbs(r, x, multiples[q + 4]);
   return r;
+}
+
+// (4 - e) r for e < 8, by the block's first eight threads
+__device__ __forceinline__ void make_multiples(fe *multiples) {
+  if (threadIdx.x < 8) {
+    const int64_t k = 4 - (int)threadIdx.x;
+    int64_t acc = 0;
+    fe v;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      acc += k * (int64_t)FrParams::m[i];
+      v.v[i] = (uint32_t)acc;
+      acc >>= 32;
+    }
+    multiples[threadIdx.x] = v;
+  }
 }
 
 // One radix-4 step of a thread's quad, in place.  `matrix` points at the lane's

@@ -246,11 +246,7 @@ public:
   // Exact workspace bytes of a batch, by a sizing capture.  Twiddle tables are
   // grown first, outside the capture.
   static hipError_t size_of(const work &w, hipStream_t s, size_t *bytes) {
-    unsigned max_log = 0;
-    for (const ntt_job &j : w.ntt)
-      max_log = std::max(max_log, j.log_n);
-    if (max_log)
-      BC_TRY(ntt_prepare(max_log, s, nullptr));
+    BC_TRY(ntt_prepare_jobs(w.ntt.data(), (unsigned)w.ntt.size(), s));
     return measure_scratch(s, [&](arena &ar) { return record(w, ar); }, bytes);
   }
 

@@ -54,3 +54,15 @@ def test_third_pass(bellman, oracle, inverse):
     x = inputs(oracle, "random", 23)
     x[5::7] = oracle.to_limbs([oracle.R - 1])[0]
     assert np.array_equal(ntt(dev, x, 23, inverse=inverse), oracle.ntt(x, 23, False, inverse))
+
+
+@pytest.mark.parametrize("log_n", [18, 19, 20, 21, 22, 24])
+def test_last_pass_sizes(bellman, oracle, log_n):
+    """6..10 stages are left for the last pass; the inverse's scaling and the
+    coset's factors are applied there."""
+    _, dev = bellman
+    x = oracle.random_fr(0xBC0000E1 + log_n, 1 << log_n)
+    x[7::11] = oracle.to_limbs([oracle.R - 1])[0]
+    assert np.array_equal(ntt(dev, x, log_n, log_ext=1, coset=1), oracle.ntt(x, log_n, False, False, 1, 1))
+    if log_n <= 22:
+        assert np.array_equal(ntt(dev, x, log_n, inverse=True, log_ext=2, coset=3), oracle.ntt(x, log_n, False, True, 2, 3))
