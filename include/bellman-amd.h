@@ -25,8 +25,10 @@ bc_error bc_amd_generator_multiples(const void *scalars, void *bases, unsigned c
  * (sum = 2*sum + results[j][i] for i = 253..0) as a canonical affine
  * Montgomery point, (0, 0) for infinity.  `results` is a host array of
  * `count` device pointers (254 Jacobian points each); `points` is device
- * memory.  The 253 dependent doublings of one MSM take under a millisecond;
- * MSMs of one call run side by side. */
+ * memory.  One MSM takes about 0.3 ms; MSMs of one call run side by side.
+ * Takes stream-ordered memory (18 KiB per MSM, at most 1.2 MiB) from the
+ * device's default pool; without any, and in a stream capture, it folds
+ * without memory in about 0.5 ms. */
 bc_error bc_amd_msm_fold(const void *const *results, void *points, unsigned count, bc_stream stream);
 
 /* msm_execute_async without any allocation.  No counterpart in the
