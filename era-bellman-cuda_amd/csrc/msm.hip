@@ -279,6 +279,8 @@ constexpr uint32_t MEDIUM_PIECES = 64;
 constexpr unsigned HEAVY_BLOCK = 256;
 constexpr unsigned HEAVY_QUADS = HEAVY_BLOCK / 4;
 constexpr unsigned HEAVY_CHUNK = HEAVY_QUADS * 8;
+constexpr unsigned LISTED_BLOCKS = 512;
+static_assert(HEAVY_BLOCK == MSM_BLOCK, "one launch for both");
 
 // Work lists of the buckets that the gather does not sum itself: medium buckets,
 // (bucket, chunk) pairs of heavy ones, and heavy buckets of several chunks.
@@ -397,6 +399,12 @@ __global__ __launch_bounds__(ACC_BLOCK) void accumulate_kernel(const job_table j
   }
 }
 
+// The top digit of window w: the last digit window tops out below B = 2^(c-1) (a
+// fixed-base job's single bucket window takes every window's digits, up to B).
+__device__ __forceinline__ uint32_t top_digit(const job_desc &jd, uint32_t w) {
+  return 1u << (w == jd.W - 1 && !jd.stride ? jd.c - (jd.Wd * jd.c - 254) - 1 : jd.c - 1);
+}
+
 // Heavy buckets are reduced in chunks of HEAVY_CHUNK partial sums, one block
 // per chunk: a quad of lanes (quad29.cuh) sums every HEAVY_QUADS-th sum, then a
 // tree in LDS; the chunk's sum overwrites the chunk's first slot.  A second
@@ -425,25 +433,43 @@ __device__ __forceinline__ f29 heavy_block_sum(const xyzz29 *base, uint32_t n, u
   return acc;
 }
 
+// where the sum of bucket b goes: slot d of its window, or the window's top when
+// d is its top digit (the bucket's digit d is at least 1)
+__device__ __forceinline__ g1_xyzz *bucket_destination(const job_desc &jd, uint32_t b, g1_xyzz *A, g1_xyzz *tops) {
+  const uint32_t B = 1u << (jd.c - 1);
+  const uint32_t local = b - jd.bucket_begin, w = local >> (jd.c - 1), d = (local & (B - 1)) + 1;
+  return d == top_digit(jd, w) ? tops + jd.top_begin + w : A + jd.bucket_begin + w * B + d;
+}
+
+// one quad: its sum to the bucket's place, added to what is there with `add`
+__device__ __forceinline__ void quad_store_bucket(g1_xyzz *dst, const f29 &sum, bool add) {
+  quad_store_xyzz(dst, add ? quad_add(quad_load_xyzz(dst), sum) : sum);
+}
+
 // 4a. one block per chunk of a heavy bucket, then one wave per medium bucket: a
 // quad sums every 16th partial sum and the quads' sums meet in a tree over the
-// wave, in the bucket's first slot (grid-stride over both lists)
-__global__ __launch_bounds__(HEAVY_BLOCK) void heavy_chunk_kernel(xyzz29 *partials, const piece_lists lists, const uint32_t *piece_offset,
-                                                                  const uint32_t *piece_count) {
-  __shared__ f29 sh[HEAVY_QUADS][4];
+// wave (grid-stride over both lists by `blocks` blocks).  The chunk of a bucket
+// of several goes to its first slot, every other sum to the bucket's place.
+__device__ __forceinline__ void sum_listed(const job_table &jobs, xyzz29 *partials, const piece_lists &lists, const uint32_t *piece_offset,
+                                           const uint32_t *piece_count, g1_xyzz *A, g1_xyzz *tops, bool add, uint32_t blocks,
+                                           f29 (&sh)[HEAVY_QUADS][4]) {
   const uint32_t chunks = lists.count[1], medium = lists.count[0];
-  for (uint32_t c = blockIdx.x; c < chunks; c += gridDim.x) {
+  for (uint32_t c = blockIdx.x; c < chunks; c += blocks) {
     const uint2 ch = lists.chunks[c];
-    const uint32_t first = ch.y * HEAVY_CHUNK, left = piece_count[ch.x] - first; // sums from the chunk start
+    const uint32_t np = piece_count[ch.x], first = ch.y * HEAVY_CHUNK, left = np - first; // sums from the chunk start
     xyzz29 *base = partials + piece_offset[ch.x] + first;
     const f29 sum = heavy_block_sum(base, left < HEAVY_CHUNK ? left : HEAVY_CHUNK, 1, sh);
-    if (threadIdx.x < 4)
-      quad_store_xyzz29(base, sum);
+    if (threadIdx.x < 4) {
+      if (np > HEAVY_CHUNK)
+        quad_store_xyzz29(base, sum);
+      else
+        quad_store_bucket(bucket_destination(jobs.job[find_job(jobs, ch.x, by_bucket())], ch.x, A, tops), sum, add);
+    }
   }
   const unsigned q = (threadIdx.x & 63) >> 2;
-  for (uint32_t m = blockIdx.x * (HEAVY_BLOCK / 64) + (threadIdx.x >> 6); m < medium; m += gridDim.x * (HEAVY_BLOCK / 64)) {
+  for (uint32_t m = blockIdx.x * (HEAVY_BLOCK / 64) + (threadIdx.x >> 6); m < medium; m += blocks * (HEAVY_BLOCK / 64)) {
     const uint32_t b = lists.medium[m], np = piece_count[b];
-    xyzz29 *base = partials + piece_offset[b];
+    const xyzz29 *base = partials + piece_offset[b];
     f29 acc = f29{};
     if (q < np)
       acc = quad_load_xyzz29(base + q);
@@ -453,21 +479,21 @@ __global__ __launch_bounds__(HEAVY_BLOCK) void heavy_chunk_kernel(xyzz29 *partia
       if (off < np) // the sums off.. of a smaller bucket are infinity
         acc = quad_add(acc, quad_from_neighbour(acc, off));
     if (q == 0)
-      quad_store_xyzz29(base, acc);
+      quad_store_bucket(bucket_destination(jobs.job[find_job(jobs, b, by_bucket())], b, A, tops), acc, add);
   }
 }
 
-// 4b. one block per heavy bucket of several chunks (grid-stride): its chunk sums into the first slot
-__global__ __launch_bounds__(HEAVY_BLOCK) void heavy_final_kernel(xyzz29 *partials, const piece_lists lists, const uint32_t *piece_offset,
-                                                                  const uint32_t *piece_count) {
+// 4b. one block per heavy bucket of several chunks (grid-stride): the sum of its chunks' sums
+__global__ __launch_bounds__(HEAVY_BLOCK) void heavy_final_kernel(const job_table jobs, const xyzz29 *partials, const piece_lists lists,
+                                                                  const uint32_t *piece_offset, const uint32_t *piece_count, g1_xyzz *A,
+                                                                  g1_xyzz *tops, bool add) {
   __shared__ f29 sh[HEAVY_QUADS][4];
   const uint32_t count = lists.count[2];
   for (uint32_t h = blockIdx.x; h < count; h += gridDim.x) {
     const uint32_t b = lists.several[h];
-    xyzz29 *base = partials + piece_offset[b];
-    const f29 sum = heavy_block_sum(base, (piece_count[b] + HEAVY_CHUNK - 1) / HEAVY_CHUNK, HEAVY_CHUNK, sh);
+    const f29 sum = heavy_block_sum(partials + piece_offset[b], (piece_count[b] + HEAVY_CHUNK - 1) / HEAVY_CHUNK, HEAVY_CHUNK, sh);
     if (threadIdx.x < 4)
-      quad_store_xyzz29(base, sum);
+      quad_store_bucket(bucket_destination(jobs.job[find_job(jobs, b, by_bucket())], b, A, tops), sum, add);
   }
 }
 
@@ -480,7 +506,7 @@ __global__ __launch_bounds__(HEAVY_BLOCK) void heavy_final_kernel(xyzz29 *partia
 // it.  With `first`, the window's infinity stores are made here.
 struct gather_item {
   g1_xyzz *dst;
-  uint32_t off, np; // np: the sums to add here, 1 when they were added before
+  uint32_t off, np; // its partial sums
   bool live;        // false: nothing to store for this bucket
 };
 
@@ -490,15 +516,12 @@ __device__ __forceinline__ gather_item gather_prepare(const job_table &jobs, uin
   const job_desc &jd = jobs.job[find_job(jobs, t, by_bucket())];
   const uint32_t B = 1u << (jd.c - 1);
   const uint32_t local = t - jd.bucket_begin, w = local >> (jd.c - 1), k = local & (B - 1);
-  // the last digit window tops out below B (a fixed-base job's single bucket
-  // window takes every window's digits, up to B)
-  const uint32_t top_signed = jd.c - (jd.Wd * jd.c - 254) - 1;
-  const uint32_t top_digit = w == jd.W - 1 && !jd.stride ? (1u << top_signed) : B;
+  const uint32_t top = top_digit(jd, w);
   // slot k of a window holds bucket k; slot 0 also hands the bucket of digit B
   // to the window's top when that is its top digit, and the top digit's own
   // slot in the last window hands it there instead
-  const bool to_top = k == 0 ? top_digit == B : k == top_digit;
-  if ((k == 0 || k == top_digit) && !add && first)
+  const bool to_top = k == 0 ? top == B : k == top;
+  if ((k == 0 || k == top) && !add && first)
     store_xyzz(A + t, xyzz_infinity());
   gather_item g{nullptr, 0, 0, false};
   if (k == 0 && !to_top)
@@ -507,16 +530,12 @@ __device__ __forceinline__ gather_item gather_prepare(const job_table &jobs, uin
   const uint32_t d = k == 0 ? B : k;
   const uint32_t b = jd.bucket_begin + w * B + d - 1;
   g.np = piece_count[b];
-  if (g.np > jd.small)
-    g.np = 1;
   g.off = piece_offset[b];
   g.dst = to_top ? tops + jd.top_begin + w : A + t;
-  g.live = !(add && g.np == 0); // nothing of this launch to add
+  g.live = g.np <= jd.small && !(add && g.np == 0); // larger ones are stored by sum_listed; nothing of this launch to add
   return g;
 }
 
-// buckets of 2..jd.small sums are summed here; the sum of a larger one is
-// already in its first slot
 __device__ __forceinline__ bool gather_sums(const gather_item &g) { return g.live && g.np >= 2; }
 
 __device__ __forceinline__ void gather_finish(const gather_item &g, const xyzz29 *__restrict__ partials, bool add) {
@@ -546,12 +565,22 @@ __device__ __forceinline__ void gather_finish(const gather_item &g, const xyzz29
 // launches sum every bucket in place.
 constexpr unsigned GATHER_LIST_MAX_LANES = 16; // a wave lists when at most this many of its lanes add
 
+// The first `listed_blocks` blocks sum the listed buckets: these take a wave or
+// a block for 50 us of additions in sequence, which as a launch of their own
+// before the gather left the GPU nearly idle.  Both launches and this one: 67 +
+// 168 -> 189 us at 2^20 points, 61 + 242 -> 245 us for 24 MSMs of 2^12..2^17, 51 +
+// 23 -> 58 us at 2^12, 95 + 530 -> 590 us at 2^24.
 template <bool LIST>
-__global__ __launch_bounds__(MSM_BLOCK) void bucket_gather_kernel(const job_table jobs, uint32_t nb, const xyzz29 *__restrict__ partials,
+__global__ __launch_bounds__(MSM_BLOCK) void bucket_gather_kernel(const job_table jobs, uint32_t nb, xyzz29 *partials, const piece_lists lists,
                                                                   const uint32_t *__restrict__ piece_offset,
                                                                   const uint32_t *__restrict__ piece_count, g1_xyzz *__restrict__ A,
-                                                                  g1_xyzz *__restrict__ tops, bool add) {
-  const uint32_t t = blockIdx.x * MSM_BLOCK + threadIdx.x;
+                                                                  g1_xyzz *__restrict__ tops, bool add, uint32_t listed_blocks) {
+  __shared__ f29 sh[HEAVY_QUADS][4];
+  if (blockIdx.x < listed_blocks) {
+    sum_listed(jobs, partials, lists, piece_offset, piece_count, A, tops, add, listed_blocks, sh);
+    return;
+  }
+  const uint32_t t = (blockIdx.x - listed_blocks) * MSM_BLOCK + threadIdx.x;
   if (!LIST) {
     if (t < nb) {
       const gather_item g = gather_prepare(jobs, t, piece_offset, piece_count, A, tops, add, true);
@@ -1065,18 +1094,10 @@ hipError_t accumulate_phase(batch_layout &bl, unsigned count, arena &ar, g1_xyzz
   bucket_slots_kernel<<<grid_for(nb, MSM_BLOCK), MSM_BLOCK, 0, s>>>(jt, offsets, counts, piece_offset, piece_count, nb, lists);
   BC_LAUNCH_CHECK();
 
-  // 4. buckets of more than a job's `small` sums; smaller ones are summed by the gather
-  if (max_np > 4) {
-    heavy_chunk_kernel<<<512, HEAVY_BLOCK, 0, s>>>(partials, lists, piece_offset, piece_count);
-    BC_LAUNCH_CHECK();
-    if (max_np > HEAVY_CHUNK) {
-      heavy_final_kernel<<<256, HEAVY_BLOCK, 0, s>>>(partials, lists, piece_offset, piece_count);
-      BC_LAUNCH_CHECK();
-    }
-  }
-  for (void *p : {(void *)lists.several, (void *)lists.chunks, (void *)lists.medium})
-    BC_TRY(ar.put(p));
-
+  // 4. the buckets' sums into the level-0 windows; where none has more than 4
+  // partial sums, none is listed
+  const uint32_t listed_blocks = max_np > 4 ? LISTED_BLOCKS : 0;
+  const uint32_t gather_blocks = listed_blocks + grid_for(nb, MSM_BLOCK);
   // the listing gather when most buckets lie in jobs whose buckets average at
   // most a quarter of a chunk
   uint64_t small_buckets = 0;
@@ -1088,10 +1109,18 @@ hipError_t accumulate_phase(batch_layout &bl, unsigned count, arena &ar, g1_xyzz
       small_buckets += job_buckets;
   }
   if (2 * small_buckets >= nb)
-    bucket_gather_kernel<true><<<grid_for(nb, MSM_BLOCK), MSM_BLOCK, 0, s>>>(jt, nb, partials, piece_offset, piece_count, A, tops, add);
+    bucket_gather_kernel<true>
+        <<<gather_blocks, MSM_BLOCK, 0, s>>>(jt, nb, partials, lists, piece_offset, piece_count, A, tops, add, listed_blocks);
   else
-    bucket_gather_kernel<false><<<grid_for(nb, MSM_BLOCK), MSM_BLOCK, 0, s>>>(jt, nb, partials, piece_offset, piece_count, A, tops, add);
+    bucket_gather_kernel<false>
+        <<<gather_blocks, MSM_BLOCK, 0, s>>>(jt, nb, partials, lists, piece_offset, piece_count, A, tops, add, listed_blocks);
   BC_LAUNCH_CHECK();
+  if (max_np > HEAVY_CHUNK) {
+    heavy_final_kernel<<<256, HEAVY_BLOCK, 0, s>>>(jt, partials, lists, piece_offset, piece_count, A, tops, add);
+    BC_LAUNCH_CHECK();
+  }
+  for (void *p : {(void *)lists.several, (void *)lists.chunks, (void *)lists.medium})
+    BC_TRY(ar.put(p));
   for (void *p : {(void *)partials, (void *)piece_offset, (void *)piece_count, (void *)sorted, (void *)offsets})
     BC_TRY(ar.put(p));
   return hipSuccess;
