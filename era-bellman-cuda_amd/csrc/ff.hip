@@ -179,6 +179,7 @@ __global__ void omega_shift_kernel(power_table w, const fe *values, fe *result, 
 }
 
 // ---------------------------------------------------------------- permutations
+// fewer than 2^BR_TILE_MIN elements: one thread an element
 __global__ void bit_reverse_kernel(const fe *__restrict__ in, fe *__restrict__ out, unsigned log_n) {
   const unsigned i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= (1u << log_n))
@@ -196,6 +197,31 @@ __global__ void bit_reverse_in_place_kernel(fe *data, unsigned log_n) {
   const fe a = load_fe(data + i), b = load_fe(data + j);
   store_fe(data + i, b);
   store_fe(data + j, a);
+}
+
+// An index is (high, middle, low) with 4 bits in high and low: a block takes the 256
+// elements of one middle, which go to the reversed middle with high and low
+// exchanged and reversed, so it reads and writes runs of 512 bytes where a thread
+// an element writes 32 bytes at a time.  In place, a block exchanges the
+// elements of a middle and its reverse.  2^20 elements 21 -> 14 us, 2^24 921 -> 254 us
+// (in place 685 -> 324; a copy takes 207), up to 2^18 a launch's 7 us either way.
+constexpr unsigned BR_BITS = 4, BR_SIDE = 1u << BR_BITS, BR_TILE_MIN = 2 * BR_BITS;
+template <bool IN_PLACE> __global__ __launch_bounds__(BR_SIDE *BR_SIDE) void bit_reverse_tile_kernel(const fe *in, fe *out, unsigned log_n) {
+  __shared__ fe tile[IN_PLACE ? 2 : 1][BR_SIDE][BR_SIDE + 1]; // a column's elements lie in different banks
+  const unsigned bits = log_n - 2 * BR_BITS, m = blockIdx.x, rm = bits ? brev_bits(m, bits) : 0;
+  if (IN_PLACE && rm < m)
+    return;
+  const unsigned hi = threadIdx.x / BR_SIDE, lo = threadIdx.x % BR_SIDE;
+  const size_t at = (size_t)hi << (log_n - BR_BITS) | lo, here = at | (size_t)m << BR_BITS, there = at | (size_t)rm << BR_BITS;
+  const unsigned col = brev_bits(hi, BR_BITS), row = brev_bits(lo, BR_BITS);
+  const bool both = IN_PLACE && rm != m;
+  tile[0][hi][lo] = load_fe(in + here);
+  if (both)
+    tile[IN_PLACE][hi][lo] = load_fe(in + there);
+  __syncthreads();
+  store_fe(out + there, tile[0][row][col]);
+  if (both)
+    store_fe(out + here, tile[IN_PLACE][row][col]);
 }
 
 __global__ void select_kernel(const fe *__restrict__ src, fe *__restrict__ dst, const unsigned *__restrict__ idx, unsigned count) {
@@ -659,7 +685,13 @@ bc_error ff_bit_reverse(const void *values, void *result, unsigned log_count, bc
     return bc_error_invalid_value;
   const unsigned n = 1u << log_count;
   hipStream_t s = to_stream(stream);
-  if (values == result)
+  if (log_count >= BR_TILE_MIN) {
+    const unsigned blocks = n >> BR_TILE_MIN;
+    if (values == result)
+      bit_reverse_tile_kernel<true><<<blocks, BR_SIDE * BR_SIDE, 0, s>>>(static_cast<const fe *>(values), static_cast<fe *>(result), log_count);
+    else
+      bit_reverse_tile_kernel<false><<<blocks, BR_SIDE * BR_SIDE, 0, s>>>(static_cast<const fe *>(values), static_cast<fe *>(result), log_count);
+  } else if (values == result)
     bit_reverse_in_place_kernel<<<grid_for(n, 256), 256, 0, s>>>(static_cast<fe *>(result), log_count);
   else
     bit_reverse_kernel<<<grid_for(n, 256), 256, 0, s>>>(static_cast<const fe *>(values), static_cast<fe *>(result), log_count);

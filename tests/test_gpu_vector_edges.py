@@ -1,5 +1,7 @@
 """Fr vector operations at the edges of their kernels' tiles and chunks, against
 the CPU oracle."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -61,3 +63,19 @@ def test_evaluation_at_special_points(bellman, oracle, point):
     dev.sync()
     assert np.array_equal(result, oracle.poly_evaluate(x, base))
     dev.free(dx)
+
+
+# one thread an element below 2^8, then tiles of 256: a single one, one with no
+# middle bit to reverse, odd and even numbers of middle bits
+@pytest.mark.parametrize("log_n", [2, 7, 8, 9, 10, 11, 15, 18])
+def test_bit_reverse_at_tile_edges(bellman, oracle, log_n):
+    B, dev = bellman
+    n = 1 << log_n
+    x = oracle.random_fr(log_n + 29, n)
+    dx, dy = dev.upload(x), dev.malloc(n * 32)
+    for src, dst in ((dx, dy), (dx, dx)):
+        B.call("ff_bit_reverse", ctypes.c_void_p(src), ctypes.c_void_p(dst), ctypes.c_uint(log_n), dev.stream)
+        dev.sync()
+        assert np.array_equal(dev.download(dst, (n, 8)), oracle.bit_reverse(x, log_n))
+    dev.free(dx)
+    dev.free(dy)
