@@ -746,8 +746,8 @@ def hbm_copy_ceiling(lab, nbytes=1 << 30, reps=5):
 
 
 def pmc_traffic():
-    """HBM bytes per ntt_pass_kernel launch from the committed rocprofv3 counter summary, if present."""
-    path = os.path.join(ROOT, "profiles", "ntt_pass_kernel_2e24_counters.md")
+    """HBM bytes per launch of the 2^24 forward transform from the committed rocprofv3 counter summary, if present."""
+    path = os.path.join(ROOT, "profiles", "ntt_2e24_counters.md")
     try:
         for line in open(path):
             if line.startswith("traffic_bytes_per_launch:"):
@@ -805,23 +805,25 @@ def main():
         ntt_ms, inv_ms, lde_ms, ntt_ok = headline_ntt(lab, args.log_ntt, args.steps, args.warmup)
         log("ntt 2^%d: %.3f ms, inverse %.3f ms, lde x4 %.3f ms, round trip ok=%s" % (args.log_ntt, ntt_ms, inv_ms, lde_ms, ntt_ok))
         n = 1 << args.log_ntt
-        launches = (args.log_ntt + 9) // 10  # passes of at most 10 stages
+        # passes: at most 10 stages each up to 2^17, from 2^18 two of 6 stages on the matrix
+        # cores and the rest, from 2^23 three and the rest
+        launches = 1 if args.log_ntt <= 10 else 2 if args.log_ntt <= 17 else 3 if args.log_ntt <= 22 else 4
         per_launch_ms = ntt_ms / launches
         # algorithmic bytes: 64 n per NTT call (each 32 B element read and written
-        # once), i.e. 64 n / passes per launch of the pass kernel
+        # once), i.e. 64 n / passes per launch
         bytes_per_launch = 64.0 * n / launches
         achieved = bytes_per_launch / (per_launch_ms * 1e-3) / 1e9
         out.update({"ntt_ms": round(ntt_ms, 3), "ntt_inverse_ms": round(inv_ms, 3), "lde_4_cosets_ms": round(lde_ms, 3),
                     "ntt_call_gbs": round(64.0 * n / (ntt_ms * 1e-3) / 1e9, 1)})
         traffic = pmc_traffic()
-        out["roofline"] = {"bound": "hbm", "kernel": "ntt_pass_kernel (2^%d, %d launches per NTT)" % (args.log_ntt, launches),
+        out["roofline"] = {"bound": "hbm", "kernel": "ntt_mfma_kernel and ntt_mfma_last_kernel (2^%d, %d launches per NTT)" % (args.log_ntt, launches),
                            "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
                            "traffic": traffic, "algorithmic_bytes_per_launch": int(bytes_per_launch), "launch_ms": round(per_launch_ms, 4)}
         if traffic:
             # counter-measured HBM bytes per launch (profiles/ summary) over this run's launch time
             per_pass = traffic / (per_launch_ms * 1e-3) / 1e9
             out["hbm_per_pass"] = {"gbs": round(per_pass, 1), "frac": round(per_pass / HBM_PEAK_GBS, 4),
-                                   "source": "rocprofv3 FETCH_SIZE/WRITE_SIZE per ntt_pass_kernel launch, scaled by a copy kernel"}
+                                   "source": "rocprofv3 FETCH_SIZE/WRITE_SIZE per launch of the transform, scaled by a copy kernel"}
         out.setdefault("parity", {})["ntt_round_trip"] = ntt_ok
     if "msm" in parts:
         msm_ms, msm_ok, tuned_ms, tuned_ok = headline_msm(lab, args.log_msm, args.steps, args.warmup)

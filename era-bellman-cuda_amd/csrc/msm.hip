@@ -407,8 +407,8 @@ __device__ __forceinline__ uint32_t top_digit(const job_desc &jd, uint32_t w) {
 
 // Heavy buckets are reduced in chunks of HEAVY_CHUNK partial sums, one block
 // per chunk: a quad of lanes (quad29.cuh) sums every HEAVY_QUADS-th sum, then a
-// tree in LDS; the chunk's sum overwrites the chunk's first slot.  A second
-// kernel adds a bucket's chunk sums into its first slot.  There are few such
+// tree in LDS; the chunk's sum overwrites the chunk's first slot when the bucket
+// has several, whose sums a second kernel adds.  There are few such
 // buckets, so the additions in sequence set the time: 13 by quads, at 2.7 us
 // each, where a thread per point takes 14 at 7 us (2^12 points, 512 sums: 98 -> 41 us).
 
