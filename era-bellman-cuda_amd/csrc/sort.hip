@@ -488,11 +488,14 @@ hipError_t segmented_sort_kv(const uint64_t *in, uint64_t *out, const seg_group 
       const size_t wide_lds = ss_wide_lds(pl.widths[p]);
       BC_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)wide_lds));
       kernel<<<pl.t[p].tiles, SS_WIDE_BLOCK, wide_lds, stream>>>(pl.t[p], src, dst, pl.shifts[p], pl.widths[p], tab);
-    } else if (pl.widths[p] == 8)
-      ss_scatter_kv_staged_kernel<SS_BLOCK, SS_ITEMS, uint32_t, 8><<<pl.t[p].tiles, SS_BLOCK, lds, stream>>>(pl.t[p], src, dst, pl.shifts[p], 8, tab);
-    else if (lds <= SS_STAGED_MAX_LDS)
-      ss_scatter_kv_staged_kernel<SS_BLOCK, SS_ITEMS, uint32_t, 0><<<pl.t[p].tiles, SS_BLOCK, lds, stream>>>(pl.t[p], src, dst, pl.shifts[p], pl.widths[p], tab);
-    else
+    } else if (lds <= SS_STAGED_MAX_LDS) {
+      // unrolled for the widths of large sorts: 2^24 points at c = 17 18.33 -> 18.01 ms, 2^22 4.80 -> 4.71
+      const auto kernel = pl.widths[p] == 9   ? ss_scatter_kv_staged_kernel<SS_BLOCK, SS_ITEMS, uint32_t, 9>
+                          : pl.widths[p] == 8 ? ss_scatter_kv_staged_kernel<SS_BLOCK, SS_ITEMS, uint32_t, 8>
+                          : pl.widths[p] == 7 ? ss_scatter_kv_staged_kernel<SS_BLOCK, SS_ITEMS, uint32_t, 7>
+                                              : ss_scatter_kv_staged_kernel<SS_BLOCK, SS_ITEMS, uint32_t, 0>;
+      kernel<<<pl.t[p].tiles, SS_BLOCK, lds, stream>>>(pl.t[p], src, dst, pl.shifts[p], pl.widths[p], tab);
+    } else
       ss_scatter_kv_kernel<<<pl.t[p].tiles, SS_BLOCK, 0, stream>>>(pl.t[p], src, dst, pl.shifts[p], pl.widths[p], tab);
     BC_LAUNCH_CHECK();
     src = dst;
