@@ -373,8 +373,10 @@ hipError_t ntt_autotune(void *scratch, unsigned log_min, unsigned log_max, hipSt
       float ms = 0;
       auto record = [&](arena &ar) {
         const ntt_job pair[2] = {{buf, buf, L, false, false, 0, 0}, {buf, buf, L, true, true, 0, 0}};
-        BC_TRY(ntt_batch_device(&pair[0], 1, ar));
-        return ntt_batch_device(&pair[1], 1, ar);
+        // from NTT_MFMA_MIN_LOG on the table's entry is for bit-reversed inputs alone
+        if (L < NTT_MFMA_MIN_LOG)
+          BC_TRY(ntt_batch_device(&pair[0], 1, ar, false));
+        return ntt_batch_device(&pair[1], 1, ar, false);
       };
       BC_TRY(ws.fit(record));
       BC_TRY(time_median(

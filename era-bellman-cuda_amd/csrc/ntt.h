@@ -81,7 +81,9 @@ hipError_t ntt_prepare(unsigned max_log_n, hipStream_t stream, ntt_tables *out);
 hipError_t ntt_prepare_jobs(const ntt_job *jobs, unsigned count, hipStream_t stream);
 
 // Up to NTT_MAX_JOBS transforms, one launch per pass index and butterfly
-// order; temporaries (coset twist tables) come from `ar`.
-hipError_t ntt_batch_device(const ntt_job *jobs, unsigned count, arena &ar);
+// order; temporaries (coset twist tables) come from `ar`.  `small_passes` false:
+// also a launch that cannot fill the GPU takes the passes that the tuning table
+// names (the autotuner times those).
+hipError_t ntt_batch_device(const ntt_job *jobs, unsigned count, arena &ar, bool small_passes = true);
 
 } // namespace bc

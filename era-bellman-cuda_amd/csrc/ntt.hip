@@ -674,18 +674,14 @@ std::vector<pass_plan> plan_small_passes(unsigned L) {
   return p;
 }
 
-// Stage runs of the HBM passes: ceil(L / NTT_LOG_TILE) passes, balanced;
-// the tuning table may name the first pass's stage count, and the rest are
-// then balanced over the remaining passes.
+// Stage runs of the HBM passes.  Large natural-order transforms start on the
+// matrix cores, whatever the tuning table names (2^24: 1.28 ms against 2.2 ms in
+// named passes); else ceil(L / NTT_LOG_TILE) passes, balanced, or a first pass of
+// the named stage count and the rest balanced over the remaining ones.
 std::vector<pass_plan> plan_passes(unsigned L, bool bitrev_in, const fe *last_rows) {
   std::vector<pass_plan> p;
   unsigned passes = ntt_passes(L), s = 0;
-  const unsigned first = passes >= 2 ? ntt_first_pass(L) : 0;
-  if (first && ntt_split_valid(L, first)) {
-    p.push_back({0, first, false});
-    s = first;
-    passes--;
-  } else if (!bitrev_in && L >= NTT_MFMA_MIN_LOG) {
+  if (!bitrev_in && L >= NTT_MFMA_MIN_LOG) {
     // a third pass where a pass of VALU butterflies would follow it anyway
     const unsigned mfma_stages = L >= NTT_MFMA_ROWS_MIN_LOG ? mf::ROWS_STAGE + mf::STAGES : mf::ROWS_STAGE;
     for (; s < mfma_stages; s += mf::STAGES)
@@ -695,6 +691,10 @@ std::vector<pass_plan> plan_passes(unsigned L, bool bitrev_in, const fe *last_ro
       p.push_back({s, L, true, last_rows});
       return p;
     }
+  } else if (const unsigned first = passes >= 2 ? ntt_first_pass(L) : 0; first && ntt_split_valid(L, first)) {
+    p.push_back({0, first, false});
+    s = first;
+    passes--;
   }
   const unsigned rest = L - s;
   for (unsigned i = 0; i < passes; i++) {
@@ -800,7 +800,7 @@ hipError_t ntt_prepare(unsigned max_log_n, hipStream_t stream, ntt_tables *out) 
 hipError_t ntt_last_rows(const ntt_job &q, hipStream_t stream, const fe **rows) {
   *rows = nullptr;
   const unsigned L = q.log_n;
-  if (q.bitrev_in || !ntt_mfma_last(L) || ntt_first_pass(L))
+  if (q.bitrev_in || !ntt_mfma_last(L))
     return hipSuccess;
   std::lock_guard<std::mutex> lock(g_tw_mutex);
   const int d = device_slot();
@@ -842,7 +842,7 @@ hipError_t ntt_prepare_jobs(const ntt_job *jobs, unsigned count, hipStream_t str
   return hipSuccess;
 }
 
-hipError_t ntt_batch_device(const ntt_job *jobs, unsigned count, arena &ar) {
+hipError_t ntt_batch_device(const ntt_job *jobs, unsigned count, arena &ar, bool small_passes) {
   using F = FrParams;
   hipStream_t stream = ar.stream();
   if (count == 0)
@@ -884,14 +884,12 @@ hipError_t ntt_batch_device(const ntt_job *jobs, unsigned count, arena &ar) {
     BC_LAUNCH_CHECK();
   }
 
-  // a launch that cannot fill the GPU (a named first pass asks for the large one's passes)
+  // a launch that cannot fill the GPU takes the small passes, whatever the tuning
+  // table names for the large ones (2^12: 17 us against 28 us)
   uint64_t elements = 0;
-  bool small = max_log <= 2 * NTT_SMALL_LOG_TILE;
-  for (unsigned j = 0; j < count; j++) {
+  for (unsigned j = 0; j < count; j++)
     elements += 1ull << jobs[j].log_n;
-    small = small && !(ntt_passes(jobs[j].log_n) >= 2 && ntt_first_pass(jobs[j].log_n));
-  }
-  small = small && elements <= NTT_SMALL_ELEMENTS;
+  const bool small = small_passes && max_log <= 2 * NTT_SMALL_LOG_TILE && elements <= NTT_SMALL_ELEMENTS;
   const unsigned log_tile = small ? NTT_SMALL_LOG_TILE : NTT_LOG_TILE;
 
   std::vector<std::vector<pass_plan>> plans(count);

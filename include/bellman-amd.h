@@ -110,7 +110,9 @@ bc_error bc_amd_ntt_batch_async(const bc_amd_ntt_job *jobs, unsigned count, bc_m
 /* entries per thread, the job's `piece`) per log size; NTT: stages of the  */
 /* first HBM pass for sizes of two or more passes (log sizes 11..28, at     */
 /* most 10 stages per pass; the other passes share the rest evenly; 0 =     */
-/* balanced).  Tuning changes no folded MSM point and no NTT output.        */
+/* balanced).  The split is for launches of more than 2^17 elements and, from */
+/* 2^18 on, for bit-reversed inputs; other transforms take faster passes of  */
+/* their own.  Tuning changes no folded MSM point and no NTT output.        */
 
 typedef struct {
   unsigned window_bits;

@@ -29,3 +29,24 @@ def test_batches_around_the_line(bellman, oracle, logs):
     for i, (p, x, l) in enumerate(zip(bufs, xs, logs)):
         assert np.array_equal(dev.download(p, (1 << l, 8)), oracle.ntt(x, l, i % 2 == 1, i % 3 == 1, i % 2, 0)), i
         dev.free(p)
+
+
+@pytest.mark.parametrize("split", [6, 7, 10])
+def test_named_first_pass_in_a_larger_launch(bellman, oracle, split):
+    """A first pass named for a size serves launches above the line, both orders."""
+    import ctypes
+
+    B, dev = bellman
+    log_n, first = 16, ctypes.c_uint()
+    xs = [oracle.random_fr(0xBC0000E1 + i, 1 << log_n) for i in range(3)]
+    B.call("bc_amd_ntt_get_split", ctypes.c_uint(log_n), ctypes.byref(first))
+    B.call("bc_amd_ntt_set_split", ctypes.c_uint(log_n), ctypes.c_uint(split))
+    try:
+        bufs = [dev.upload(x) for x in xs]
+        ntt_batch(dev, [B.ntt_job(p, p, log_n, bitrev=i == 1, inverse=i == 2) for i, p in enumerate(bufs)])
+        for i, (p, x) in enumerate(zip(bufs, xs)):
+            assert np.array_equal(dev.download(p, (1 << log_n, 8)), oracle.ntt(x, log_n, i == 1, i == 2)), i
+            dev.free(p)
+        assert np.array_equal(ntt(dev, xs[0], log_n), oracle.ntt(xs[0], log_n))
+    finally:
+        B.call("bc_amd_ntt_set_split", ctypes.c_uint(log_n), first)
