@@ -124,11 +124,19 @@ private:
 };
 
 // Stream-ordered pool temporaries, streams and events of one call, released
-// on every return path (after everything the call enqueued).
+// on every return path, after everything the call enqueued.  Where a call ends
+// early its stream may not have waited for the work on the call's own streams yet
+// and does so here; streams_joined() says that it has.
 class call_resources {
 public:
   call_resources(hipMemPool_t pool, hipStream_t s) : pool_(pool), s_(s) {}
   ~call_resources() {
+    for (size_t i = joined_; i < streams_.size(); i++) {
+      const hipStream_t t = streams_[i];
+      hipEvent_t done = nullptr;
+      if (event(&done) != hipSuccess || hipEventRecord(done, t) != hipSuccess || hipStreamWaitEvent(s_, done, 0) != hipSuccess)
+        (void)hipStreamSynchronize(t);
+    }
     for (auto it = mem_.rbegin(); it != mem_.rend(); ++it)
       (void)hipFreeAsync(*it, s_);
     for (hipEvent_t e : events_)
@@ -153,6 +161,7 @@ public:
     streams_.push_back(*t);
     return hipSuccess;
   }
+  void streams_joined() { joined_ = streams_.size(); }
 
 private:
   hipMemPool_t pool_;
@@ -160,6 +169,7 @@ private:
   std::vector<void *> mem_;
   std::vector<hipEvent_t> events_;
   std::vector<hipStream_t> streams_;
+  size_t joined_ = 0; // of streams_, the first ones
 };
 
 enum class mem_kind { device, host_pinned, host_pageable };

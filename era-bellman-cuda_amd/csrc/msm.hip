@@ -1447,6 +1447,7 @@ hipError_t msm_execute_chunks(const msm_configuration &cfg, unsigned chunk_log, 
     return enqueue_copy(k + 1);
   };
   BC_TRY(msm_chunked_device(full, chunk_log, ar, inputs_of, consumed));
+  res.streams_joined(); // `s` has waited for every copy; it need not for the callback
   if (results_host) {
     BC_TRY(hipMemcpyAsync(cfg.results, d_results, sizeof(g1_jacobian) * 254, hipMemcpyDeviceToHost, s));
     if (cfg.d2h_copy_finished.handle)

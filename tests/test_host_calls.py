@@ -1,0 +1,98 @@
+"""What the library asks of the HIP runtime, and in which order, read on the CPU:
+libbellman.so is loaded over a runtime that runs nothing and lists the calls it
+gets (tests/hostrt/fake_hip.cpp).  Each test is a process of its own."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+PKG = os.path.join(ROOT, "era-bellman-cuda_amd")
+
+PRELUDE = """
+import ctypes, sys
+fake = ctypes.CDLL(%r, mode=ctypes.RTLD_GLOBAL)  # before libbellman.so, whose runtime calls it takes
+fake.fake_log.restype = ctypes.c_char_p
+import bellman_amd as B
+DEVICE = 32 << 40  # an address in device 0's memory
+PEER = 33 << 40    # and in device 1's
+
+def calls():
+    lines = fake.fake_log().decode().splitlines()
+    fake.fake_clear()
+    return [l.split() for l in lines]
+
+def stream_of(call):
+    return call[-1]
+
+def set_up():
+    B.call("ff_set_up", ctypes.c_uint(25), ctypes.c_uint(14))
+    B.call("ntt_set_up")
+    s = B.bc_stream()
+    B.call("bc_stream_create", ctypes.byref(s), ctypes.c_bool(False))
+    fake.fake_clear()
+    return s
+"""
+
+
+@pytest.fixture(scope="session")
+def run(tmp_path_factory):
+    """Runs a snippet in a process whose HIP runtime is the listing one."""
+    import bellman_amd as B
+
+    if not os.path.exists(B.LIB_PATH):
+        pytest.skip("libbellman.so not built")
+    fake = str(tmp_path_factory.mktemp("hostrt") / "libfakehip.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-Wno-attributes",
+                    os.path.join(ROOT, "tests", "hostrt", "fake_hip.cpp"), "-o", fake], check=True, capture_output=True)
+
+    def go(body):
+        p = subprocess.run([sys.executable, "-c", PRELUDE % fake + body], capture_output=True, text=True, env=dict(os.environ, PYTHONPATH=PKG), timeout=120)
+        assert p.returncode == 0, p.stdout + p.stderr
+
+    return go
+
+
+@pytest.mark.parametrize("log_n", [20, 22])
+def test_staging_memory_is_released_after_the_copies(run, log_n):
+    """An MSM over host inputs that fails with a chunk's copy still running on
+    the copy stream: the call's stream waits for that stream before it gives the
+    staging memory back."""
+    run("""
+s = set_up()
+cfg = B.msm_configuration()
+scalars = ctypes.create_string_buffer(32)  # not read: copies are only listed
+cfg.stream, cfg.bases, cfg.scalars, cfg.results, cfg.log_scalars_count = s, DEVICE, ctypes.addressof(scalars), DEVICE, %d
+cfg.h2d_copy_finished_callback = B.bc_host_fn(lambda data: None)
+fake.fake_fail(b"host_func")  # enqueued after the last copy, before the call's stream waits for it
+assert B.lib().msm_execute_async(cfg) != 0
+log = calls()
+mine = "s=%%x" %% s.handle
+last = max(i for i, c in enumerate(log) if c[0] == "memcpy")
+side = stream_of(log[last])
+assert side != mine
+freed = min(i for i, c in enumerate(log) if c[0] == "free_async" and i > last)
+events = [c[1] for c in log[last:freed] if c[0] == "record" and c[2] == side]
+waits = [c[1] for c in log[last:freed] if c[0] == "wait" and c[2] == mine]
+assert set(events) & set(waits), log[last:]
+""" % log_n)
+
+
+def test_a_finished_msm_does_not_wait_for_the_callback(run):
+    """Where the call succeeds, its stream waits for the copies (events recorded
+    before the callback), not for the callback after them."""
+    run("""
+s = set_up()
+cfg = B.msm_configuration()
+scalars = ctypes.create_string_buffer(32)
+cfg.stream, cfg.bases, cfg.scalars, cfg.results, cfg.log_scalars_count = s, DEVICE, ctypes.addressof(scalars), DEVICE, 20
+cfg.h2d_copy_finished_callback = B.bc_host_fn(lambda data: None)
+B.call("msm_execute_async", cfg)
+log = calls()
+mine = "s=%x" % s.handle
+at = next(i for i, c in enumerate(log) if c[0] == "host_func")
+assert log[at][1] != mine
+after = [c[1] for c in log[at:] if c[0] == "record" and c[2] == log[at][1]]
+assert not [c for c in log if c[0] == "wait" and c[2] == mine and c[1] in after]
+""")
