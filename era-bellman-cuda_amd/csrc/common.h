@@ -179,4 +179,8 @@ enum class mem_kind { device, host_pinned, host_pageable };
 // with an error is treated as unregistered host memory.
 mem_kind classify_pointer(const void *p);
 
+// Memory of the GPU that `stream` runs on, which its kernels may write whatever
+// peer access there is.
+bool on_device_of(hipStream_t stream, const void *p);
+
 } // namespace bc

@@ -518,11 +518,11 @@ hipError_t poly_evaluate(const fe *values, const void *point, void *result, size
     power_digits_kernel<<<1, 1, 0, s>>>(point_ref, tables, levels, EVAL_DIGITS + 1, log_tile);
     BC_LAUNCH_CHECK();
   }
-  const bool to_device = classify_pointer(result) == mem_kind::device;
-  fe *sums = nullptr; // the partial sums of every level, then the result if it goes to the host
-  if (partials || !to_device)
+  const bool in_place = on_device_of(s, result); // else it is copied: to the host, or to a GPU whose memory may not be mapped here
+  fe *sums = nullptr; // the partial sums of every level, then the result to copy
+  if (partials || !in_place)
     BC_TRY(res.get(&sums, partials + 1));
-  fe *last = to_device ? static_cast<fe *>(result) : sums + partials;
+  fe *last = in_place ? static_cast<fe *>(result) : sums + partials;
   for (unsigned level = 0; level < levels; level++) {
     power_digits arg;
     if (!tables)
@@ -539,8 +539,8 @@ hipError_t poly_evaluate(const fe *values, const void *point, void *result, size
     for (size_t i = 1; !tables && i < tile; i <<= 1)
       x = mul<FrParams>(x, x);
   }
-  if (!to_device)
-    BC_TRY(hipMemcpyAsync(result, last, sizeof(fe), hipMemcpyDeviceToHost, s));
+  if (!in_place)
+    BC_TRY(hipMemcpyAsync(result, last, sizeof(fe), hipMemcpyDefault, s));
   return hipSuccess;
 }
 

@@ -26,6 +26,15 @@ mem_kind classify_pointer(const void *p) {
   }
 }
 
+bool on_device_of(hipStream_t stream, const void *p) {
+  hipPointerAttribute_t attr{};
+  hipDevice_t device = -1;
+  if (hipPointerGetAttributes(&attr, p) == hipSuccess && hipStreamGetDevice(stream, &device) == hipSuccess)
+    return attr.type == hipMemoryTypeDevice && attr.device == device;
+  (void)hipGetLastError();
+  return false;
+}
+
 // HIP statuses are CUDA's values (cudaError_t of CUDA 11.8, the toolkit the
 // reference builds with) with four exceptions, which are mapped to the CUDA
 // status of the same meaning; a value outside both enumerations reads as

@@ -131,6 +131,7 @@ hipError_t hipMemsetAsync(void *, int, size_t, hipStream_t) { return hipSuccess;
 
 hipError_t hipStreamCreate(hipStream_t *s) { return handle("stream", s); }
 hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { return handle("stream", s); }
+hipError_t hipStreamGetDevice(hipStream_t, hipDevice_t *d) { return *d = 0, hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t s) { return note("synchronize s=%llx", n(s)), hipSuccess; }
 hipError_t hipStreamQuery(hipStream_t) { return hipSuccess; }

@@ -96,3 +96,20 @@ assert log[at][1] != mine
 after = [c[1] for c in log[at:] if c[0] == "record" and c[2] == log[at][1]]
 assert not [c for c in log if c[0] == "wait" and c[2] == mine and c[1] in after]
 """)
+
+
+@pytest.mark.parametrize("count", [0, 100, 65539, 1 << 22])
+@pytest.mark.parametrize("where", ["own", "peer", "host"])
+def test_a_polynomial_value_for_another_gpu_is_copied(run, count, where):
+    """Kernels write a result in the memory of the stream's GPU; one in the host's
+    or another GPU's memory, which no kernel here may reach, is copied."""
+    run("""
+s = set_up()
+host = ctypes.create_string_buffer(32)
+result = {"own": DEVICE + 4096, "peer": PEER, "host": ctypes.addressof(host)}[%r]
+point = (ctypes.c_uint * 8)(3)
+B.call("ff_poly_evaluate", B.ff_poly_evaluate_configuration(B.bc_mem_pool(), s, DEVICE, ctypes.addressof(point), result, %d))
+copies = [c for c in calls() if c[0] == "memcpy"]
+assert [int(c[1], 16) for c in copies] == ([] if result == DEVICE + 4096 else [result])
+assert all(c[3] == "32" and stream_of(c) == "s=%%x" %% s.handle for c in copies)
+""" % (where, count))
