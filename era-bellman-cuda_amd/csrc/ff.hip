@@ -449,8 +449,13 @@ hipError_t poly_eval_launch(unsigned K, const power_digits &arg, const power_dig
   return hipGetLastError();
 }
 
-// A scalar argument: the value of a host scalar, or where a device one lies.
-const fe *scalar_argument(const void *p, fe *value) {
+// A scalar argument of a call over n elements: the value of a host scalar, or
+// where a device one lies.  One element has the power 0 alone, whatever the
+// scalar, which may then be missing.
+const fe *scalar_argument(const void *p, size_t n, fe *value) {
+  *value = fe_zero();
+  if (n <= 1)
+    return nullptr;
   if (classify_pointer(p) == mem_kind::device)
     return static_cast<const fe *>(p);
   memcpy(value, p, sizeof(fe));
@@ -461,7 +466,7 @@ hipError_t multiply_by_powers(const fe *in, const void *base, fe *out, unsigned 
   const unsigned digits = power_digits_for(n);
   power_digits arg;
   fe b;
-  const fe *base_ref = scalar_argument(base, &b);
+  const fe *base_ref = scalar_argument(base, n, &b);
   call_resources res(pool, s);
   power_digits *ref = nullptr;
   if (base_ref) {
@@ -507,7 +512,7 @@ hipError_t poly_evaluate(const fe *values, const void *point, void *result, size
     partials += m;
   }
   fe x;
-  const fe *point_ref = scalar_argument(point, &x);
+  const fe *point_ref = scalar_argument(point, n, &x);
   call_resources res(pool, s);
   power_digits *tables = nullptr;
   if (point_ref) {

@@ -113,3 +113,39 @@ copies = [c for c in calls() if c[0] == "memcpy"]
 assert [int(c[1], 16) for c in copies] == ([] if result == DEVICE + 4096 else [result])
 assert all(c[3] == "32" and stream_of(c) == "s=%%x" %% s.handle for c in copies)
 """ % (where, count))
+
+
+def test_at_most_one_element_needs_no_scalar(run):
+    """The only power of the point or base is then the 0th."""
+    run("""
+s = set_up()
+pool = B.bc_mem_pool()
+for n in (0, 1):
+    B.call("ff_poly_evaluate", B.ff_poly_evaluate_configuration(pool, s, DEVICE, None, DEVICE + 4096, n))
+    assert [c[0] for c in calls()] == ["launch"]
+B.call("ff_multiply_by_powers", B.ff_multiply_by_powers_configuration(pool, s, DEVICE, None, DEVICE + 4096, 1))
+assert [c[0] for c in calls()] == ["launch"]
+""")
+
+
+@pytest.mark.gpu
+def test_one_element_with_and_without_a_scalar(bellman, oracle):
+    import ctypes
+
+    import numpy as np
+
+    B, dev = bellman
+    x = oracle.random_fr(0xBC0000F1, 1)
+    dx, dy = dev.upload(x), dev.malloc(32)
+    point = oracle.random_fr(0xBC0000F2, 1)
+    for p in (None, point.ctypes.data):
+        for name in ("ff_poly_evaluate", "ff_multiply_by_powers"):
+            B.call("bc_memset", B.ptr(dy), ctypes.c_int(0x5A), ctypes.c_size_t(32))
+            if name == "ff_poly_evaluate":
+                B.call(name, B.ff_poly_evaluate_configuration(dev.pool, dev.stream, dx, p, dy, 1))
+            else:
+                B.call(name, B.ff_multiply_by_powers_configuration(dev.pool, dev.stream, dx, p, dy, 1))
+            dev.sync()
+            assert np.array_equal(dev.download(dy, (1, 8)), x), name
+    for p in (dx, dy):
+        dev.free(p)
