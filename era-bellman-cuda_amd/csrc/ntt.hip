@@ -462,8 +462,9 @@ __global__ __launch_bounds__(mf::BLOCK, 4) void ntt_mfma_kernel(const pass_table
     for (unsigned i = 0; i < 4; i++)
       x[i] = mul_lazy<F>(x[i], w[i]);
   }
-  // inputs below 2r (the transform's, products), or below 4r as this kernel leaves them: 2r off
-  if (s_lo == 0 || a.pre_table) {
+  // products are below 2r; the transform's inputs and what this kernel leaves are below
+  // 4r and taken 2r off, as the matrix products need |x| < 2.64 r
+  if (a.pre_table) {
 #pragma unroll
     for (unsigned i = 0; i < 4; i++)
       x[i] = mf::add_offset(x[i], mf::offset(0, 1));
