@@ -266,7 +266,7 @@ template <unsigned G, unsigned K> __global__ __launch_bounds__(INV_BLOCK, G == 1
     for (unsigned k = 0; k < K; k++) {
       before[k] = acc;
       if (!fe_is_zero(v[k]))
-        acc = mul_lazy<F>(acc, v[k]);
+        acc = mul<F>(acc, v[k]); // canonical: then v may be any 256 bits
     }
   };
 #pragma unroll 1
@@ -308,7 +308,7 @@ template <unsigned G, unsigned K> __global__ __launch_bounds__(INV_BLOCK, G == 1
           store_fe(out + i, v);
         } else {
           store_fe(out + i, mul<F>(before[k], inv));
-          inv = mul_lazy<F>(inv, v);
+          inv = mul<F>(inv, v);
         }
       }
     }
@@ -382,7 +382,8 @@ __global__ __launch_bounds__(256) void multiply_by_powers_kernel(const fe *fine,
   const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= count)
     return;
-  const fe v = load_fe(in + i), w = mul_lazy<FrParams>(load_fe(fine + (i & (POWERS_FINE - 1))), load_fe(coarse + (i >> POWERS_LOG_FINE)));
+  // the power canonical: then v may be any 256 bits
+  const fe v = load_fe(in + i), w = mul<FrParams>(load_fe(fine + (i & (POWERS_FINE - 1))), load_fe(coarse + (i >> POWERS_LOG_FINE)));
   store_fe(out + i, mul<FrParams>(v, w));
 }
 
@@ -407,8 +408,8 @@ __global__ __launch_bounds__(EVAL_BLOCK) void poly_eval_kernel(const power_digit
       v[k] = i < n ? load_fe(values + i) : fe_zero();
     }
 #pragma unroll
-    for (unsigned k = G; k-- > 0;) // acc < 3m, x^EVAL_BLOCK canonical: the product is below 2m
-      acc = K == 1 ? v[0] : add_raw(mul_lazy<F>(acc, t.p[EVAL_DIGITS][0]), v[k]);
+    for (unsigned k = G; k-- > 0;) // any v is below 5.3 m, below 3.3 m reduced; x^EVAL_BLOCK is canonical, so a product is below 2m and acc below 2^256
+      acc = K == 1 ? v[0] : add_raw(mul_lazy<F>(acc, t.p[EVAL_DIGITS][0]), reduce2<F>(v[k]));
   }
   acc = mul_lazy<F>(acc, power_of(t, threadIdx.x, EVAL_DIGITS));
 #pragma unroll

@@ -31,3 +31,61 @@ def test_natural_order_transforms_below_4r(bellman, oracle, log_n, inverse, log_
     x[::5] = oracle.to_limbs([oracle.R - 1])[0]
     got = ntt(dev, add_multiples(oracle, x, 3), log_n, inverse=inverse, log_ext=log_ext, coset=log_ext)
     assert np.array_equal(got, oracle.ntt(x, log_n, False, inverse, log_ext, log_ext))
+
+
+def wide(oracle, seed, n):
+    """Reduced values, and the same with up to 5 r added (no multiple of r but 0 itself)."""
+    x = oracle.random_fr(seed, n)
+    x[::5] = oracle.to_limbs([oracle.R - 1])[0]
+    x[::7] = oracle.to_limbs([1])[0]
+    return x, add_multiples(oracle, x, 5)
+
+
+# every form of the inverse (blocks of 512, 2048, 4096 and 8192 elements)
+@pytest.mark.parametrize("n", [2, 600, 65539, (1 << 19) + 1, (1 << 20) + 3, (1 << 21) + 5])
+@pytest.mark.parametrize("in_place", [False, True])
+def test_batch_inverse_of_any_256_bits(bellman, oracle, n, in_place):
+    B, dev = bellman
+    x, y = wide(oracle, 0xBC0000B7 + n, n)
+    x[3::11] = y[3::11] = 0
+    d_in = dev.upload(y)
+    d_out = d_in if in_place else dev.malloc(n * 32)
+    B.call("ff_inverse", B.ff_inverse_configuration(dev.pool, dev.stream, d_in, d_out, n))
+    dev.sync()
+    got = dev.download(d_out, (n, 8))
+    for p in {d_in, d_out}:
+        dev.free(p)
+    assert np.array_equal(got, oracle.batch_inverse(x))
+
+
+# one, two, eight and 32 elements a thread, one to three launches
+@pytest.mark.parametrize("n", [2, 256, 257, 513, 2048, 2049, 65539, (1 << 17) + 1, (1 << 21) + 1, 4194299])
+def test_polynomial_values_of_any_256_bits(bellman, oracle, n):
+    B, dev = bellman
+    x, y = wide(oracle, 0xBC0000C7 + n, n)
+    point = oracle.random_fr(0xBC0000C8, 1)
+    values = []
+    for v in (x, y):
+        d_in, d_out = dev.upload(v), dev.malloc(32)
+        B.call("ff_poly_evaluate", B.ff_poly_evaluate_configuration(dev.pool, dev.stream, d_in, point.ctypes.data, d_out, n))
+        dev.sync()
+        values.append(dev.download(d_out, (1, 8)))
+        dev.free(d_in)
+        dev.free(d_out)
+    assert np.array_equal(values[1], values[0])
+
+
+@pytest.mark.parametrize("n", [2, 65539, (1 << 17) + 1, (1 << 20) + 7])
+def test_products_with_powers_of_any_256_bits(bellman, oracle, n):
+    B, dev = bellman
+    x, y = wide(oracle, 0xBC0000D7 + n, n)
+    base = oracle.random_fr(0xBC0000D8, 1)
+    got = []
+    for v in (x, y):
+        d_in, d_out = dev.upload(v), dev.malloc(n * 32)
+        B.call("ff_multiply_by_powers", B.ff_multiply_by_powers_configuration(dev.pool, dev.stream, d_in, base.ctypes.data, d_out, n))
+        dev.sync()
+        got.append(dev.download(d_out, (n, 8)))
+        dev.free(d_in)
+        dev.free(d_out)
+    assert np.array_equal(got[1], got[0])
