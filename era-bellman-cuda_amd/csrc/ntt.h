@@ -31,7 +31,8 @@ constexpr uint64_t NTT_SMALL_ELEMENTS = 1u << 17;
 
 // Transforms whose last pass (6..10 stages, one launch) starts on the matrix
 // cores.  Its row factors are a table of 2^log_n elements per direction, so it is
-// kept to tables of 512 MB.
+// kept to tables of 512 MB: for all sizes 56 MB a direction to 2^20, 760 MB to 2^24,
+// beside twiddles of 32 and 512 MB.
 constexpr unsigned NTT_MFMA_LAST_MAX_LOG = 24;
 inline bool ntt_mfma_last(unsigned log_n) {
   return log_n >= NTT_MFMA_MIN_LOG && log_n <= NTT_MFMA_LAST_MAX_LOG && log_n != NTT_MFMA_ROWS_MIN_LOG;
@@ -69,6 +70,7 @@ struct ntt_tables {
   const fe *fwd, *inv, *inv_sizes;
   const int8_t *mfma_fwd, *mfma_inv;
   const fe *rows_fwd, *rows_inv;
+  const fe *last_rows[2][NTT_MFMA_LAST_MAX_LOG + 1]; // by direction and size; null: VALU passes
   unsigned log_size;
 };
 
@@ -77,7 +79,7 @@ struct ntt_tables {
 // afterwards every batch of transforms up to that size is capturable.
 hipError_t ntt_prepare(unsigned max_log_n, hipStream_t stream, ntt_tables *out);
 
-// The same for these jobs, with the tables that are made per size and direction.
+// The same for the largest of these jobs.
 hipError_t ntt_prepare_jobs(const ntt_job *jobs, unsigned count, hipStream_t stream);
 
 // Up to NTT_MAX_JOBS transforms, one launch per pass index and butterfly

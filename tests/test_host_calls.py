@@ -149,3 +149,68 @@ def test_one_element_with_and_without_a_scalar(bellman, oracle):
             assert np.array_equal(dev.download(dy, (1, 8)), x), name
     for p in (dx, dy):
         dev.free(p)
+
+
+NTT = """
+def transform(log_n, inverse, bitrev=False, log_ext=0):
+    cfg = B.ntt_configuration()
+    cfg.stream, cfg.inputs, cfg.outputs, cfg.log_values_count, cfg.inverse, cfg.bit_reversed_inputs = s, DEVICE, DEVICE, log_n, inverse, bitrev
+    cfg.log_extension_degree = log_ext
+    B.call("ntt_execute_async", cfg)
+    return calls()
+
+def kernels(log):
+    return [c[1] for c in log if c[0] == "launch"]
+
+def waits_or_allocates(log):
+    return [c for c in log if c[0] in ("malloc", "synchronize", "device")]
+"""
+
+
+def test_transforms_neither_allocate_nor_wait(run):
+    """Up to the size that the tables were made for, from the first transform on,
+    with and without the field's power tables."""
+    run(NTT + """
+s = set_up()
+for tear_down in (False, True):
+    if tear_down:
+        B.call("ff_tear_down")
+        calls()
+    for log_n in (12, 17, 18, 19, 20):
+        for inverse in (False, True):
+            log = transform(log_n, inverse)
+            assert [c[0] for c in log] == ["launch"] * len(log), log
+            assert any("ntt_mfma_last" in k for k in kernels(log)) == (log_n >= 18)
+""")
+
+
+def test_one_growth_makes_every_table(run):
+    run(NTT + """
+s = set_up()
+grown = transform(24, False)
+assert waits_or_allocates(grown)
+for log_n in (18, 21, 22, 23, 24):
+    for inverse in (False, True):
+        log = transform(log_n, inverse)
+        assert not waits_or_allocates(log), log
+        assert any("ntt_mfma_last" in k for k in kernels(log)) == (log_n != 23)
+B.call("ntt_tear_down")
+freed = [c for c in calls() if c[0] == "free"]
+# twiddles of both sizes, powers of 1/2, matrices, row factors of the third pass and of the last pass of six sizes
+assert len(freed) == 2 + 2 + 1 + 1 + 1 + 12 and len(set(c[1] for c in freed)) == len(freed)
+""")
+
+
+def test_a_nearly_full_gpu_keeps_its_memory(run):
+    """Without room to spare the last stages are VALU passes, and no call tries again."""
+    run(NTT + """
+fake.fake_memory(ctypes.c_size_t(30 << 30), ctypes.c_size_t(256 << 30))
+s = set_up()
+transform(24, True)
+for log_n in (18, 20, 22, 24):
+    for inverse in (False, True):
+        log = transform(log_n, inverse)
+        assert not waits_or_allocates(log), log
+        names = kernels(log)
+        assert not any("ntt_mfma_last" in k for k in names) and any("ntt_pass_kernel" in k for k in names) and "ntt_mfma" in names[0], names
+""")
