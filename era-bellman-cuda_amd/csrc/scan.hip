@@ -288,11 +288,22 @@ hipError_t prefix_product(const fe *in, fe *out, size_t n, arena &ar) {
       prefix_product_tile_kernel<4><<<1, SCAN_BLOCK, 0, stream>>>(in, out, nullptr, n);
     return hipGetLastError();
   }
-  const bool chunked = n > PP_TILES_MAX;
-  const size_t items = chunked ? (n + PP_CHUNK - 1) / PP_CHUNK : n; // elements or chunk products to scan in tiles
-  const size_t tiles = (items + PP_TILE - 1) / PP_TILE;
+  // the chunk products are n / 8 elements; a pool without them still has the tile
+  // products' n / 1024
+  bool chunked = n > PP_TILES_MAX;
+  size_t items = 0, tiles = 0; // elements or chunk products to scan in tiles
   fe *temp = nullptr;
-  BC_TRY(ar.get(&temp, tiles + (chunked ? items : 0)));
+  for (;;) {
+    items = chunked ? (n + PP_CHUNK - 1) / PP_CHUNK : n;
+    tiles = (items + PP_TILE - 1) / PP_TILE;
+    const hipError_t e = ar.get(&temp, tiles + (chunked ? items : 0));
+    if (e == hipSuccess)
+      break;
+    if (e != hipErrorOutOfMemory || !chunked)
+      return e;
+    (void)hipGetLastError();
+    chunked = false;
+  }
   fe *tile_products = temp, *chunk_products = temp + tiles;
   if (chunked) {
     prefix_product_chunk_kernel<<<grid_for(items, SCAN_BLOCK), SCAN_BLOCK, 0, stream>>>(in, chunk_products, n);

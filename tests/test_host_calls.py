@@ -214,3 +214,49 @@ for log_n in (18, 20, 22, 24):
         names = kernels(log)
         assert not any("ntt_mfma_last" in k for k in names) and any("ntt_pass_kernel" in k for k in names) and "ntt_mfma" in names[0], names
 """)
+
+
+def test_grand_product_where_the_pool_is_small(run):
+    """4194299 elements: 16 MiB of chunk products, or 132 KiB of tile products where
+    the pool has no more."""
+    run("""
+s = set_up()
+cfg = B.ff_grand_product_configuration(B.bc_mem_pool(), s, DEVICE, DEVICE, 4194299)
+B.call("ff_grand_product", cfg)
+assert any("chunk" in c[1] for c in calls() if c[0] == "launch")
+fake.fake_largest(ctypes.c_size_t(1 << 20))
+B.call("ff_grand_product", cfg)
+log = calls()
+names = [c[1] for c in log if c[0] == "launch"]
+assert len(names) == 5 and not any("chunk" in k or "apply" in k for k in names), names
+assert sorted(c[1] for c in log if c[0] == "malloc_async" and c[1] != "refused") == sorted(c[1] for c in log if c[0] == "free_async")
+fake.fake_largest(ctypes.c_size_t(1 << 10))
+assert B.lib().ff_grand_product(cfg) == B.bc_error_memory_allocation
+""")
+
+
+@pytest.mark.gpu
+def test_grand_product_from_a_pool_of_four_mebibytes(bellman, oracle):
+    import ctypes
+
+    import numpy as np
+
+    B, dev = bellman
+
+    class pool_properties(ctypes.Structure):  # hipMemPoolProps
+        _fields_ = [("type", ctypes.c_int), ("handles", ctypes.c_int), ("location", ctypes.c_int), ("device", ctypes.c_int),
+                    ("attributes", ctypes.c_void_p), ("most", ctypes.c_size_t), ("reserved", ctypes.c_ubyte * 56)]
+
+    pool = B.bc_mem_pool()
+    assert B.lib().hipMemPoolCreate(ctypes.byref(pool), ctypes.byref(pool_properties(type=1, location=1, device=0, most=4 << 20))) == 0
+    n = 4194299
+    x = oracle.random_fr(0xBC0000F9, n)
+    dx, dy = dev.upload(x), dev.malloc(n * 32)
+    p = ctypes.c_void_p()
+    assert B.lib().bc_malloc_from_pool_async(ctypes.byref(p), ctypes.c_size_t(16 << 20), pool, dev.stream) == B.bc_error_memory_allocation
+    B.call("ff_grand_product", B.ff_grand_product_configuration(pool, dev.stream, dx, dy, n))
+    dev.sync()
+    assert np.array_equal(dev.download(dy, (n, 8)), oracle.grand_product(x))
+    B.call("bc_mem_pool_destroy", pool)
+    dev.free(dx)
+    dev.free(dy)
