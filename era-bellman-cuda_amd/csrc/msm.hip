@@ -1392,11 +1392,12 @@ hipError_t msm_execute_chunks(const msm_configuration &cfg, unsigned chunk_log, 
   BC_TRY(res.get(&block, bytes));
   arena ar = arena::bump_mode(block, bytes, s);
 
-  // Several chunks' copies run on their own stream: chunk k's copy is enqueued
-  // right after chunk k - 1's kernels (so a pageable copy, which holds the host
-  // thread, overlaps them), into slot k % 2 once chunk k - 2 has been consumed.
-  // A single copy runs on the call's stream.
-  const bool own_stream = copying && K > 1;
+  // Copies run on their own stream: chunk k's copy is enqueued right after chunk
+  // k - 1's kernels (so a pageable copy, which holds the host thread, overlaps
+  // them), into slot k % 2 once chunk k - 2 has been consumed.  A single copy runs
+  // on the call's stream, unless a callback follows it, which would hold up the
+  // kernels there.
+  const bool own_stream = copying && (K > 1 || cfg.h2d_copy_finished_callback);
   hipStream_t cs = s;
   std::vector<hipEvent_t> loaded(K), freed(2);
   auto enqueue_copy = [&](unsigned k) -> hipError_t {

@@ -79,23 +79,24 @@ assert set(events) & set(waits), log[last:]
 """ % log_n)
 
 
-def test_a_finished_msm_does_not_wait_for_the_callback(run):
+@pytest.mark.parametrize("log_n", [4, 18, 20])
+def test_a_finished_msm_does_not_wait_for_the_callback(run, log_n):
     """Where the call succeeds, its stream waits for the copies (events recorded
     before the callback), not for the callback after them."""
     run("""
 s = set_up()
 cfg = B.msm_configuration()
 scalars = ctypes.create_string_buffer(32)
-cfg.stream, cfg.bases, cfg.scalars, cfg.results, cfg.log_scalars_count = s, DEVICE, ctypes.addressof(scalars), DEVICE, 20
+cfg.stream, cfg.bases, cfg.scalars, cfg.results, cfg.log_scalars_count = s, DEVICE, ctypes.addressof(scalars), DEVICE, %d
 cfg.h2d_copy_finished_callback = B.bc_host_fn(lambda data: None)
 B.call("msm_execute_async", cfg)
 log = calls()
-mine = "s=%x" % s.handle
+mine = "s=%%x" %% s.handle
 at = next(i for i, c in enumerate(log) if c[0] == "host_func")
 assert log[at][1] != mine
 after = [c[1] for c in log[at:] if c[0] == "record" and c[2] == log[at][1]]
 assert not [c for c in log if c[0] == "wait" and c[2] == mine and c[1] in after]
-""")
+""" % log_n)
 
 
 @pytest.mark.parametrize("count", [0, 100, 65539, 1 << 22])
