@@ -48,7 +48,7 @@ def run(tmp_path_factory):
                     os.path.join(ROOT, "tests", "hostrt", "fake_hip.cpp"), "-o", fake], check=True, capture_output=True)
 
     def go(body):
-        p = subprocess.run([sys.executable, "-c", PRELUDE % fake + body], capture_output=True, text=True, env=dict(os.environ, PYTHONPATH=PKG), timeout=120)
+        p = subprocess.run([sys.executable, "-c", PRELUDE % fake + body], capture_output=True, text=True, env=dict(os.environ, PYTHONPATH=os.pathsep.join((PKG, ROOT))), timeout=120)
         assert p.returncode == 0, p.stdout + p.stderr
 
     return go
@@ -261,3 +261,62 @@ def test_grand_product_from_a_pool_of_four_mebibytes(bellman, oracle):
     B.call("bc_mem_pool_destroy", pool)
     dev.free(dx)
     dev.free(dy)
+
+
+def test_plain_msm_memory_is_its_footprint(run):
+    """The one block that a plain MSM takes is the footprint of its window width
+    with some chunk of sorted entries, the chunk grows with the size, and the largest
+    call of the fixed array is the last whose footprint fits it."""
+    run("""
+from oracle import oracle as O
+s = set_up()
+def footprint(log_n, piece):
+    job, out = B.bc_amd_job(), ctypes.c_size_t()
+    job.kind, job.msm = B.BC_AMD_JOB_MSM, B.msm_job(DEVICE, DEVICE, DEVICE, log_n, O.msm_window_bits(log_n), piece)
+    B.call("bc_amd_job_footprint", ctypes.byref(job), ctypes.byref(out))
+    return out.value
+taken, pieces = [], []
+for log_n in range(27):
+    cfg = B.msm_configuration()
+    cfg.stream, cfg.bases, cfg.scalars, cfg.results, cfg.log_scalars_count = s, DEVICE, DEVICE, DEVICE, log_n
+    B.call("msm_execute_async", cfg)
+    blocks = [int(c[2]) for c in calls() if c[0] == "malloc_async"]
+    fitting = [p for p in (4, 8, 16, 32, 64, 128) if footprint(log_n, p) == blocks[0]]
+    assert len(blocks) == 1 and fitting, (log_n, blocks)
+    taken.append(blocks[0])
+    pieces.append(max(fitting))
+assert all(a <= b for a, b in zip(pieces[10:], pieces[11:])) and pieces[26] == 128, pieces
+for log_n in (16, 17, 18):
+    cfg.log_scalars_count = log_n
+    fits = taken[log_n] <= 192 << 20
+    assert fits == (log_n <= 17)
+    assert (B.lib().bc_amd_msm_execute_no_alloc(cfg) == B.bc_success) == fits
+    assert not [c for c in calls() if c[0].startswith("malloc")]
+""")
+
+
+def test_four_chunks_of_host_inputs_reuse_two_slots(run):
+    """At 2^22 points the copy of chunk k + 2 waits for the kernels of chunk k."""
+    run("""
+s = set_up()
+scalars = ctypes.create_string_buffer(32)
+cfg = B.msm_configuration()
+cfg.stream, cfg.bases, cfg.scalars, cfg.results, cfg.log_scalars_count = s, DEVICE, ctypes.addressof(scalars), DEVICE, 22
+B.call("msm_execute_async", cfg)
+log = calls()
+mine = "s=%x" % s.handle
+copies = [i for i, c in enumerate(log) if c[0] == "memcpy"]
+assert [int(log[i][3]) for i in copies] == [32 << 20] * 4
+assert log[copies[0]][1] == log[copies[2]][1] != log[copies[1]][1] == log[copies[3]][1]
+side = stream_of(log[copies[0]])
+accumulated = [i for i, c in enumerate(log) if c[0] == "launch" and "bucket_gather" in c[1]]
+assert len(accumulated) == 4 and all(stream_of(log[i]) == mine for i in accumulated)
+for k in (2, 3):
+    waits = [c[1] for c in log[copies[k - 1]:copies[k]] if c[0] == "wait" and c[2] == side]
+    freed = [c[1] for c in log[accumulated[k - 2]:copies[k]] if c[0] == "record" and c[2] == mine]
+    assert set(waits) & set(freed), (k, log[copies[k - 1]:copies[k]])
+for k in range(4):  # and a chunk's kernels wait for its copy
+    loaded = [c[1] for c in log[copies[k]:] if c[0] == "record" and c[2] == side][0]
+    digits = [i for i, c in enumerate(log) if c[0] == "launch" and "digits" in c[1]][k]
+    assert any(c[0] == "wait" and c[1] == loaded and c[2] == mine for c in log[copies[k]:digits])
+""")
