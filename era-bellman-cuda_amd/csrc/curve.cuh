@@ -94,28 +94,6 @@ BC_HD g1_xyzz xyzz_add_affine(const g1_xyzz &p, const g1_affine &q) {
   return {X3, Y3, mul_lazy<Fq>(p.zz, PP), mul_lazy<Fq>(p.zzz, PPP)};
 }
 
-// add-2008-s: p + q
-BC_HD g1_xyzz xyzz_add(const g1_xyzz &p, const g1_xyzz &q) {
-  if (xyzz_is_infinity(p))
-    return q;
-  if (xyzz_is_infinity(q))
-    return p;
-  const fe U1 = mul_lazy<Fq>(p.x, q.zz);
-  const fe U2 = mul_lazy<Fq>(q.x, p.zz);
-  const fe S1 = mul_lazy<Fq>(p.y, q.zzz);
-  const fe S2 = mul_lazy<Fq>(q.y, p.zzz);
-  const fe P = sub2<Fq>(U2, U1);
-  const fe R = sub2<Fq>(S2, S1);
-  if (fq_is_zero_lazy(P) && fq_is_zero_lazy(R))
-    return xyzz_dbl(p);
-  const fe PP = mul_lazy<Fq>(P, P);
-  const fe PPP = mul_lazy<Fq>(P, PP);
-  const fe Q = mul_lazy<Fq>(U1, PP);
-  const fe X3 = sub2<Fq>(sub2<Fq>(mul_lazy<Fq>(R, R), PPP), dbl2<Fq>(Q));
-  const fe Y3 = mul2_lazy<Fq>(R, sub2<Fq>(Q, X3), S1, neg2<Fq>(PPP)); // R (Q - X3) - S1 PPP
-  return {X3, Y3, mul_lazy<Fq>(p.zz, mul_lazy<Fq>(q.zz, PP)), mul_lazy<Fq>(p.zzz, mul_lazy<Fq>(q.zzz, PPP))};
-}
-
 // XYZZ -> Jacobian: Z = ZZ*ZZZ, X = X*ZZ*ZZZ^2, Y = Y*ZZ^3*ZZZ^2 (infinity -> (0, 1, 0))
 BC_HD g1_jacobian xyzz_to_jacobian(const g1_xyzz &p) {
   if (xyzz_is_infinity(p))

@@ -19,7 +19,11 @@ namespace bc {
 
 namespace divsteps {
 
-// 254-bit operands need at most (49 * 254 + 57) / 17 = 735 steps
+// A cap, not a count: the loop ends with g = 0.  The steps above start half a
+// step lower (delta = 1/2) than those for which the paper proves at most
+// (49 d + 57) / 17, 735 for d = 254 bits, and need fewer: 590 suffice for 256 bits
+// by the convex-hull computation of Wuille, "Bounds on divsteps iterations in
+// safegcd", 2021.
 constexpr int BATCH = 29, MAX_BATCHES = (735 + BATCH - 1) / BATCH;
 
 struct s29 {

@@ -29,10 +29,11 @@
 //                  heavy bucket (e.g. digit 1 of window 0 when many scalars
 //                  are 1) is spread over many threads; the same pass records
 //                  each bucket's run [start, end) of sorted entries;
-//   4. fix-up:     a bucket's sums lie in consecutive slots; buckets of more
-//                  than 32 are listed and reduced by one-wave blocks (chunks
-//                  of 512 sums: serial sums of 8, then an LDS tree); smaller
-//                  ones are summed as the buckets are gathered into windows;
+//   4. bucket sums: a bucket's partial sums lie in consecutive slots; one launch
+//                  adds them into the windows, a thread a bucket of up to a few
+//                  (4..32, small_pieces), a wave of quads a listed bucket of up to
+//                  64, and a block of quads every 512 sums of a larger one, whose
+//                  chunks a second launch joins;
 //   5. per-bit reduction: windows are split recursively into low/high halves
 //                  of their index bits (sums split across threads, then folded,
 //                  or by quads of lanes) until they hold at most 8 bits; then a

@@ -9,11 +9,13 @@ namespace bc {
 
 constexpr unsigned NTT_MAX_LOG = 28;
 constexpr unsigned NTT_MAX_JOBS = 64;
-// Stages per HBM pass at most (tiles of 2^10 elements, 32 KiB of LDS): five
-// blocks share a CU, so one block's loads and stores overlap the others'
-// butterflies.  Measured on MI355X against 2^9..2^12-element tiles, it is the
-// fastest at every size from 2^14 to 2^24 (2^24: 1.80 ms in three passes
-// against 2.27 ms in two passes of 2^12-element tiles).
+// Stages per HBM pass of VALU butterflies at most (tiles of 2^10 elements, 32 KiB
+// of LDS): five blocks share a CU, so one block's loads and stores overlap the
+// others' butterflies.  Against tiles of 2^9..2^12 elements it is the fastest of
+// these passes wherever they fill the GPU (2^24: 1.80 ms in three
+// passes against 2.27 ms in two passes of 2^12-element tiles); launches of
+// NTT_SMALL_ELEMENTS and less, and natural-order transforms from
+// NTT_MFMA_MIN_LOG on, take passes of their own.
 constexpr unsigned NTT_LOG_TILE = 10;
 
 // Smallest natural-order transform whose first twelve stages run on the matrix

@@ -305,7 +305,7 @@ template <bool GS> __global__ __launch_bounds__(NTT_BLOCK) void ntt_pass_kernel(
 // a stage (tiles of at most 512 elements for 256 threads, one wave per SIMD)
 // where a radix-4 step of the kernel above has four products in a row, and the
 // next stage's twiddle is loaded during the current one.  2^12 elements 29 ->
-// 21 us, 2^17 41 -> 31 us (34 bit-reversed to natural).
+// 17 us, 2^17 42 -> 31 us.
 template <bool GS> __global__ __launch_bounds__(NTT_SMALL_BLOCK) void ntt_small_pass_kernel(const pass_table pt) {
   using F = FrParams;
   __shared__ fe tile[2 * NTT_SMALL_BLOCK];
