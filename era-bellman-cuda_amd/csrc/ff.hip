@@ -243,8 +243,10 @@ __global__ void select_kernel(const fe *__restrict__ src, fe *__restrict__ dst, 
 // form the products inside a group twice) and 50 / (G K INV_WAVES) for the
 // inversion.  The inverting wave moves with the block index, or every inversion
 // would land on the CU's first SIMD.
-// 4194299 elements 0.58 -> 0.20 ms, 65539 0.33 -> 0.048 ms (one power
-// a^(r-2) per 32 consecutive elements of a thread before).
+// 4194299 elements 0.58 -> 0.23 ms, 65539 0.33 -> 0.048 ms (one power
+// a^(r-2) per 32 consecutive elements of a thread before).  Elements may be any
+// 256 bits, so the running products stay canonical; only for lazy elements (< 2m) could
+// they be lazy, at 0.20 ms.
 constexpr unsigned INV_BLOCK = 256, INV_WAVES = INV_BLOCK / 64;
 template <unsigned G, unsigned K> __global__ __launch_bounds__(INV_BLOCK, G == 1 ? 2 : 3) void batch_inverse_kernel(const fe *in, fe *out, unsigned count) {
   using F = FrParams;
@@ -382,9 +384,9 @@ __global__ __launch_bounds__(256) void multiply_by_powers_kernel(const fe *fine,
   const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= count)
     return;
-  // the power canonical: then v may be any 256 bits
-  const fe v = load_fe(in + i), w = mul<FrParams>(load_fe(fine + (i & (POWERS_FINE - 1))), load_fe(coarse + (i >> POWERS_LOG_FINE)));
-  store_fe(out + i, mul<FrParams>(v, w));
+  // an element, any 256 bits, times a canonical value is below 2m
+  const fe v = mul_lazy<FrParams>(load_fe(in + i), load_fe(coarse + (i >> POWERS_LOG_FINE)));
+  store_fe(out + i, mul<FrParams>(v, load_fe(fine + (i & (POWERS_FINE - 1)))));
 }
 
 // sum_i values[i] x^i: block b writes its tile's sum_j values[b tile + j] x^j to
@@ -399,18 +401,34 @@ __global__ __launch_bounds__(EVAL_BLOCK) void poly_eval_kernel(const power_digit
   const power_digits &t = REF ? *ref : arg;
   constexpr unsigned G = K < 8 ? K : 8; // loads in flight
   const size_t first = (size_t)blockIdx.x * (EVAL_BLOCK * K) + threadIdx.x;
-  fe acc = fe_zero();
-  for (unsigned g = K / G; g-- > 0;) {
-    fe v[G];
+  fe acc;
+  // Values may be any 256 bits; almost all are below 3m, as the sums need them.  A wave
+  // that meets a top word of 2m or more, a compare an element, computes once more
+  // with its values reduced (every value reduced: 4194299 elements 58 -> 62 us).
+  bool wide = false, again = false;
+  do {
+    bool seen = false;
+    acc = fe_zero();
+    for (unsigned g = K / G; g-- > 0;) {
+      fe v[G];
 #pragma unroll
-    for (unsigned k = 0; k < G; k++) {
-      const size_t i = first + (size_t)(g * G + k) * EVAL_BLOCK;
-      v[k] = i < n ? load_fe(values + i) : fe_zero();
+      for (unsigned k = 0; k < G; k++) {
+        const size_t i = first + (size_t)(g * G + k) * EVAL_BLOCK;
+        v[k] = i < n ? load_fe(values + i) : fe_zero();
+      }
+      if (wide)
+#pragma unroll
+        for (unsigned k = 0; k < G; k++)
+          v[k] = reduce2<F>(v[k]); // < 2^256 - 2m
+#pragma unroll
+      for (unsigned k = G; k-- > 0;) { // x^EVAL_BLOCK is canonical, so the product is below 2m for any acc
+        seen |= v[k].v[7] >= F::m2[7];
+        acc = K == 1 ? v[0] : add_raw(mul_lazy<F>(acc, t.p[EVAL_DIGITS][0]), v[k]);
+      }
     }
-#pragma unroll
-    for (unsigned k = G; k-- > 0;) // any v is below 5.3 m, below 3.3 m reduced; x^EVAL_BLOCK is canonical, so a product is below 2m and acc below 2^256
-      acc = K == 1 ? v[0] : add_raw(mul_lazy<F>(acc, t.p[EVAL_DIGITS][0]), reduce2<F>(v[k]));
-  }
+    again = K > 1 && !wide && __any(seen);
+    wide = again;
+  } while (again);
   acc = mul_lazy<F>(acc, power_of(t, threadIdx.x, EVAL_DIGITS));
 #pragma unroll
   for (unsigned off = 32; off > 0; off >>= 1) {
