@@ -231,6 +231,13 @@ __global__ void select_kernel(const fe *__restrict__ src, fe *__restrict__ dst, 
   store_fe(dst + i, load_fe(src + idx[i]));
 }
 
+// Elements of a vector may be any 256 bits; products of products need lazy values
+// (< 2m).  Almost all elements are canonical, so a wave computes for lazy ones and
+// notes by a compare of the top word whether some may not be (2m and more have one
+// from m2[7] on); only then does it compute once more with reduced ones.
+__device__ __forceinline__ bool may_be_wide(const fe &a) { return a.v[7] >= FrParams::m2[7]; }
+__device__ __forceinline__ fe lazy_of_wide(const fe &a) { return reduce2<FrParams>(reduce2<FrParams>(a)); } // 2^256 < 6m
+
 // ---------------------------------------------------------------- batch inverse
 // Montgomery's trick in two levels, in one kernel and without scratch memory.
 // A thread multiplies up G groups of K elements (a block's threads take
@@ -243,12 +250,10 @@ __global__ void select_kernel(const fe *__restrict__ src, fe *__restrict__ dst, 
 // form the products inside a group twice) and 50 / (G K INV_WAVES) for the
 // inversion.  The inverting wave moves with the block index, or every inversion
 // would land on the CU's first SIMD.
-// 4194299 elements 0.58 -> 0.23 ms, 65539 0.33 -> 0.048 ms (one power
-// a^(r-2) per 32 consecutive elements of a thread before).  Elements may be any
-// 256 bits, so the running products stay canonical; only for lazy elements (< 2m) could
-// they be lazy, at 0.20 ms.
+// 4194299 elements 0.58 -> 0.20 ms, 65539 0.33 -> 0.048 ms (one power
+// a^(r-2) per 32 consecutive elements of a thread before).
 constexpr unsigned INV_BLOCK = 256, INV_WAVES = INV_BLOCK / 64;
-template <unsigned G, unsigned K> __global__ __launch_bounds__(INV_BLOCK, G == 1 ? 2 : 3) void batch_inverse_kernel(const fe *in, fe *out, unsigned count) {
+template <unsigned G, unsigned K> __global__ __launch_bounds__(INV_BLOCK, G == 2 ? 3 : 2) void batch_inverse_kernel(const fe *in, fe *out, unsigned count) {
   using F = FrParams;
   __shared__ fe totals[INV_WAVES][64], earlier[INV_WAVES][64]; // `earlier` in LDS: the inversion needs the registers
   __shared__ fe start[G][INV_BLOCK];                               // product of the thread's groups before g
@@ -256,6 +261,7 @@ template <unsigned G, unsigned K> __global__ __launch_bounds__(INV_BLOCK, G == 1
   const size_t first = (size_t)blockIdx.x * (G * K * INV_BLOCK) + threadIdx.x;
   fe before[K]; // product of the thread's elements before element k of the group
   fe acc = fe_one<F>();
+  bool wide = false;
   // zero inverts to zero and leaves the products alone
   auto multiply_up = [&](unsigned g) {
     fe v[K];
@@ -266,9 +272,20 @@ template <unsigned G, unsigned K> __global__ __launch_bounds__(INV_BLOCK, G == 1
     }
 #pragma unroll
     for (unsigned k = 0; k < K; k++) {
+      wide |= may_be_wide(v[k]);
       before[k] = acc;
       if (!fe_is_zero(v[k]))
-        acc = mul<F>(acc, v[k]); // canonical: then v may be any 256 bits
+        acc = mul_lazy<F>(acc, v[k]);
+    }
+  };
+  // `acc` times the first `n` elements of group g, reduced
+  auto multiply_up_wide = [&](unsigned g, unsigned n) {
+#pragma unroll 1
+    for (unsigned k = 0; k < n; k++) {
+      const size_t i = first + (g * K + k) * INV_BLOCK;
+      const fe v = i < count ? lazy_of_wide(load_fe(in + i)) : fe_zero();
+      if (!fe_is_zero(v))
+        acc = mul_lazy<F>(acc, v);
     }
   };
 #pragma unroll 1
@@ -276,6 +293,15 @@ template <unsigned G, unsigned K> __global__ __launch_bounds__(INV_BLOCK, G == 1
     if (G > 1)
       start[g][threadIdx.x] = acc;
     multiply_up(g);
+  }
+  wide = __any(wide);
+  if (wide) {
+    acc = fe_one<F>();
+#pragma unroll 1
+    for (unsigned g = 0; g < G; g++) {
+      start[g][threadIdx.x] = acc;
+      multiply_up_wide(g, K);
+    }
   }
   totals[wave][lane] = acc;
   __syncthreads();
@@ -295,6 +321,27 @@ template <unsigned G, unsigned K> __global__ __launch_bounds__(INV_BLOCK, G == 1
   }
   __syncthreads();
   fe inv = totals[wave][lane];
+  auto put = [&](size_t i, const fe &v, const fe &product_before) {
+    if (fe_is_zero(v)) {
+      store_fe(out + i, v);
+    } else {
+      store_fe(out + i, mul<F>(product_before, inv));
+      inv = mul_lazy<F>(inv, v);
+    }
+  };
+  if (wide) { // rare: the products before an element once more for each, without registers for them
+#pragma unroll 1
+    for (unsigned g = G; g-- > 0;)
+#pragma unroll 1
+      for (unsigned k = K; k-- > 0;) {
+        acc = start[g][threadIdx.x];
+        multiply_up_wide(g, k);
+        const size_t i = first + (g * K + k) * INV_BLOCK;
+        if (i < count)
+          put(i, lazy_of_wide(load_fe(in + i)), acc);
+      }
+    return;
+  }
 #pragma unroll 1
   for (unsigned g = G; g-- > 0;) {
     if (G > 1) {
@@ -304,15 +351,8 @@ template <unsigned G, unsigned K> __global__ __launch_bounds__(INV_BLOCK, G == 1
 #pragma unroll
     for (unsigned k = K; k-- > 0;) {
       const size_t i = first + (g * K + k) * INV_BLOCK;
-      if (i < count) {
-        const fe v = load_fe(in + i);
-        if (fe_is_zero(v)) {
-          store_fe(out + i, v);
-        } else {
-          store_fe(out + i, mul<F>(before[k], inv));
-          inv = mul<F>(inv, v);
-        }
-      }
+      if (i < count)
+        put(i, load_fe(in + i), before[k]);
     }
   }
 }
@@ -325,7 +365,9 @@ template <unsigned G, unsigned K> void batch_inverse_launch(const fe *in, fe *ou
 // the whole vector (four, two, then two or three blocks a CU): a second round
 // of blocks waits for an inversion again (700000 elements: 107 us in two rounds
 // of K = 2, 75 us in one of K = 8), and a longer share than needed lengthens
-// the chain (524288 elements: 60 us at K = 2).
+// the chain (524288 elements: 60 us at K = 2).  32 elements a thread as 8 groups of
+// 4, whose way back is half the instructions: 4194299 elements 202 us, 219 as 4
+// groups of 8; above, 64 elements: 2^23 371 us against 387, 2^24 717 against 719.
 void batch_inverse(const fe *in, fe *out, unsigned count, hipStream_t s) {
   if (count <= 1u << 19)
     batch_inverse_launch<1, 2>(in, out, count, s);
@@ -333,8 +375,10 @@ void batch_inverse(const fe *in, fe *out, unsigned count, hipStream_t s) {
     batch_inverse_launch<1, 8>(in, out, count, s);
   else if (count <= 1u << 21)
     batch_inverse_launch<2, 8>(in, out, count, s);
+  else if (count <= 1u << 22)
+    batch_inverse_launch<8, 4>(in, out, count, s);
   else
-    batch_inverse_launch<4, 8>(in, out, count, s);
+    batch_inverse_launch<8, 8>(in, out, count, s);
 }
 
 // ---------------------------------------------------------------- powers of one point
@@ -402,9 +446,7 @@ __global__ __launch_bounds__(EVAL_BLOCK) void poly_eval_kernel(const power_digit
   constexpr unsigned G = K < 8 ? K : 8; // loads in flight
   const size_t first = (size_t)blockIdx.x * (EVAL_BLOCK * K) + threadIdx.x;
   fe acc;
-  // Values may be any 256 bits; almost all are below 3m, as the sums need them.  A wave
-  // that meets a top word of 2m or more, a compare an element, computes once more
-  // with its values reduced (every value reduced: 4194299 elements 58 -> 62 us).
+  // every value reduced: 4194299 elements 58 -> 62 us
   bool wide = false, again = false;
   do {
     bool seen = false;
@@ -419,10 +461,10 @@ __global__ __launch_bounds__(EVAL_BLOCK) void poly_eval_kernel(const power_digit
       if (wide)
 #pragma unroll
         for (unsigned k = 0; k < G; k++)
-          v[k] = reduce2<F>(v[k]); // < 2^256 - 2m
+          v[k] = lazy_of_wide(v[k]);
 #pragma unroll
-      for (unsigned k = G; k-- > 0;) { // x^EVAL_BLOCK is canonical, so the product is below 2m for any acc
-        seen |= v[k].v[7] >= F::m2[7];
+      for (unsigned k = G; k-- > 0;) { // x^EVAL_BLOCK canonical: the product is below 2m, acc below 4m
+        seen |= may_be_wide(v[k]);
         acc = K == 1 ? v[0] : add_raw(mul_lazy<F>(acc, t.p[EVAL_DIGITS][0]), v[k]);
       }
     }

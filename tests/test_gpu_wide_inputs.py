@@ -41,13 +41,15 @@ def wide(oracle, seed, n):
     return x, add_multiples(oracle, x, 5)
 
 
-# every form of the inverse (blocks of 512, 2048, 4096 and 8192 elements)
-@pytest.mark.parametrize("n", [2, 600, 65539, (1 << 19) + 1, (1 << 20) + 3, (1 << 21) + 5])
+# every form of the inverse (blocks of 512, 2048, 4096, 8192 and 16384 elements)
+@pytest.mark.parametrize("n", [2, 600, 65539, (1 << 19) + 1, (1 << 20) + 3, (1 << 21) + 5, 1 << 22, (1 << 22) + 16385])
 @pytest.mark.parametrize("in_place", [False, True])
 def test_batch_inverse_of_any_256_bits(bellman, oracle, n, in_place):
     B, dev = bellman
     x, y = wide(oracle, 0xBC0000B7 + n, n)
     x[3::11] = y[3::11] = 0
+    if n > 65539:
+        y[:n // 2] = x[:n // 2]  # whole waves of reduced elements
     d_in = dev.upload(y)
     d_out = d_in if in_place else dev.malloc(n * 32)
     B.call("ff_inverse", B.ff_inverse_configuration(dev.pool, dev.stream, d_in, d_out, n))
