@@ -462,17 +462,12 @@ __global__ __launch_bounds__(mf::BLOCK, 4) void ntt_mfma_kernel(const pass_table
     for (unsigned i = 0; i < 4; i++)
       x[i] = mul_lazy<F>(x[i], w[i]);
   }
-  // products are below 2r; the transform's inputs and what this kernel leaves are below
-  // 4r and taken 2r off, as the matrix products need |x| < 2.64 r
-  if (a.pre_table) {
+  // the transform's inputs and what this kernel leaves are below 4r, products (of any
+  // 256 bits and a lazy value) below 3r: all are taken 2r off, as the matrix products
+  // need |x| < 2.64 r
 #pragma unroll
-    for (unsigned i = 0; i < 4; i++)
-      x[i] = mf::add_offset(x[i], mf::offset(0, 1));
-  } else {
-#pragma unroll
-    for (unsigned i = 0; i < 4; i++)
-      x[i] = mf::add_offset(x[i], mf::offset(-2, 1));
-  }
+  for (unsigned i = 0; i < 4; i++)
+    x[i] = mf::add_offset(x[i], mf::offset(-2, 1));
   __syncthreads(); // `multiples`
   mf::radix4(x, block_matrices(0), block_matrices(0), multiples, two16);
 #pragma unroll

@@ -33,6 +33,17 @@ def test_natural_order_transforms_below_4r(bellman, oracle, log_n, inverse, log_
     assert np.array_equal(got, oracle.ntt(x, log_n, False, inverse, log_ext, log_ext))
 
 
+@pytest.mark.parametrize("log_n", [9, 12, 17, 18, 20, 23])
+def test_forward_coset_transforms_of_any_256_bits(bellman, oracle, log_n):
+    """The coset's factors are applied first, which leaves lazy values."""
+    _, dev = bellman
+    x = oracle.random_fr(0xBC0000A9 + log_n, 1 << log_n)
+    x[::5] = oracle.to_limbs([oracle.R - 1])[0]
+    x[::7] = oracle.to_limbs([1])[0]
+    got = ntt(dev, add_multiples(oracle, x, 5), log_n, log_ext=2, coset=3)
+    assert np.array_equal(got, oracle.ntt(x, log_n, False, False, 2, 3))
+
+
 def wide(oracle, seed, n):
     """Reduced values, and the same with up to 5 r added (no multiple of r but 0 itself)."""
     x = oracle.random_fr(seed, n)
