@@ -231,13 +231,6 @@ __global__ void select_kernel(const fe *__restrict__ src, fe *__restrict__ dst, 
   store_fe(dst + i, load_fe(src + idx[i]));
 }
 
-// Elements of a vector may be any 256 bits; products of products need lazy values
-// (< 2m).  Almost all elements are canonical, so a wave computes for lazy ones and
-// notes by a compare of the top word whether some may not be (2m and more have one
-// from m2[7] on); only then does it compute once more with reduced ones.
-__device__ __forceinline__ bool may_be_wide(const fe &a) { return a.v[7] >= FrParams::m2[7]; }
-__device__ __forceinline__ fe lazy_of_wide(const fe &a) { return reduce2<FrParams>(reduce2<FrParams>(a)); } // 2^256 < 6m
-
 // ---------------------------------------------------------------- batch inverse
 // Montgomery's trick in two levels, in one kernel and without scratch memory.
 // A thread multiplies up G groups of K elements (a block's threads take

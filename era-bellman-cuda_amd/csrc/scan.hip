@@ -172,6 +172,18 @@ __device__ __forceinline__ fe shfl_up_fe(const fe &a, unsigned off) {
   return r;
 }
 
+// Reduces a thread's elements if one of the wave's may not be lazy.
+template <unsigned K> __device__ __forceinline__ void make_lazy(fe (&v)[K]) {
+  bool wide = false;
+#pragma unroll
+  for (unsigned k = 0; k < K; k++)
+    wide |= may_be_wide(v[k]);
+  if (__any(wide))
+#pragma unroll
+    for (unsigned k = 0; k < K; k++)
+      v[k] = lazy_of_wide(v[k]);
+}
+
 // Scans tiles of SCAN_BLOCK * K elements, K consecutive ones a thread; the
 // product of a whole tile goes to tile_products (if any).
 template <unsigned K>
@@ -184,6 +196,7 @@ __global__ __launch_bounds__(SCAN_BLOCK) void prefix_product_tile_kernel(const f
 #pragma unroll
   for (unsigned k = 0; k < K; k++)
     v[k] = first + k < n ? load_fe(in + first + k) : fe_one<F>();
+  make_lazy(v);
 #pragma unroll
   for (unsigned k = 1; k < K; k++)
     v[k] = mul_lazy<F>(v[k - 1], v[k]);
@@ -235,6 +248,7 @@ __device__ __forceinline__ void load_chunk(const fe *in, size_t first, size_t n,
 #pragma unroll
   for (unsigned k = 0; k < PP_CHUNK; k++)
     v[k] = first + k < n ? load_fe(in + first + k) : fe_one<FrParams>();
+  make_lazy(v);
 }
 
 __global__ __launch_bounds__(SCAN_BLOCK) void prefix_product_chunk_kernel(const fe *in, fe *products, size_t n) {

@@ -71,6 +71,25 @@ def test_batch_inverse_of_any_256_bits(bellman, oracle, n, in_place):
     assert np.array_equal(got, oracle.batch_inverse(x))
 
 
+# one element a thread, tiles of 1024, tiles and their products, chunks of 8
+@pytest.mark.parametrize("n", [2, 255, 1000, 65539, (1 << 20) + 9, 4194299])
+@pytest.mark.parametrize("every", [1, 37])
+def test_prefix_products_of_any_256_bits(bellman, oracle, n, every):
+    B, dev = bellman
+    x, y = wide(oracle, 0xBC0000E7 + n, n)
+    if every > 1:  # single elements among reduced ones
+        z = x.copy()
+        z[::every] = y[::every]
+        y = z
+    d_in, d_out = dev.upload(y), dev.malloc(n * 32)
+    B.call("ff_grand_product", B.ff_grand_product_configuration(dev.pool, dev.stream, d_in, d_out, n))
+    dev.sync()
+    got = dev.download(d_out, (n, 8))
+    dev.free(d_in)
+    dev.free(d_out)
+    assert np.array_equal(got, oracle.grand_product(x))
+
+
 # one, two, eight and 32 elements a thread, one to three launches
 @pytest.mark.parametrize("n", [2, 256, 257, 513, 2048, 2049, 65539, (1 << 17) + 1, (1 << 21) + 1, 4194299])
 def test_polynomial_values_of_any_256_bits(bellman, oracle, n):
