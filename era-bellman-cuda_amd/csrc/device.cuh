@@ -45,10 +45,9 @@ __device__ __forceinline__ unsigned brev_bits(unsigned x, unsigned bits) { retur
 
 inline unsigned grid_for(size_t n, unsigned block) { return static_cast<unsigned>((n + block - 1) / block); }
 
-// Elements of a vector may be any 256 bits; products of products need lazy values
-// (< 2m).  Almost all elements are canonical, so a wave computes for lazy ones and
-// notes by a compare of the top word whether some may not be (2m and more have one
-// from m2[7] on); only then does it compute once more with reduced ones.
+// Elements of a vector may be any 256 bits; products of products and sums need lazy
+// values (< 2m).  Almost all elements are canonical, so only a wave that meets a top
+// word of 2m or more, one compare an element, goes over its elements reduced.
 __device__ __forceinline__ bool may_be_wide(const fe &a) { return a.v[7] >= FrParams::m2[7]; }
 __device__ __forceinline__ fe lazy_of_wide(const fe &a) { return reduce2<FrParams>(reduce2<FrParams>(a)); } // 2^256 < 6m
 
